@@ -186,8 +186,10 @@ int pp_dump_state(const char *agents_path, const char *cells_path, int append,
 
 /* Per-kernel timing, the counterpart of the reference's profiler summary and
  * --prof-agg export (pp_gpu.c:318-321, :1868-1881; pp_common.c:248-260).
- * When enabled, each kernel launch of init/step/run is bracketed by HIP events
- * on the simulation's stream and no graph is used. */
+ * When enabled, the iterations run as the staged step (one kernel for each of
+ * the sort, the actions and the move, which the names tell apart; otherwise
+ * one kernel does an iteration's work), each kernel launch of init/step/run is
+ * bracketed by HIP events on the simulation's stream, and no graph is used. */
 int pp_sim_set_profiling(pp_sim_t *s, int enable);
 /* Number of kernels tracked, and for kernel i its name, launch count and
  * total / average duration in nanoseconds. A name can cover more than one
@@ -316,10 +318,13 @@ int pp_batch_info(const pp_batch_t *b, uint32_t *sort_passes,
 
 /* Sort of the agents by cell: mode 0 = the radix sort every iteration;
  * 8..11 = from the second iteration after a change of the replicas, row
- * buckets (blocks of 2^mode cells of a grid row); 1 (the default) = row
- * buckets of 2^11 cells for a single replica, and for a batch with at most
- * 16384 of them or at least 64 agents per bucket (its replicas' agents as
- * last collected), else the radix sort. Results do not depend on it. */
+ * buckets (blocks of 2^mode cells of a grid row); 1 (the default) = no sort of
+ * its own: from the second iteration on, one kernel an iteration sorts, acts
+ * and moves tile by tile. Populations too dense for its tiles (several agents
+ * a cell) then sort by row buckets of 2^11 cells for a single replica, and for
+ * a batch with at most 16384 of them or at least 64 agents per bucket (its
+ * replicas' agents as last collected), else by the radix sort. Results do not
+ * depend on it. */
 int pp_batch_set_sort(pp_batch_t *b, uint32_t mode);
 
 /* Radix sort launch shape: keys per thread (8 or 16; tile = 256 x that) and
@@ -338,12 +343,12 @@ int pp_batch_get_launch(const pp_batch_t *b, uint32_t *tile_rounds,
 	uint32_t *bucket_eighths);
 
 /* Autotuner: runs trial_ticks iterations of the batch under each candidate
- * sort (bucket widths 2^8..2^11, radix shapes; the iterations count as
- * normal progress), keeps the fastest and reports it (bucket_shift 0 = radix
- * sort) with its seconds per tick. When the fastest is what the automatic
+ * sort (the automatic mode's tiles, bucket widths 2^8..2^11, radix shapes; the
+ * iterations count as normal progress), keeps the fastest and reports it
+ * (bucket_shift 0 = radix sort, 1 = tiles) with its seconds per tick. When the fastest is what the automatic
  * mode (pp_batch_set_sort 1) picks for the current replicas, the batch stays
  * in the automatic mode; otherwise the winner is pinned as if set with
- * pp_batch_set_sort / pp_batch_set_shape. Then, under that sort, each
+ * pp_batch_set_sort / pp_batch_set_shape. Then, under a sort of its own, each
  * launch shape (tile_rounds 1, 2, 4, 8; bucket_eighths 4, 8) is timed and
  * the fastest kept (pp_batch_get_launch reports it). A trial during which
  * replicas finish is timed again. */

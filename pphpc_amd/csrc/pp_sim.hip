@@ -47,6 +47,13 @@
  * t0_r, is at its local iteration s = tick - t0_r. Grass regrow steps are
  * stored in ticks, so the grass of every replica uses one clock.
  *
+ * Two forms of the step. The staged step sorts (by row buckets, or by radix),
+ * acts and emits in a kernel each, over the whole batch. The tile step
+ * (pp_tile.h) does an iteration in one kernel, tile by tile; it is the default
+ * and hands over to the staged step where a population is too dense for its
+ * tiles, for the first iteration after a change of the replicas, under an
+ * explicit sort mode, and for per-kernel profiles.
+ *
  * No kernel waits on another work-group: every cross-group dependency is a
  * kernel boundary, so the step has no spin loops.
  *
@@ -188,7 +195,9 @@ struct RepCtl {
 	uint32_t status;   /* RS_* */
 	int32_t error;     /* PP_* code of a failed replica */
 	uint32_t err_step; /* iteration at which it failed */
-	uint32_t pad[2];
+	uint32_t ovf;      /* tick + 1 in which an agent of a tile passed the
+	                    * energy limit (0: none) */
+	uint32_t pad;
 	unsigned long long dead_cells;  /* grass cells with countdown > 0 */
 	unsigned long long cd_sum;      /* sum of grass countdowns */
 	unsigned long long acc[NACC];   /* this iteration, AC_* */
@@ -212,6 +221,13 @@ struct Ctl {
 	 * table holds one replica: the emit's work-group 0 then ends the tick
 	 * (advances Ctl::tick) while the others still run, so they read this */
 	uint32_t emit_tick;
+	/* the tile step: the tick whose state each parity of the record buffers
+	 * holds; where to stop, and whether a launch has (tile_runs) */
+	uint32_t tt[2];
+	uint32_t stop, halt;
+	uint32_t in_tick;  /* tick at which the records were written from the SoA
+	                    * state */
+	uint32_t pad;
 	/* sums over completed ticks of: agents at the start, alive after the
 	 * move, after actions, occupied cells, grass eaten, births */
 	unsigned long long agent_steps, sum_live, sum_out, sum_occ, sum_eaten,
@@ -889,6 +905,58 @@ __global__ __launch_bounds__(WG) void k_move0(const uint32_t *__restrict__ cell,
 		for (int i = 0; i < NWAVE; i++) sum += s_red[i];
 		if (sum) atomicAdd(&ctl->live[tick & 1], (uint32_t)sum);
 	}
+}
+
+/* Before k_move_soa: no pairs (positions of replicas that have ended stay
+ * so), no survivors counted, and the partial sums at zero. */
+__global__ __launch_bounds__(WG) void k_pairs_clear(uint32_t *keys, Ctl *ctl,
+	unsigned long long *part) {
+	const uint32_t i0 = blockIdx.x * WG + threadIdx.x, n = ctl->n;
+	for (uint32_t i = i0; i < n; i += gridDim.x * WG) keys[i] = DEAD_KEY;
+	if (i0 < PART_SLOTS * PART_STRIDE) part[i0] = 0;
+	if (i0 < 2) ctl->live[i0] = 0;
+}
+
+/* Move of one replica's agents in the SoA state (positions from RepCtl::base,
+ * in id order): their pairs and the live count, as k_move0. */
+__global__ __launch_bounds__(WG) void k_move_soa(const uint32_t *__restrict__ cell,
+	const int32_t *__restrict__ energy, const uint8_t *__restrict__ type,
+	uint32_t *__restrict__ keys, uint32_t *__restrict__ vals, Ctl *ctl,
+	Tables T, uint32_t slot, Params P) {
+	if (ctl->error) return;
+	const uint32_t tick = ctl->tick;
+	const Rep &rp = T.rep[slot];
+	const RepCtl &rc = T.rctl[slot];
+	if (rc.status != RS_ACTIVE) return;
+	RM m;
+	m.cb = rp.cb;
+	m.C = rp.C;
+	m.gx = rp.gx;
+	m.gy = rp.gy;
+	m.sheep_prob = rp.sheep_prob;
+	m.wolves_prob = rp.wolves_prob;
+	m.key0 = rp.key0;
+	m.key1 = rp.key1;
+	m.step = tick - rp.t0;
+	m.bbase = 0;
+	m.nb = row_blocks(rp.gx, P.bshift);
+	m.h = rows_per_bucket(rp.gx, P.bshift);
+	const uint32_t base = rc.base, n = rc.n;
+	unsigned long long live = 0;
+	for (uint32_t l = blockIdx.x * WG + threadIdx.x; l < n; l += gridDim.x * WG) {
+		const uint32_t g = base + l, c = cell[g] - m.cb;
+		const uint32_t y = c / m.gx, x = c - y * m.gx;
+		uint32_t v, bkt;
+		const uint32_t k = move_agent(l, x, y, energy[g], type[g], m, P.bshift, &v,
+			&bkt);
+		keys[g] = k;
+		vals[g] = v;
+		live += k != DEAD_KEY;
+	}
+	/* (the sort's first kernel adds up the slots) */
+	live = wave_sum(live);
+	if ((threadIdx.x & (WAVE - 1)) == 0 && live)
+		atomicAdd(&P.part[(blockIdx.x % PART_SLOTS) * PART_STRIDE + PART_LIVE], live);
 }
 
 /* ------------------------------------------------------------------- sort */
@@ -3073,6 +3141,8 @@ __global__ __launch_bounds__(NT) void k_emit_move(
 	}
 }
 
+#include "pp_tile.h"
+
 /* ------------------------------------------------------------ host layer */
 
 enum KernelId {
@@ -3193,6 +3263,44 @@ std::vector<SortShape> tune_candidates(uint32_t key_bits, uint32_t cap) {
 	return out;
 }
 
+/* FORM_* of a batch (pp_batch::form). */
+enum { FORM_PAIRS = 0, FORM_TILES, FORM_SOA };
+
+/* The tile step of the current replica table: whether it can run, the kernel
+ * (group shape) and the device arrays its arguments name. */
+struct TilePlan {
+	int on = 0;
+	int cfg = 0;
+	bool d2 = false;      /* some replica's rows are cut into several tiles */
+	uint32_t ntiles = 0, nbands = 0, rows = 0, slot = 0, nmax = 0, hmax = 0;
+	uint2 *rec[2] = {nullptr, nullptr};
+	uint4 *hdr[2] = {nullptr, nullptr};
+	uint32_t *rowv[2] = {nullptr, nullptr};
+	uint2 *edge[2] = {nullptr, nullptr};
+	uint32_t *spare = nullptr;
+	uint32_t spare0 = 0;
+	TileStat *stat[2] = {nullptr, nullptr};
+	uint32_t *idoff = nullptr, *rtot = nullptr, *bsum = nullptr;
+	uint32_t *tk = nullptr, *bk = nullptr;
+	TileRep *trep = nullptr;
+	TileRep one{};
+	/* of several replicas: what trep, tk and bk hold */
+	std::vector<TileRep> h_trep;
+	std::vector<uint32_t> h_tk, h_bk;
+	TileStat *bstat = nullptr;
+	unsigned long long *tot = nullptr;
+};
+
+/* Grids wider than this have their rows cut into tiles of 256 cells; a single
+ * replica's tiles of whole rows hold at least TILE_MIN cells. */
+constexpr uint32_t TILE_WIDE = 2048, TILE_MIN = 400;
+
+/* Shapes of k_tile: threads, slots a thread, cells a tile. */
+struct TileShape {
+	uint32_t nt, ipt, cells;
+};
+const TileShape tile_shapes[] = {{256, 8, 4096}, {512, 8, 8192}};
+
 } /* namespace */
 
 struct pp_batch {
@@ -3239,6 +3347,13 @@ struct pp_batch {
 	 * through ncnt, with no argument of its own) */
 	uint32_t *brep_dev = nullptr;
 	int need_radix = 1;   /* the next tick sorts with the radix sort */
+	/* where the agents are between runs: moved pairs (the staged step), the
+	 * tiles' records, or only the SoA state, in cell order */
+	int form = FORM_PAIRS;
+	int soa_fresh = 0;    /* the SoA state is that of the current tick */
+	TilePlan plan;        /* the tiles of the replica table */
+	uint32_t tile_par = 0;   /* parity of the record buffers in use */
+	uint32_t tile_dense = 0; /* halvings of the tiles after a stop */
 	/* 0: radix sort every tick; 1: automatic; 8..11: row buckets of
 	 * 2^mode cells */
 	uint32_t sort_mode = 1;
@@ -3262,6 +3377,7 @@ struct pp_batch {
 
 	hipGraphExec_t graph_exec = nullptr;   /* 8 bucket-sort ticks */
 	hipGraphExec_t graph_radix = nullptr;  /* 8 radix-sort ticks */
+	hipGraphExec_t graph_tile = nullptr;   /* 8 tile ticks from parity 0 */
 	int graph_steps = 0;
 
 	int profiling = 0;
@@ -3277,6 +3393,8 @@ struct pp_batch {
 	std::map<uint32_t, Replica> reps;
 	uint32_t next_id = 0;
 	uint64_t table_version = 0;   /* replica table uploads */
+	uint32_t table_nrep = 0;      /* replicas in the table */
+	std::vector<uint32_t> table_slots;
 
 	Tables tables() const {
 		return Tables{rep_dev, rctl_dev, cbs_dev, order_dev, bbase_dev, crep_dev};
@@ -3489,6 +3607,8 @@ static int enqueue_step(pp_batch_t *b, int radix) {
 static void drop_graph(pp_batch_t *b) {
 	if (b->graph_exec) (void)hipGraphExecDestroy(b->graph_exec);
 	if (b->graph_radix) (void)hipGraphExecDestroy(b->graph_radix);
+	if (b->graph_tile) (void)hipGraphExecDestroy(b->graph_tile);
+	b->graph_tile = nullptr;
 	b->graph_exec = nullptr;
 	b->graph_radix = nullptr;
 	b->graph_steps = 0;
@@ -3555,14 +3675,18 @@ static void apply_launch(pp_batch_t *b, uint32_t tile_rounds,
 	apply_shape(b, b->shape);
 }
 
-/* Capture `steps` ticks into one executable graph (kernels only; no memset
- * or copy nodes). */
-static int build_graph(pp_batch_t *b, int steps, int radix,
+static int enqueue_tile(pp_batch_t *b);
+
+/* Capture `steps` ticks (kind 0: bucket sort, 1: radix sort, 2: tiles, an
+ * even number) into one executable graph (kernels only; no memset or copy
+ * nodes). */
+static int build_graph(pp_batch_t *b, int steps, int kind,
 	hipGraphExec_t *out) {
 	hipGraph_t g = nullptr;
 	HIP_OK(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
 	int rc = PP_SUCCESS;
-	for (int i = 0; i < steps && rc == PP_SUCCESS; i++) rc = enqueue_step(b, radix);
+	for (int i = 0; i < steps && rc == PP_SUCCESS; i++)
+		rc = kind == 2 ? enqueue_tile(b) : enqueue_step(b, kind);
 	hipError_t e = hipStreamEndCapture(b->stream, &g);
 	if (rc != PP_SUCCESS) {
 		if (g) (void)hipGraphDestroy(g);
@@ -3576,31 +3700,449 @@ static int build_graph(pp_batch_t *b, int steps, int radix,
 	return PP_SUCCESS;
 }
 
-/* Enqueue `ticks` ticks: after a change of the replica table the first one
- * sorts with the radix sort (the moved order is not the cell order yet, or
- * the bucket layout changed); then whole graphs of 8, then single launches.
- * The last tick's emit writes the SoA state that state_of reads. */
+/* The arguments of the tile kernels with the buffers of parity par as input. */
+static TileArgs tile_args(const pp_batch_t *b, uint32_t par) {
+	const TilePlan &p = b->plan;
+	TileArgs a{};
+	a.in = p.rec[par];
+	a.out = p.rec[1 - par];
+	a.hin = p.hdr[par];
+	a.hout = p.hdr[1 - par];
+	a.rin = p.rowv[par];
+	a.rout = p.rowv[1 - par];
+	a.sin = p.stat[par];
+	a.sout = p.stat[1 - par];
+	a.idoff = p.idoff;
+	a.rtot = p.rtot;
+	a.bsum = p.bsum;
+	a.bstat = p.bstat;
+	a.trep = p.trep;
+	a.one = p.one;
+	a.tk = p.tk;
+	a.bk = p.bk;
+	a.tot = p.tot;
+	a.ein = p.edge[par];
+	a.eout = p.edge[1 - par];
+	a.spare = p.spare;
+	a.slot = p.slot;
+	a.spare0 = p.spare0;
+	a.ntiles = p.ntiles;
+	a.nbands = p.nbands;
+	a.nfin = b->table_nrep;
+	a.par = par;
+	a.rows = p.rows;
+	a.nmax = p.nmax;
+	a.hmax = p.hmax;
+	return a;
+}
+
+template <typename GT, bool D2, bool SOLO>
+static void launch_tile(pp_batch_t *b) {
+	const TileArgs a = tile_args(b, b->tile_par);
+	const uint32_t grid = a.nfin + ceil_div(a.ntiles, NXCD) * NXCD;
+	GT *g = (GT *)b->grass_at;
+	if (b->plan.cfg == 0)
+		k_tile<GT, 256, 8, 4096, D2, SOLO><<<grid, 256, 0, b->stream>>>(a, b->ctl,
+			b->tables(), b->P, b->table_nrep, g);
+	else
+		k_tile<GT, 512, 8, 8192, D2, SOLO><<<grid, 512, 0, b->stream>>>(a, b->ctl,
+			b->tables(), b->P, b->table_nrep, g);
+	if (D2)
+		k_tile_scan<<<a.nbands, WG, 0, b->stream>>>(a, b->ctl, b->tables(),
+			b->table_nrep);
+}
+
+template <typename GT>
+static void launch_tile_gt(pp_batch_t *b) {
+	if (b->plan.d2) {
+		if (b->table_nrep == 1) launch_tile<GT, true, true>(b);
+		else launch_tile<GT, true, false>(b);
+	} else {
+		if (b->table_nrep == 1) launch_tile<GT, false, true>(b);
+		else launch_tile<GT, false, false>(b);
+	}
+}
+
+/* Enqueue one tick of the tile step. */
+static int enqueue_tile(pp_batch_t *b) {
+	if (b->grass_bytes == 1) launch_tile_gt<uint8_t>(b);
+	else if (b->grass_bytes == 2) launch_tile_gt<uint16_t>(b);
+	else launch_tile_gt<uint32_t>(b);
+	HIP_OK(hipGetLastError());
+	b->tile_par ^= 1u;
+	return PP_SUCCESS;
+}
+
+template <typename GT, bool D2>
+static void launch_tiles_in(pp_batch_t *b) {
+	const TileArgs a = tile_args(b, 0);
+	k_tile_clear<<<ceil_div(2ull * a.nbands + 1, WG), WG, 0, b->stream>>>(a, b->ctl);
+	k_tiles_in<GT, D2><<<a.ntiles, WG, 0, b->stream>>>(a, b->ctl, b->tables(),
+		b->P, b->table_nrep, (GT *)b->grass_at, b->cell, b->energy, b->type);
+	/* the ids of the rows, as after a tick whose output is parity 0 */
+	if (D2)
+		k_tile_scan<<<a.nbands, WG, 0, b->stream>>>(tile_args(b, 1), b->ctl,
+			b->tables(), b->table_nrep);
+}
+
+template <typename GT, bool D2>
+static void launch_tiles_out(pp_batch_t *b) {
+	const TileArgs a = tile_args(b, 0);
+	k_tile_base<<<1, WAVE, 0, b->stream>>>(b->ctl, b->tables(), b->table_nrep);
+	k_tiles_out<GT, D2><<<a.ntiles, WG, 0, b->stream>>>(a, b->ctl, b->tables(),
+		b->P, b->table_nrep, (GT *)b->grass_at, b->cell, b->energy, b->type);
+}
+
+/* SoA state (in cell order) -> tiles. */
+static int tiles_in(pp_batch_t *b) {
+	const bool d2 = b->plan.d2;
+	const TilePlan &p = b->plan;
+	if (b->table_nrep > 1) {
+		HIP_OK(hipMemcpyAsync(p.trep, p.h_trep.data(), p.h_trep.size() * sizeof(TileRep),
+			hipMemcpyHostToDevice, b->stream));
+		HIP_OK(hipMemcpyAsync(p.tk, p.h_tk.data(), p.h_tk.size() * 4,
+			hipMemcpyHostToDevice, b->stream));
+		HIP_OK(hipMemcpyAsync(p.bk, p.h_bk.data(), p.h_bk.size() * 4,
+			hipMemcpyHostToDevice, b->stream));
+	}
+	if (b->grass_bytes == 1) d2 ? launch_tiles_in<uint8_t, true>(b) : launch_tiles_in<uint8_t, false>(b);
+	else if (b->grass_bytes == 2) d2 ? launch_tiles_in<uint16_t, true>(b) : launch_tiles_in<uint16_t, false>(b);
+	else d2 ? launch_tiles_in<uint32_t, true>(b) : launch_tiles_in<uint32_t, false>(b);
+	HIP_OK(hipGetLastError());
+	b->tile_par = 0;
+	b->form = FORM_TILES;
+	return PP_SUCCESS;
+}
+
+/* Tiles -> SoA state (the tiles stay valid). */
+static int tiles_out(pp_batch_t *b) {
+	if (b->form != FORM_TILES || b->soa_fresh) return PP_SUCCESS;
+	{
+		const bool d2 = b->plan.d2;
+		if (b->grass_bytes == 1) d2 ? launch_tiles_out<uint8_t, true>(b) : launch_tiles_out<uint8_t, false>(b);
+		else if (b->grass_bytes == 2) d2 ? launch_tiles_out<uint16_t, true>(b) : launch_tiles_out<uint16_t, false>(b);
+		else d2 ? launch_tiles_out<uint32_t, true>(b) : launch_tiles_out<uint32_t, false>(b);
+		HIP_OK(hipGetLastError());
+	}
+	b->soa_fresh = 1;
+	b->ctl_fresh = 0;
+	return PP_SUCCESS;
+}
+
+/* The SoA state as the only form (before the replica table changes). */
+static int to_soa(pp_batch_t *b) {
+	if (b->form != FORM_TILES) return PP_SUCCESS;
+	PP_TRY(tiles_out(b));
+	b->form = FORM_SOA;
+	return PP_SUCCESS;
+}
+
+/* SoA state -> moved pairs for the staged step, which then sorts them with
+ * the radix sort. */
+static int to_pairs(pp_batch_t *b) {
+	PP_TRY(to_soa(b));
+	if (b->form != FORM_SOA) return PP_SUCCESS;
+	k_pairs_clear<<<8 * (uint32_t)b->num_cu, WG, 0, b->stream>>>(b->keys[0], b->ctl,
+		b->P.part);
+	for (uint32_t k = 0; k < b->table_nrep; k++)
+		k_move_soa<<<8 * (uint32_t)b->num_cu, WG, 0, b->stream>>>(b->cell, b->energy,
+			b->type, b->keys[0], b->vals[0], b->ctl, b->tables(),
+			b->table_nrep == 1 ? b->P.one_slot : b->table_slots[k], b->P);
+	HIP_OK(hipGetLastError());
+	b->ctl_fresh = 0;
+	b->form = FORM_PAIRS;
+	b->soa_fresh = 1;
+	b->need_radix = 1;
+	return PP_SUCCESS;
+}
+
+/* Enqueue `ticks` ticks. The tile step runs where the plan allows it, from
+ * the state the staged step left (one staged tick after a change of the
+ * replica table: new agents are in no cell order yet), in graphs of 8 ticks
+ * and single launches. Otherwise the staged step: after a change of the
+ * replica table the first tick sorts with the radix sort (the moved order is
+ * not the cell order yet, or the bucket layout changed); then whole graphs of
+ * 8, then single launches; the last tick's emit writes the SoA state that
+ * state_of reads. */
 static int enqueue_ticks(pp_batch_t *b, uint32_t ticks) {
 	b->ctl_fresh = 0;
 	const int use_graph = !b->profiling && !b->no_graph &&
 		getenv("PPHPC_NO_GRAPH") == nullptr;
 	const int radix = !b->P.bucket_on;
+	const bool tile = b->plan.on && !b->profiling;
 	uint32_t i = 0;
-	if (ticks) {
-		k_state_tick<<<1, WAVE, 0, b->stream>>>(b->ctl, ticks);
+	if (!ticks) return PP_SUCCESS;
+	if (!tile) PP_TRY(to_pairs(b));
+	if (b->form == FORM_PAIRS && !(tile && b->soa_fresh)) {
+		k_state_tick<<<1, WAVE, 0, b->stream>>>(b->ctl, tile ? 1u : ticks);
 		HIP_OK(hipGetLastError());
+		if (tile || (b->need_radix && !radix)) {
+			PP_TRY(enqueue_step(b, radix || b->need_radix));
+			i = 1;
+		}
+		b->need_radix = 0;
+		b->soa_fresh = 1;    /* once the last of these ticks has run */
 	}
-	if (ticks && b->need_radix && !radix) {
-		PP_TRY(enqueue_step(b, 1));
-		i = 1;
+	if (tile) {
+		if (i < ticks && b->form != FORM_TILES) PP_TRY(tiles_in(b));
+		if (i < ticks) b->soa_fresh = 0;
+		if (i < ticks && b->tile_par) {
+			PP_TRY(enqueue_tile(b));
+			i++;
+		}
+		if (use_graph && ticks - i >= 8) {
+			if (!b->graph_tile) PP_TRY(build_graph(b, 8, 2, &b->graph_tile));
+			for (; i + 8 <= ticks; i += 8)
+				HIP_OK(hipGraphLaunch(b->graph_tile, b->stream));
+		}
+		for (; i < ticks; i++) PP_TRY(enqueue_tile(b));
+		if (b->form == FORM_TILES) {
+			const TileArgs a = tile_args(b, 0);
+			if (b->plan.d2)
+				k_tile_end<true><<<a.nfin, WG, 0, b->stream>>>(a, b->ctl, b->tables(),
+					b->P, b->table_nrep);
+			else
+				k_tile_end<false><<<a.nfin, WG, 0, b->stream>>>(a, b->ctl, b->tables(),
+					b->P, b->table_nrep);
+			HIP_OK(hipGetLastError());
+		}
+		return PP_SUCCESS;
 	}
-	b->need_radix = 0;
 	if (use_graph && ticks - i >= 8) {
 		hipGraphExec_t *g = radix ? &b->graph_radix : &b->graph_exec;
 		if (!*g) PP_TRY(build_graph(b, 8, radix, g));
 		for (; i + 8 <= ticks; i += 8) HIP_OK(hipGraphLaunch(*g, b->stream));
 	}
 	for (; i < ticks; i++) PP_TRY(enqueue_step(b, radix));
+	return PP_SUCCESS;
+}
+
+/* Grid of a replica and the agents it is expected to hold. */
+struct TileGrid {
+	const Rep *rep;
+	uint32_t slot;
+	uint64_t agents;
+};
+
+/* Chooses the tiles of a replica table (n grids in table order) and places
+ * the tile step's arrays in the memory of the bucket sort's tables, which the
+ * tile step does not use. Up to TILE_WIDE columns a tile is a run of whole rows
+ * (its ids then follow from one sum over the tiles' counts; 1600 x 1600: 18.6
+ * us an iteration, against 28 in tiles of 256 x 16 with their scan of the
+ * rows' counts after each iteration); wider grids are cut into 256 columns.
+ * One replica takes about as many tiles as run at once: four groups of 256
+ * threads a CU hold up to 1024, of which 256 are taken (400 x 400: 10.3 us
+ * with tiles of 2 or 4 rows, 11.2 of 8), else two groups of 512 (1600 x 1600:
+ * 18.6 us with 400 tiles of 4 rows, 20.4 with 320 of 5, 23.7 with 534 of 3, a
+ * second round). Several replicas fill the GPU with tiles as large as fit,
+ * which move fewer neighbours' agents twice (30 x 1600 x 1600: 248 us with 5
+ * rows, 284 with 4). PPHPC_TILE=shape,columns,rows sets them (columns 0: whole
+ * rows; shape -1: the staged step); results do not depend on them. */
+static void tile_layout(const pp_batch_t *b, const TileGrid *grid, uint32_t n,
+	TilePlan &p) {
+	if (n == 0 || b->sort_mode != 1 || getenv("PPHPC_WIDE_GROUPS") ||
+		getenv("PPHPC_BPREFIX_MIN"))
+		return;
+	/* agents per cell that the tiles are laid out for: at least 0.3 (young
+	 * populations grow), and more after each stop */
+	double dens = 0.3;
+	uint32_t width = 0;
+	uint64_t cells = 0;
+	for (uint32_t i = 0; i < n; i++) {
+		dens = std::max(dens, (double)grid[i].agents / grid[i].rep->C);
+		width = std::max(width, grid[i].rep->gx);
+		cells += grid[i].rep->C;
+	}
+	for (uint32_t i = 0; i < b->tile_dense; i++) dens *= 1.5;
+	p.d2 = width > TILE_WIDE;
+	uint32_t ebx = 0, eby = 0;
+	int ecfg = -2;
+	if (const char *e = getenv("PPHPC_TILE")) sscanf(e, "%d,%u,%u", &ecfg, &ebx, &eby);
+	if (ecfg == -1) return;
+	if (ebx) p.d2 = true;
+	/* rows of a tile (at most) in shape c: its cells, and most of the agents
+	 * it may hold */
+	const double fill = n > 1 ? 0.85 : 0.75;
+	auto limits = [&](int c) {
+		const uint32_t ag = tile_shapes[c].nt * tile_shapes[c].ipt;
+		const uint32_t wide = p.d2 ? std::min<uint32_t>(ebx ? ebx : 256, width) : width;
+		p.cfg = c;
+		p.hmax = std::min<uint32_t>(ag / 3, (uint32_t)(1.4 * dens * wide) + 64);
+		p.nmax = ag - 2 * p.hmax - (p.d2 ? 2 * TILE_ECAP : 0);
+	};
+	auto rows_max = [&](uint32_t w) {
+		return std::min((double)tile_shapes[p.cfg].cells / w, fill * p.nmax / (dens * w));
+	};
+	if (p.d2) {
+		limits(0);
+	} else {
+		limits(0);
+		/* one replica: enough tiles to use every CU */
+		const double want = n > 1 ? 1e9 : (double)cells / width / 256;
+		if (want > rows_max(width)) limits(1);
+	}
+	if (ecfg >= 0) limits(ecfg);
+	const TileShape sh = tile_shapes[p.cfg];
+	uint64_t tiles = 0, bands = 0;
+	uint32_t rows = 0;
+	if (n > 1) {
+		p.h_trep.resize(n);
+		p.h_tk.clear();
+		p.h_bk.clear();
+	}
+	for (uint32_t i = 0; i < n; i++) {
+		TileRep t{};
+		const Rep &rp = *grid[i].rep;
+		const uint32_t gx = rp.gx, gy = rp.gy;
+		t.slot = grid[i].slot;
+		t.gx = gx;
+		t.gy = gy;
+		t.cb = rp.cb;
+		t.t0 = rp.t0;
+		t.iters = rp.iters;
+		t.cap = rp.cap;
+		t.R = rp.R;
+		t.key0 = rp.key0;
+		t.key1 = rp.key1;
+		t.sheep_gain = rp.sheep_gain;
+		t.wolves_gain = rp.wolves_gain;
+		t.sheep_thr = rp.sheep_thr;
+		t.wolves_thr = rp.wolves_thr;
+		t.sheep_prob = rp.sheep_prob;
+		t.wolves_prob = rp.wolves_prob;
+		t.gxm = rp.gx_magic;
+		t.gxs = rp.gx_shift;
+		const uint64_t gb = b->grass_bytes;
+		if (!p.d2) {
+			t.bx = gx;
+			const double most = rows_max(gx);
+			uint32_t by = (uint32_t)std::min(most, 65535.0);
+			if (!by) return;
+			if (n == 1) {
+				/* one round of groups: as many tiles as fit, of at least
+				 * TILE_MIN cells */
+				const uint32_t round = p.cfg == 0 ? 256 : 512;
+				by = min_u32(by, std::max(ceil_div(gy, round), ceil_div(TILE_MIN, gx)));
+			}
+			/* whole 16-byte chunks of grass where a few rows more give them */
+			uint32_t m = 1;
+			while (m < 16 && (uint64_t)m * gx * gb % 16) m *= 2;
+			const uint32_t up = ceil_div(by, m) * m;
+			if (up <= most) by = up;
+			else if (by >= m) by -= by % m;
+			t.by = by;
+		} else {
+			t.bx = min_u32(ebx ? ebx : 256, gx);
+			t.shift = 4;
+			while ((1u << t.shift) < t.bx) t.shift++;
+			t.by = (uint32_t)std::min(std::min(rows_max(t.bx),
+				(double)(sh.cells >> t.shift)), (double)TILE_ROWS);
+			if (!t.by) return;
+		}
+		if (eby) t.by = eby;
+		t.by = min_u32(t.by, gy);
+		t.nbx = ceil_div(gx, t.bx);
+		t.nby = ceil_div(gy, t.by);
+		/* rows (or, in one piece, tiles) of whole 16-byte chunks of grass */
+		t.vec = rp.cb * gb % 16 == 0 && (p.d2
+			? gx * gb % 16 == 0 && t.bx * gb % 16 == 0
+			: t.by * (uint64_t)gx * gb % 16 == 0 && rp.C * gb % 16 == 0);
+		t.tile0 = (uint32_t)tiles;
+		t.band0 = (uint32_t)bands;
+		t.ntiles = t.nbx * t.nby;
+		tiles += (uint64_t)t.nbx * t.nby;
+		bands += t.nby;
+		rows = std::max(rows, t.by);
+		if (tiles > (1u << 24)) return;
+		if (n > 1) {
+			p.h_trep[i] = t;
+			p.h_tk.insert(p.h_tk.end(), t.ntiles, i);
+			p.h_bk.insert(p.h_bk.end(), t.nby, i);
+		} else {
+			p.one = t;
+		}
+	}
+	p.ntiles = (uint32_t)tiles;
+	p.nbands = (uint32_t)bands;
+	p.rows = rows;
+	const uint32_t ag = sh.nt * sh.ipt;
+	/* each record buffer (1.5 A records): slots of half the capacity in all,
+	 * and spare records for the whole capacity */
+	const uint64_t A4 = ((uint64_t)b->P.cap + 3) & ~3ull;
+	p.slot = (uint32_t)std::min<uint64_t>(2 * ag, A4 / 2 / tiles);
+	p.spare0 = (uint32_t)(A4 / 2);
+	p.rec[0] = reinterpret_cast<uint2 *>(b->keys[0]);
+	p.rec[1] = reinterpret_cast<uint2 *>(b->keys[0] + 3 * A4);
+	/* the arrays, 16-byte aligned */
+	const uint64_t words = (uint64_t)brec_off(b->P.nb_cap) + (uint64_t)BR_WORDS * b->P.nb_cap;
+	uint64_t off = 0;
+	auto take = [&](uint64_t bytes) {
+		void *q = (char *)b->ocnt + off;
+		off += (bytes + 15) & ~15ull;
+		return q;
+	};
+	for (int i = 0; i < 2; i++) {
+		p.hdr[i] = (uint4 *)take(tiles * sizeof(uint4));
+		p.stat[i] = (TileStat *)take(tiles * sizeof(TileStat));
+		p.rowv[i] = (uint32_t *)take(p.d2 ? tiles * (rows + 1) * 4 : 0);
+		p.edge[i] = (uint2 *)take(p.d2 ? tiles * 2 * TILE_ECAP * sizeof(uint2) : 0);
+	}
+	p.tot = (unsigned long long *)take(3 * PART_SLOTS * 8);
+	p.idoff = (uint32_t *)take(p.d2 ? tiles * rows * 4 : 0);
+	p.bsum = (uint32_t *)take(bands * 2 * 4);
+	p.bstat = (TileStat *)take(bands * sizeof(TileStat));
+	p.rtot = (uint32_t *)take(n * 4ull);
+	p.spare = (uint32_t *)take(2 * 4);
+	p.trep = (TileRep *)take(n * sizeof(TileRep));
+	p.tk = (uint32_t *)take(tiles * 4);
+	p.bk = (uint32_t *)take(bands * 4);
+	if (off > words * 4) return;
+	p.on = 1;
+}
+
+static void tile_plan(pp_batch_t *b, const TileGrid *grid, uint32_t n) {
+	TilePlan p;
+	tile_layout(b, grid, n, p);
+	const TilePlan &o = b->plan;
+	/* the graph names the arrays (which follow from these), and, of one
+	 * replica, its constants */
+	const bool same = p.on == o.on && p.cfg == o.cfg && p.d2 == o.d2 &&
+		p.ntiles == o.ntiles && p.nbands == o.nbands && p.rows == o.rows &&
+		p.slot == o.slot && p.hmax == o.hmax && p.nmax == o.nmax &&
+		memcmp(&p.one, &o.one, sizeof(TileRep)) == 0 &&
+		p.h_trep.size() == o.h_trep.size();
+	if (!same && b->graph_tile) {
+		(void)hipGraphExecDestroy(b->graph_tile);
+		b->graph_tile = nullptr;
+	}
+	b->plan = std::move(p);
+}
+
+static void table_plan(pp_batch_t *b) {
+	std::vector<TileGrid> g;
+	for (const uint32_t s : b->table_slots) {
+		const Rep &rp = b->rep_host[s];
+		auto it = b->reps.find((uint32_t)b->slot_rid[s]);
+		g.push_back({&rp, s, it == b->reps.end() ? rp.n0 : it->second.n});
+	}
+	tile_plan(b, g.data(), (uint32_t)g.size());
+}
+
+/* After a run, with the control words read back: the parity of the records,
+ * and, where a tile has outgrown its limits, the SoA state and the need for
+ * another plan (returned in *again). */
+static int tile_settle(pp_batch_t *b, int *again) {
+	*again = 0;
+	if (b->form != FORM_TILES || b->ctl_host->error) return PP_SUCCESS;
+	const Ctl *c = b->ctl_host;
+	b->tile_par = (int32_t)(c->tt[1] - c->tt[0]) > 0 ? 1u : 0u;
+	if (!c->stop) return PP_SUCCESS;
+	/* (records that did not fit in the first place are not complete: the SoA
+	 * state they were read from is) */
+	if (c->tick == c->in_tick) b->soa_fresh = 1;
+	PP_TRY(to_soa(b));
+	b->tile_dense++;
+	*again = 1;
 	return PP_SUCCESS;
 }
 
@@ -3617,6 +4159,10 @@ static int read_ctl(pp_batch_t *b) {
 /* Replica table: the slots in use sorted by first cell, and its length. The
  * stream must be idle. */
 static int upload_table(pp_batch_t *b) {
+	if (b->form == FORM_TILES) {
+		PP_TRY(to_soa(b));
+		HIP_OK(hipStreamSynchronize(b->stream));
+	}
 	std::vector<std::pair<uint32_t, uint32_t>> t;
 	for (uint32_t s = 0; s < b->max_rep; s++)
 		if (b->slot_rid[s] >= 0) t.push_back({b->rep_host[s].cb, s});
@@ -3720,6 +4266,10 @@ static int upload_table(pp_batch_t *b) {
 	b->ctl_host->nbuckets = nb32;
 	b->need_radix = 1;
 	b->table_version++;
+	b->table_nrep = nrep;
+	b->table_slots = order;
+	b->tile_dense = 0;
+	table_plan(b);
 	return PP_SUCCESS;
 }
 
@@ -3820,7 +4370,10 @@ static int collect(pp_batch_t *b) {
 			dirty = 1;
 		}
 	}
+	int again = 0;
+	PP_TRY(tile_settle(b, &again));
 	if (dirty) PP_TRY(upload_table(b));
+	else if (again) table_plan(b);
 	return PP_SUCCESS;
 }
 
@@ -3829,6 +4382,24 @@ static uint32_t active_count(const pp_batch_t *b) {
 	for (auto &kv : b->reps)
 		if (kv.second.slot >= 0 && kv.second.status == RS_ACTIVE) n++;
 	return n;
+}
+
+/* Runs `ticks` ticks and collects; where the tiles stop short (tile_settle),
+ * the rest with the new plan. The control words must be fresh. */
+static int run_ticks(pp_batch_t *b, uint32_t ticks) {
+	const uint32_t target = b->ctl_host->tick + ticks;
+	while (b->ctl_host->tick != target) {
+		const uint32_t t0 = b->ctl_host->tick;
+		const uint32_t dense0 = b->tile_dense;
+		PP_TRY(enqueue_ticks(b, target - t0));
+		PP_TRY(collect(b));
+		if (b->ctl_host->error) break;
+		/* (a plan can stop at its first tick; the next one is finer) */
+		if (b->ctl_host->tick == t0 && b->tile_dense == dense0)
+			return PP_LIBRARY_ERROR;
+		if (active_count(b) == 0) break;
+	}
+	return PP_SUCCESS;
 }
 
 /* Runs up to `ticks` ticks in chunks that the stats rings hold, collecting
@@ -3843,8 +4414,7 @@ static int advance(pp_batch_t *b, uint32_t ticks) {
 	const uint32_t chunk_max = b->stats_rows / 2;
 	while (done < ticks && active_count(b) > 0) {
 		const uint32_t chunk = min_u32(ticks - done, chunk_max);
-		PP_TRY(enqueue_ticks(b, chunk));
-		PP_TRY(collect(b));
+		PP_TRY(run_ticks(b, chunk));
 		done += chunk;
 		if (b->ctl_host->error) return b->ctl_host->error;
 	}
@@ -3863,10 +4433,7 @@ static void batch_free(pp_batch_t *b) {
 	(void)hipFree(b->cell);
 	(void)hipFree(b->energy);
 	(void)hipFree(b->type);
-	for (int i = 0; i < 3; i++) {
-		(void)hipFree(b->keys[i]);
-		(void)hipFree(b->vals[i]);
-	}
+	(void)hipFree(b->keys[0]);   /* every pair buffer */
 	(void)hipFree(b->grass_at);
 	(void)hipFree(b->ring);
 	(void)hipFree(b->hist);
@@ -3909,7 +4476,7 @@ static uint64_t batch_bytes(uint64_t A, uint64_t C, uint32_t max_rep,
 	t += 4ull * (brec_off(nb_cap_for(C)) - cnt_words(nb_cap_for(C)))
 		+ 4ull * BR_WORDS * nb_cap_for(C);
 	t += 4ull * ((C >> CREP_SHIFT) + 1);   /* the cell-chunk table */
-	t += C * grass_bytes_for(R);
+	t += (C * grass_bytes_for(R) + 3) & ~3ull;
 	t += (uint64_t)max_rep * (R + 1) * 8;
 	t += hist_words * 4 + RADIX_MAX * 4;
 	{
@@ -3944,11 +4511,15 @@ static int batch_buffers(pp_batch_t *b, Take &&take) {
 	HIP_OK(take((void **)&b->cell, A4 * 4));
 	HIP_OK(take((void **)&b->energy, A4 * 4));
 	HIP_OK(take((void **)&b->type, A4));
+	/* three buffers of pairs; the tile step's two record buffers are their
+	 * halves (1.5 A records each) */
+	HIP_OK(take((void **)&b->keys[0], 6 * A4 * 4));
 	for (int i = 0; i < 3; i++) {
-		HIP_OK(take((void **)&b->keys[i], A4 * 4));
-		HIP_OK(take((void **)&b->vals[i], A4 * 4));
+		b->keys[i] = b->keys[0] + 2 * i * A4;
+		b->vals[i] = b->keys[i] + A4;
 	}
-	HIP_OK(take((void **)&b->grass_at, C * b->grass_bytes));
+	/* (the tile step reads the grass as 32-bit words) */
+	HIP_OK(take((void **)&b->grass_at, ((size_t)C * b->grass_bytes + 3) & ~(size_t)3));
 	b->ring_stride = b->P.R + 1;
 	HIP_OK(take((void **)&b->ring, (size_t)b->max_rep * b->ring_stride * 8));
 	HIP_OK(take((void **)&b->hist, (size_t)b->hist_alloc_words * 4));
@@ -4089,6 +4660,8 @@ static int batch_reset(pp_batch_t *b) {
 	b->free_cells[0] = b->P.C;
 	b->reserved = 0;
 	b->need_radix = 1;
+	b->form = FORM_PAIRS;
+	b->soa_fresh = 0;
 	return PP_SUCCESS;
 }
 
@@ -4117,6 +4690,7 @@ static int admit(pp_batch_t *b, const pp_params_t *p, uint64_t seed,
 	if (p->grass_restart > b->P.R || C > b->P.C) return PP_INVALID_ARGS;
 	if (reserve == 0) reserve = std::max<uint64_t>(4ull * n0, 1);
 	if (reserve < n0 || reserve > b->P.cap) return PP_INVALID_ARGS;
+	PP_TRY(to_pairs(b));
 	if (!b->ctl_fresh) PP_TRY(read_ctl(b));
 	if (b->ctl_host->error) return b->ctl_host->error;
 	const uint32_t tick = b->ctl_host->tick, pos = b->ctl_host->n;
@@ -4225,6 +4799,7 @@ static int admit(pp_batch_t *b, const pp_params_t *p, uint64_t seed,
 	prof_end(b, pe);
 	HIP_OK(hipGetLastError());
 	b->ctl_fresh = 0;
+	b->soa_fresh = 0;    /* the new agents are in no cell order */
 	if (id_out) *id_out = id;
 	return PP_SUCCESS;
 }
@@ -4471,6 +5046,9 @@ static int simulate_noalloc(const pp_params_t *p, uint64_t seed,
 	HIP_OK(hipMemcpy(&b->ctl->nrep, &one, 4, hipMemcpyHostToDevice));
 	HIP_OK(hipMemcpy(&b->ctl->nbuckets, &nb32, 4, hipMemcpyHostToDevice));
 	b->need_radix = 1;
+	b->table_nrep = 1;
+	const TileGrid tg{&rp, 0, n0};
+	tile_plan(b, &tg, 1);
 
 	const Tables T = b->tables();
 	const uint32_t cu = (uint32_t)b->num_cu;
@@ -4491,7 +5069,8 @@ static int simulate_noalloc(const pp_params_t *p, uint64_t seed,
 	HIP_OK(hipMemcpy(&rows[0], b->stats_dev, sizeof(pp_stats64_t),
 		hipMemcpyDeviceToHost));
 
-	/* Chunks of at most half the stats ring, rows copied after each. */
+	/* Chunks of at most half the stats ring, rows copied after each (less
+	 * than a chunk where the tiles stop short). */
 	uint32_t done = 0;
 	while (done < p->iters) {
 		const uint32_t chunk = min_u32(p->iters - done, b->stats_rows / 2);
@@ -4506,7 +5085,10 @@ static int simulate_noalloc(const pp_params_t *p, uint64_t seed,
 			HIP_OK(hipMemcpy(&rows[i], b->stats_dev + i % b->stats_rows,
 				sizeof(pp_stats64_t), hipMemcpyDeviceToHost));
 		if (rc.status == RS_FAILED) return rc.error;
-		if (last != done + chunk) return PP_LIBRARY_ERROR;
+		int again = 0;
+		PP_TRY(tile_settle(b, &again));
+		if (again) tile_plan(b, &tg, 1);
+		if (last != done + chunk && !again) return PP_LIBRARY_ERROR;
 		done = last;
 	}
 	return PP_SUCCESS;
@@ -4596,6 +5178,7 @@ int pp_sim_run(pp_sim_t *s, uint32_t iters, pp_stats64_t *out) {
 		if (!r) return PP_INVALID_ARGS;
 		pp_batch_t *b = s->b;
 		HIP_OK(hipSetDevice(b->device));
+		if (!b->ctl_fresh) PP_TRY(read_ctl(b));
 		if (b->ctl_host->error) return b->ctl_host->error;
 		if (r->error) return r->error;
 		const uint64_t last = (uint64_t)b->ctl_host->tick + iters + b->P.R + 1;
@@ -4606,8 +5189,7 @@ int pp_sim_run(pp_sim_t *s, uint32_t iters, pp_stats64_t *out) {
 			const uint32_t step0 = r->rows_have - 1;
 			r->sink = out ? out + done : nullptr;
 			r->sink_from = step0 + 1;
-			int rc = enqueue_ticks(b, chunk);
-			if (!rc) rc = collect(b);
+			const int rc = run_ticks(b, chunk);
 			r->sink = nullptr;
 			if (rc) return rc;
 			const uint32_t got = r->rows_have - 1 - step0;
@@ -4673,6 +5255,7 @@ int pp_sim_get_state(pp_sim_t *s, uint32_t *cell, int32_t *energy,
 		Replica *r = sim_rep(s);
 		if (!r) return PP_INVALID_ARGS;
 		HIP_OK(hipSetDevice(s->b->device));
+		PP_TRY(tiles_out(s->b));
 		PP_TRY(read_ctl(s->b));
 		return state_of(s->b, *r, cell, energy, type, grass);
 	});
@@ -4684,6 +5267,7 @@ int pp_sim_dump(pp_sim_t *s, const char *agents_path, const char *cells_path,
 		Replica *r = sim_rep(s);
 		if (!r) return PP_INVALID_ARGS;
 		HIP_OK(hipSetDevice(s->b->device));
+		PP_TRY(tiles_out(s->b));
 		PP_TRY(read_ctl(s->b));
 		if (r->slot < 0) return PP_INVALID_ARGS;
 		const uint64_t n = s->b->rctl_host[r->slot].n;
@@ -4831,6 +5415,7 @@ int pp_batch_get_state(pp_batch_t *b, uint32_t id, uint32_t *n_agents,
 		auto it = b->reps.find(id);
 		if (it == b->reps.end()) return PP_INVALID_ARGS;
 		HIP_OK(hipSetDevice(b->device));
+		PP_TRY(tiles_out(b));
 		PP_TRY(read_ctl(b));
 		const Replica &r = it->second;
 		if (r.slot < 0) return PP_INVALID_ARGS;
@@ -4949,10 +5534,11 @@ int pp_batch_tune(pp_batch_t *b, uint32_t trial_ticks, uint32_t *bucket_shift,
 		if (!b || trial_ticks == 0 || trial_ticks + 8 > b->stats_rows / 2)
 			return PP_INVALID_ARGS;
 		HIP_OK(hipSetDevice(b->device));
-		/* candidates: the bucket sort at each block width, then the radix sort
-		 * at each shape */
+		/* candidates: the automatic mode's tile step, the bucket sort at each
+		 * block width, then the radix sort at each shape */
 		struct Cand { uint32_t shift; SortShape sh; };
 		std::vector<Cand> cands;
+		cands.push_back({1, default_shape(b->key_bits)});
 		for (uint32_t sft = 8; sft <= 11; sft++) cands.push_back({sft, b->shape});
 		for (const SortShape &sh : tune_candidates(b->key_bits, b->P.cap))
 			cands.push_back({0, sh});
@@ -4978,7 +5564,8 @@ int pp_batch_tune(pp_batch_t *b, uint32_t trial_ticks, uint32_t *bucket_shift,
 			if (active_count(b) == 0) break;
 			PP_TRY(pp_batch_set_sort(b, c.shift));
 			PP_TRY(pp_batch_set_shape(b, (uint32_t)c.sh.kpt, (uint32_t)c.sh.max_bits));
-			if (c.shift && !b->P.bucket_on) continue;   /* layout too fine */
+			if (c.shift == 1 && !b->plan.on) continue;  /* no tiles: as below */
+			if (c.shift > 1 && !b->P.bucket_on) continue;   /* layout too fine */
 			double t = 0;
 			PP_TRY(trial(t));
 			if (best_t < 0 || t < best_t) {
@@ -4997,7 +5584,8 @@ int pp_batch_tune(pp_batch_t *b, uint32_t trial_ticks, uint32_t *bucket_shift,
 			const SortShape def = default_shape(b->key_bits);
 			PP_TRY(pp_batch_set_sort(b, 1));
 			PP_TRY(pp_batch_set_shape(b, (uint32_t)def.kpt, (uint32_t)def.max_bits));
-			const bool auto_wins = b->P.bucket_on ? best.shift == 11
+			const bool auto_wins = best.shift == 1 ? true : b->plan.on ? false
+				: b->P.bucket_on ? best.shift == 11
 				: (best.shift == 0 && best.sh.kpt == def.kpt &&
 					best.sh.max_bits == def.max_bits);
 			if (!auto_wins) {
@@ -5011,7 +5599,7 @@ int pp_batch_tune(pp_batch_t *b, uint32_t trial_ticks, uint32_t *bucket_shift,
 		 * or whole round. (The emit width is left to its rule, which follows
 		 * the replica set: choosing it here, in trials with every replica
 		 * running, made the 64-replica workload's run 8% slower.) */
-		if (best_t >= 0) {
+		if (best_t >= 0 && best.shift != 1) {
 			uint32_t best_r = b->tile_rounds, best_e = b->bucket_eighths;
 			double best_l = -1.0;
 			for (uint32_t r : {1u, 2u, 4u, 8u})

@@ -1,0 +1,1337 @@
+/*
+ * pp_tile.h -- the tile step: one kernel per iteration.
+ *
+ * The grid of every replica is cut into tiles of cells, one work-group each.
+ * Between iterations a tile's agents lie in its own slot of a record buffer,
+ * in id order (cells ascending, within a cell in acting order): they are the
+ * state itself, an agent's id being the number of agents before it in the
+ * replica, row by row. In one iteration a tile's group
+ *   1. reads its own agents and those of the rows (and, where a grid row is
+ *      cut into several tiles, the edge cells) next to it, moves each (one
+ *      Philox block per agent: neighbours' agents on the border are moved by
+ *      both tiles, which costs less than exchanging them would) and keeps
+ *      those that land in the tile;
+ *   2. sorts them by cell in LDS (a counting sort; agents of one cell are put
+ *      in id order when the cell acts);
+ *   3. acts on every occupied cell, the tile's grass being in LDS;
+ *   4. writes the survivors and newborns, in order, to the other record
+ *      buffer, with their number per tile, from which the next iteration
+ *      derives the ids.
+ * It replaces the three kernels of the staged step (sort, act, emit): one
+ * launch, and each agent is read once and written once. Agents move one cell
+ * along a row or a column (move_agent, pp_gpu.cl:744-821), so a tile reads no
+ * more than its four neighbours' border cells.
+ *
+ * What bounds it: on small grids the chain of one group's phases (two round
+ * trips to memory, eight barriers, and fetching some 20 KB of instructions
+ * that each wave runs through about once); on large ones the vector units.
+ * Per iteration, against the three staged kernels: 100 x 100 24.5 -> 8.2 us,
+ * 400 x 400 27.5 -> 10.5, 1600 x 1600 41 -> 18.6, 12800 x 12800 768 -> 564;
+ * 30 replicas of 1600 x 1600 402 -> 250.
+ *
+ * A tile that outgrows its LDS or border lists sets Ctl::stop; the tick
+ * after it is then not run (every group of a later launch returns), and the
+ * host goes on with smaller tiles or the staged step.
+ *
+ * Included by pp_sim.hip, inside its namespace.
+ */
+
+/* Where a replica's tiles are: tiles of bx x by cells, nbx to a grid row,
+ * nby rows of them, tile0 the first; nbx == 1: bx = the grid's width. Cell
+ * (x, r) of a tile has LDS cell index r * pitch + x. */
+struct TileRep {
+	uint32_t tile0, ntiles, nbx, nby, bx, by, shift, band0;
+	/* its constants (Rep), here so that they come with one load */
+	uint32_t slot, gx, gy, cb, t0, iters, cap, R;
+	uint32_t key0, key1, sheep_gain, wolves_gain, sheep_thr, wolves_thr;
+	uint32_t sheep_prob, wolves_prob, gxm, gxs;
+	uint32_t vec;     /* its tiles' grass is read and written 16 bytes at a time */
+};
+/* ... in the constant address space: scalar loads, placed where they are used */
+typedef __attribute__((address_space(4))) const TileRep TileRepC;
+
+__device__ __forceinline__ TileRep tile_rep(const TileRep *p, uint32_t k) {
+	const TileRepC *c = (const TileRepC *)p + k;
+	TileRep r;
+	r.tile0 = c->tile0; r.ntiles = c->ntiles; r.nbx = c->nbx; r.nby = c->nby;
+	r.bx = c->bx; r.by = c->by; r.shift = c->shift; r.band0 = c->band0;
+	r.slot = c->slot; r.gx = c->gx; r.gy = c->gy; r.cb = c->cb;
+	r.t0 = c->t0; r.iters = c->iters; r.cap = c->cap; r.R = c->R;
+	r.key0 = c->key0; r.key1 = c->key1;
+	r.sheep_gain = c->sheep_gain; r.wolves_gain = c->wolves_gain;
+	r.sheep_thr = c->sheep_thr; r.wolves_thr = c->wolves_thr;
+	r.sheep_prob = c->sheep_prob; r.wolves_prob = c->wolves_prob;
+	r.gxm = c->gxm; r.gxs = c->gxs; r.vec = c->vec;
+	return r;
+}
+
+/* Sums of one tile's iteration, for the statistics row: sheep, wolves, grass
+ * eaten, occupied cells, births, agents alive after the move, sheep energy,
+ * wolf energy. */
+struct TileStat {
+	unsigned long long v[8];
+};
+
+/* Arguments of the tile kernels. A tile's header: its records, those in its
+ * first and last row (low, high half), those in its edge lists (left, right),
+ * and where its records start. They start in the tile's slot, or, when they
+ * are more than it holds, in the spare records after the slots, taken with an
+ * atomic add: these hold as many as there may be agents at all, so that they
+ * run out only where the capacity is exceeded, too. */
+struct TileArgs {
+	const uint2 *in;       /* records: (x | r << 16, energy | V_WOLF) */
+	uint2 *out;
+	const uint4 *hin;
+	uint4 *hout;
+	const uint32_t *rin;   /* D2: per tile, the first record of each row */
+	uint32_t *rout;
+	uint32_t *idoff;       /* D2: per tile and row, id minus record index */
+	uint32_t *rtot;        /* D2: agents per replica of the table */
+	uint32_t *bsum;        /* D2: agents per band (row of tiles), two parities */
+	const TileRep *trep;
+	TileRep one;           /* the tiles of a table of one replica */
+	const uint32_t *tk;    /* table entry of each tile */
+	const uint32_t *bk;    /* table entry of each band */
+	const TileStat *sin;
+	TileStat *sout;
+	TileStat *bstat;       /* D2: per band */
+	unsigned long long *tot; /* outputs of a tick, three turns of PART_SLOTS */
+	const uint2 *ein;      /* D2: edge lists, per tile left and right */
+	uint2 *eout;
+	uint32_t *spare;       /* spare records taken, by parity */
+	uint32_t slot;         /* records of a slot */
+	uint32_t spare0;       /* first spare record */
+	uint32_t ntiles, nbands, nfin, par, rows;
+	uint32_t nmax, hmax;   /* a tile's agents; a border row's */
+};
+
+constexpr uint32_t TILE_ROWS = 64;    /* rows of a tile, D2 */
+constexpr uint32_t TILE_ECAP = 64;    /* records of an edge list */
+constexpr uint32_t TILE_RESTAMP = 32; /* ticks between re-stamps of the grass */
+
+/* The buffers (parity) that hold the current state: the parity whose tick
+ * is the later. */
+__device__ __forceinline__ uint32_t tile_cur(const Ctl *ctl) {
+	return (int32_t)(ctl->tt[1] - ctl->tt[0]) > 0 ? 1u : 0u;
+}
+
+/* Whether tick t may run: no error, and not at or past a stop. A stop set
+ * during tick t names tick t + 1 (as t + 2: 0 is none), so it does not touch
+ * the groups of tick t that start later; the first launch that does not run
+ * halts the others, which would find the tick before in their buffers. */
+__device__ __forceinline__ bool tile_runs(const Ctl *ctl, uint32_t t) {
+	/* (all loads at once, not one after another) */
+	const uint32_t stop = ctl->stop, halt = ctl->halt;
+	const int32_t error = ctl->error;
+	return (error == 0) & (halt == 0) & ((stop == 0) | ((int32_t)(t + 1 - stop) < 0));
+}
+
+/* End of tick t for the k-th replica of the table, by one work-group: sums
+ * the units' statistics (tiles, or bands of tiles), then does what
+ * end_tick_solo and k_act_scan do. Nothing happens when the replica has
+ * ended that tick already. */
+template <int NT>
+__device__ void tile_finish(const TileStat *units, uint32_t nunits, uint32_t k,
+	uint32_t t, unsigned long long *tot, Ctl *ctl, const Tables &T,
+	const Params &P, uint32_t nrep) {
+	__shared__ unsigned long long s_f[NT / WAVE][8];
+	const uint32_t tid = threadIdx.x, lane = tid & (WAVE - 1), w = tid / WAVE;
+	const uint32_t slot = nrep == 1 ? P.one_slot : T.order[k];
+	RepCtl &rc = T.rctl[slot];
+	const Rep &rp = T.rep[slot];
+	const uint32_t s = t - rp.t0;
+	const bool due = rc.status == RS_ACTIVE && rc.step == s && !ctl->error;
+	unsigned long long v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+	if (due) {
+		for (uint32_t i = tid; i < nunits; i += NT) {
+			const TileStat &u = units[i];
+#pragma unroll
+			for (int q = 0; q < 8; q++) v[q] += u.v[q];
+		}
+	}
+#pragma unroll
+	for (int i = 0; i < 8; i++) {
+		v[i] = wave_sum(v[i]);
+		if (lane == 0) s_f[w][i] = v[i];
+	}
+	__syncthreads();
+	if (w != 0) return;
+	/* the outputs of all replicas, which the agent buffers bound */
+	unsigned long long total = 0;
+	if (nrep > 1) total = wave_sum(tot[(t % 3) * PART_SLOTS + lane]);
+	unsigned long long sum = 0, a[8];
+	if (lane < 8)
+#pragma unroll 1
+		for (int q = 0; q < NT / WAVE; q++) sum += s_f[q][lane];
+#pragma unroll
+	for (int i = 0; i < 8; i++) a[i] = __shfl(sum, i);
+	if (lane != 0) return;
+	/* (the tick counts on when every replica is done) */
+	if (k == 0 && (int32_t)(t + 1 - ctl->tick) > 0) ctl->tick = t + 1;
+	if (!due) return;
+	const unsigned long long out64 = a[0] + a[1];
+	if (nrep == 1) total = out64;
+	if (total > P.cap) {
+		if (k == 0) ctl->tick = t;
+		set_error(ctl, PP_OUT_OF_RESOURCES, t, -1);
+		return;
+	}
+	const uint32_t out = (uint32_t)out64;
+	atomicAdd(&ctl->sum_live, a[5]);
+	atomicAdd(&ctl->sum_out, out64);
+	const bool over = rc.ovf == t + 1;
+	if (over || out > rp.cap) {
+		rc.status = RS_FAILED;
+		rc.error = over ? PP_ENERGY_OVERFLOW : PP_OUT_OF_RESOURCES;
+		rc.err_step = s;
+		rc.n = 0;
+		return;
+	}
+	const uint32_t M = rp.R + 1;
+	unsigned long long D = rc.dead_cells, S = rc.cd_sum;
+	S -= D;
+	const uint32_t expire = (t + 1) % M;
+	D -= rp.ring[expire];
+	rp.ring[expire] = 0;
+	const unsigned long long E = a[2];
+	rp.ring[t % M] += E;
+	D += E;
+	S += E * (unsigned long long)rp.R;
+	rc.dead_cells = D;
+	rc.cd_sum = S;
+	pp_stats64_t *row = &rp.stats[(s + 1) % rp.stats_rows];
+	row->sheep = a[0];
+	row->wolves = a[1];
+	row->grass = (unsigned long long)rp.C - D;
+	row->sheep_en = a[6];
+	row->wolves_en = a[7];
+	row->grass_en = S;
+	row->errors = 0;
+	atomicAdd(&ctl->agent_steps, (unsigned long long)rc.n);
+	atomicAdd(&ctl->sum_occ, a[3]);
+	atomicAdd(&ctl->sum_eaten, E);
+	atomicAdd(&ctl->sum_births, a[4]);
+	rc.agent_steps += rc.n;
+	rc.step = s + 1;
+	rc.n = out;
+	if (s + 1 >= rp.iters) {
+		rc.status = RS_DONE;
+		rc.n = 0;
+	}
+}
+
+/* One cell of k agents (2 <= k <= N <= 8) at LDS slots p .. p + k - 1, in
+ * registers: the steps of k_act's register path, the starting order being
+ * the agents' id order (their ranks) instead of the slots'. Written without
+ * branches (places from k on hold no agent): a wave runs through it about
+ * once, so its length is what it costs. The acted values go back to the slots
+ * in acting order. Returns whether the grass was eaten; *ovf is set by an
+ * agent above the energy limit. (Slots up to p + N - 1 are read.) */
+template <uint32_t N>
+__device__ __forceinline__ bool tile_cell(uint32_t *s_val, const uint32_t *s_id,
+	uint32_t p, uint32_t k, bool grass, uint32_t c_local, uint32_t step,
+	uint32_t key0, uint32_t key1, uint32_t sheep_gain, uint32_t wolves_gain,
+	uint32_t sheep_thr, uint32_t wolves_thr, uint32_t *ovf) {
+	static_assert(N == 4 || N == 8, "4-bit indices in one word");
+	uint32_t id[N], v0[4];
+#pragma unroll
+	for (uint32_t q = 0; q < N; q++) id[q] = lds_ld(s_id + p + q);
+	if constexpr (N == 4)
+#pragma unroll
+		for (uint32_t q = 0; q < 4; q++) v0[q] = lds_ld(s_val + p + q);
+	const uint4 w0 = pp_philox(c_local, step, PP_STREAM_SHUFFLE, 0, key0, key1);
+	uint4 w1 = make_uint4(0, 0, 0, 0);
+	if constexpr (N == 8)
+		w1 = pp_philox(c_local, step, PP_STREAM_SHUFFLE, 1, key0, key1);
+#pragma unroll
+	for (uint32_t q = 0; q < N; q++) id[q] = q < k ? id[q] : 0xFFFFFFFFu;
+	/* ranks by id: of each pair one comes first */
+	uint32_t rank[N];
+#pragma unroll
+	for (uint32_t q = 0; q < N; q++) rank[q] = 0;
+#pragma unroll
+	for (uint32_t q = 0; q < N; q++)
+#pragma unroll
+		for (uint32_t o = q + 1; o < N; o++) {
+			const uint32_t lt = id[q] < id[o] ? 1u : 0u;
+			rank[o] += lt;
+			rank[q] += 1u - lt;
+		}
+	uint32_t perm = 0;
+#pragma unroll
+	for (uint32_t q = 0; q < N; q++) perm |= q << (4 * rank[q]);
+	/* Fisher-Yates from place k - 1 down, draw m = k - 1 - i for place i */
+#pragma unroll
+	for (uint32_t i = N - 1; i >= 1; i--) {
+		const uint32_t m = k - 1 - i;
+		uint32_t word = m == 0 ? w0.x : m == 1 ? w0.y : m == 2 ? w0.z : w0.w;
+		if constexpr (N == 8) {
+			const uint32_t hi = m == 4 ? w1.x : m == 5 ? w1.y : w1.z;
+			word = m >= 4 ? hi : word;
+		}
+		const uint32_t jj = i < k ? pp_bounded(word, i + 1) : i;
+		const uint32_t x = ((perm >> (4 * i)) ^ (perm >> (4 * jj))) & 0xFu;
+		perm ^= (x << (4 * i)) | (x << (4 * jj));
+	}
+	uint32_t V[N];
+	uint32_t sheep = 0;
+	const uint32_t there = (1u << k) - 1u;
+#pragma unroll
+	for (uint32_t q = 0; q < N; q++) {
+		const uint32_t at = (perm >> (4 * q)) & 0xFu;
+		if constexpr (N == 4) {
+			const uint32_t a = (at & 1u) ? v0[1] : v0[0], b = (at & 1u) ? v0[3] : v0[2];
+			V[q] = (at & 2u) ? b : a;
+		} else {
+			V[q] = lds_ld(s_val + p + at);
+		}
+		sheep |= (V[q] & V_WOLF) ? 0u : 1u << q;
+	}
+	sheep &= there;
+	uint32_t killed = 0, g = grass ? 1u : 0u, over = 0;
+#pragma unroll
+	for (uint32_t q = 0; q < N; q++) {
+		const uint32_t v = V[q];
+		const bool acts = ((there & ~killed) >> q) & 1u, wolf = (v & V_WOLF) != 0;
+		const uint32_t prey = sheep & ~killed;
+		const uint32_t hunt = acts & wolf ? prey & (0u - prey) : 0u;
+		const uint32_t graze = acts & !wolf ? g : 0u;
+		killed |= hunt;
+		g ^= graze;
+		int32_t e = (int32_t)(v & V_ENERGY);
+		e += (int32_t)((hunt ? wolves_gain : 0u) + (graze ? sheep_gain : 0u));
+		const bool child = acts & (e > (int32_t)(wolf ? wolves_thr : sheep_thr)) &
+			((v & V_REPRO) != 0);
+		const uint32_t flags = V_CHILD | ((e & 1) ? V_ODD : 0u);
+		e -= child ? e >> 1 : 0;
+		over |= e > (int32_t)V_ENERGY ? 1u : 0u;
+		V[q] = (v & V_WOLF) | (child ? flags : 0u) | ((uint32_t)e & V_ENERGY);
+	}
+#pragma unroll
+	for (uint32_t q = 0; q < N; q++)
+		if (q < k) lds_st(s_val + p + q, V[q] | (((killed >> q) & 1u) ? V_KILLED : 0u));
+	*ovf |= over;
+	return grass && !g;
+}
+
+/* The same for a cell of any number of agents, in LDS. */
+__device__ __forceinline__ bool tile_cell_any(uint32_t *s_val_, uint32_t *s_id_,
+	uint32_t p, uint32_t k, bool grass, uint32_t c_local, uint32_t step,
+	uint32_t key0, uint32_t key1, uint32_t sheep_gain, uint32_t wolves_gain,
+	uint32_t sheep_thr, uint32_t wolves_thr, uint32_t *ovf) {
+	uint32_t *s_val = s_val_ + p, *s_id = s_id_ + p;
+	for (uint32_t i = 1; i < k; i++) {
+		const uint32_t id = lds_ld(s_id + i), v = lds_ld(s_val + i);
+		uint32_t j = i;
+		while (j > 0 && lds_ld(s_id + j - 1) > id) {
+			lds_st(s_id + j, lds_ld(s_id + j - 1));
+			lds_st(s_val + j, lds_ld(s_val + j - 1));
+			j--;
+		}
+		lds_st(s_id + j, id);
+		lds_st(s_val + j, v);
+	}
+	uint4 r = make_uint4(0, 0, 0, 0);
+	for (uint32_t i = k - 1, m = 0; i > 0; i--, m++) {
+		if ((m & 3u) == 0)
+			r = pp_philox(c_local, step, PP_STREAM_SHUFFLE, m >> 2, key0, key1);
+		const uint32_t word = (m & 3u) == 0 ? r.x : (m & 3u) == 1 ? r.y
+			: (m & 3u) == 2 ? r.z : r.w;
+		const uint32_t jj = pp_bounded(word, i + 1);
+		if (jj != i) {
+			const uint32_t a = lds_ld(s_val + i);
+			lds_st(s_val + i, lds_ld(s_val + jj));
+			lds_st(s_val + jj, a);
+		}
+	}
+	bool ate = false;
+	for (uint32_t q = 0; q < k; q++) {
+		const uint32_t v = lds_ld(s_val + q);
+		if (v & V_KILLED) continue;
+		int32_t e = (int32_t)(v & V_ENERGY);
+		uint32_t thr;
+		if (!(v & V_WOLF)) {
+			if (grass) {
+				grass = false;
+				ate = true;
+				e += (int32_t)sheep_gain;
+			}
+			thr = sheep_thr;
+		} else {
+			for (uint32_t o = 0; o < k; o++) {
+				const uint32_t u = lds_ld(s_val + o);
+				if (!(u & (V_WOLF | V_KILLED))) {
+					lds_st(s_val + o, u | V_KILLED);
+					e += (int32_t)wolves_gain;
+					break;
+				}
+			}
+			thr = wolves_thr;
+		}
+		uint32_t nv = v & V_WOLF;
+		if (e > (int32_t)thr && (v & V_REPRO)) {
+			nv |= V_CHILD | ((e & 1) ? V_ODD : 0u);
+			e -= e / 2;
+		}
+		if (e > (int32_t)V_ENERGY) *ovf = 1;
+		lds_st(s_val + q, nv | ((uint32_t)e & V_ENERGY));
+	}
+	return ate;
+}
+
+/* Geometry of one tile. */
+struct TileGeo {
+	uint32_t x0, y0, w, h;       /* its cells */
+	uint32_t up, down, left, right;
+	uint32_t pitch;
+};
+
+template <bool D2>
+__device__ __forceinline__ TileGeo tile_geo(const TileRep &tr, uint32_t lt,
+	uint32_t gx, uint32_t gy) {
+	TileGeo g;
+	const uint32_t ty = D2 ? lt / tr.nbx : lt, tx = D2 ? lt - ty * tr.nbx : 0u;
+	g.x0 = tx * tr.bx;
+	g.y0 = ty * tr.by;
+	g.w = min(tr.bx, gx - g.x0);
+	g.h = min(tr.by, gy - g.y0);
+	const uint32_t yu = ty ? ty - 1 : tr.nby - 1, yd = ty + 1 < tr.nby ? ty + 1 : 0;
+	if (D2) {
+		const uint32_t xl = tx ? tx - 1 : tr.nbx - 1, xr = tx + 1 < tr.nbx ? tx + 1 : 0;
+		g.up = tr.tile0 + yu * tr.nbx + tx;
+		g.down = tr.tile0 + yd * tr.nbx + tx;
+		g.left = tr.tile0 + ty * tr.nbx + xl;
+		g.right = tr.tile0 + ty * tr.nbx + xr;
+		g.pitch = 1u << tr.shift;
+	} else {
+		g.up = tr.tile0 + yu;
+		g.down = tr.tile0 + yd;
+		g.left = g.right = 0;
+		g.pitch = gx;
+	}
+	return g;
+}
+
+/* The tile's grass as rows of 32-bit words: one row of w * h cells (D2 false:
+ * the tile's cells are contiguous), or h rows of w cells. A row starts at any
+ * cell, so its first word may begin with cells of a neighbour (`phase`). */
+template <typename GT, bool D2>
+struct TileGrass {
+	static constexpr uint32_t VPW = 4 / sizeof(GT);
+	uint32_t start, gx, n, wpr, wsh, rows;   /* first cell, row stride, cells a row */
+	__device__ __forceinline__ TileGrass(uint32_t cell0, uint32_t gx_, uint32_t w,
+		uint32_t h, uint32_t shift) {
+		start = cell0;
+		gx = gx_;
+		n = D2 ? w : w * h;
+		rows = D2 ? h : 1u;
+		wsh = D2 ? shift - (VPW == 4 ? 2u : VPW == 2 ? 1u : 0u) : 0u;
+		wpr = 1u << wsh;
+	}
+	/* words in all, and word i: its row and place; false past the row's end */
+	__device__ __forceinline__ uint32_t words() const {
+		return D2 ? rows * (wpr + 1) : (n + VPW - 1) / VPW + 1;
+	}
+	__device__ __forceinline__ bool word(uint32_t i, uint32_t &cell, int32_t &lo,
+		uint32_t &at) const {
+		uint32_t r = 0, c = i;
+		if (D2) {
+			if (i < rows * wpr) {
+				r = i >> wsh;
+				c = i & (wpr - 1);
+			} else {
+				r = i - rows * wpr;
+				c = wpr;
+			}
+		}
+		const uint32_t s = start + r * gx, ph = s & (VPW - 1);
+		cell = (s & ~(VPW - 1)) + c * VPW;    /* global cell of the word */
+		lo = (int32_t)(c * VPW) - (int32_t)ph;  /* row cell of its first */
+		at = D2 ? r * (wpr + 1) + c : c;
+		return lo < (int32_t)n;
+	}
+	/* 16-byte chunk i of the tile (rows of 2^csh chunks): its first cell */
+	static constexpr uint32_t VPC = 16 / sizeof(GT);
+	__device__ __forceinline__ bool chunk(uint32_t i, uint32_t &cell) const {
+		if (!D2) {
+			cell = start + i * VPC;
+			return i * VPC < n;
+		}
+		const uint32_t csh = wsh - 2, r = i >> csh, x = (i & ((1u << csh) - 1)) * VPC;
+		cell = start + r * gx + x;
+		return r < rows && x < n;
+	}
+	/* LDS index (in cells) of cell (x, r); c its linear index (D2 false) */
+	__device__ __forceinline__ uint32_t index(uint32_t c, uint32_t x, uint32_t r) const {
+		if (!D2) return (start & (VPW - 1)) + c;
+		return r * (wpr + 1) * VPW + ((start + r * gx) & (VPW - 1)) + x;
+	}
+};
+
+/* One iteration of every tile (see the head of this file). Blocks
+ * [0, nfin) end the tick before for a replica each, beside the others. */
+template <typename GT, int NT, int IPT, uint32_t CELLS, bool D2, bool SOLO>
+__global__ __launch_bounds__(NT) void k_tile(TileArgs A, Ctl *ctl, Tables T,
+	Params P, uint32_t nrep, GT *grass) {
+	constexpr uint32_t AG = NT * IPT, NW = NT / WAVE;
+	constexpr uint32_t WPT = CELLS / 2 / NT;   /* counter words a thread scans */
+	using TG = TileGrass<GT, D2>;
+	constexpr uint32_t GWORDS = CELLS / TG::VPW + (D2 ? TILE_ROWS : 0u) + 1;
+	constexpr uint32_t GIT = (GWORDS + NT - 1) / NT;
+	constexpr uint32_t VIT = (CELLS / TG::VPC + NT - 1) / NT;
+	static_assert(AG <= 4096 && CELLS <= 16384, "list entries");
+	static_assert(NW * IPT <= WAVE, "one wave scans the waves' counts");
+	static_assert(WPT * NT * 2 == CELLS && WPT % 2 == 0, "counter words");
+	__shared__ __align__(16) uint32_t s_cnt[CELLS / 2 + 4];
+	__shared__ uint32_t s_val[AG + 8];
+	__shared__ uint32_t s_id[AG + 8];
+	__shared__ uint16_t s_cell[AG + 2];
+	__shared__ uint32_t s_list[AG / 2];
+	__shared__ __align__(16) uint32_t s_grass[GWORDS];
+	__shared__ uint32_t s_tmp[NW], s_sum[2 * NW], s_wt[WAVE];
+	__shared__ uint32_t s_idoff[D2 ? 3 * TILE_ROWS : 1];
+	__shared__ unsigned long long s_red[NW][8];   /* in TileStat's order */
+	__shared__ uint32_t s_nlist, s_ovf, s_go, s_edge[2];
+
+	const uint32_t tid = threadIdx.x, lane = tid & (WAVE - 1);
+	const uint32_t w = __builtin_amdgcn_readfirstlane(tid / WAVE);
+	const uint32_t tick = __builtin_amdgcn_readfirstlane(ctl->tt[A.par]);
+	if (blockIdx.x < A.nfin) {
+		const uint32_t k = blockIdx.x;
+		if (k == 0) {
+			if (tid == 0) {
+				if (tile_runs(ctl, tick)) {
+					ctl->tt[1 - A.par] = tick + 1;
+					A.spare[A.par] = 0;   /* for the next tick's outputs */
+				} else {
+					ctl->halt = 1;
+				}
+			}
+			if (!SOLO && tid < PART_SLOTS)
+				A.tot[((tick + 1) % 3) * PART_SLOTS + tid] = 0;
+		}
+		const TileRep tr = SOLO ? A.one : tile_rep(A.trep, k);
+		if (D2) tile_finish<NT>(A.bstat + tr.band0, tr.nby, k, tick - 1, A.tot, ctl, T,
+				P, nrep);
+		else tile_finish<NT>(A.sin + tr.tile0, tr.ntiles, k, tick - 1, A.tot, ctl, T, P,
+				nrep);
+		return;
+	}
+	/* groups of one XCD take neighbouring tiles (their borders are then read
+	 * through one L2) */
+	const uint32_t b = blockIdx.x - A.nfin, per = (A.ntiles + NXCD - 1) / NXCD;
+	const uint32_t tile = (b % NXCD) * per + b / NXCD;
+	if (b / NXCD >= per || tile >= A.ntiles) return;
+	const uint32_t k = SOLO ? 0u : __builtin_amdgcn_readfirstlane(A.tk[tile]);
+	const TileRep tr = SOLO ? A.one : tile_rep(A.trep, k);
+	const uint32_t gx = tr.gx, gy = tr.gy, cb = tr.cb, step = tick - tr.t0;
+	const uint32_t key0 = tr.key0, key1 = tr.key1;
+	const uint32_t c_status = T.rctl[tr.slot].status, c_ovf = T.rctl[tr.slot].ovf;
+	const uint32_t lt = tile - tr.tile0;
+	const TileGeo g = tile_geo<D2>(tr, lt, gx, gy);
+	const bool wrapx = tr.nbx == 1, wrapy = tr.nby == 1;
+	const uint4 h_own = A.hin[tile], h_up = A.hin[g.up], h_dn = A.hin[g.down];
+	/* the ids: the agents of the replica's tiles before this one */
+	uint32_t bef = 0, all = 0;
+	if (!D2) {
+		for (uint32_t i = tid; i < tr.ntiles; i += NT) {
+			const uint32_t n = A.hin[tr.tile0 + i].x;
+			all += n;
+			bef += i < lt ? n : 0u;
+		}
+	}
+	uint4 h_l = make_uint4(0, 0, 0, 0), h_r = h_l;
+	if (D2 && !wrapx) {
+		h_l = A.hin[g.left];
+		h_r = A.hin[g.right];
+	}
+	if (D2 && tid < 3 * TILE_ROWS) {
+		const uint32_t q = tid / TILE_ROWS, r = tid % TILE_ROWS;
+		if (r < g.h) {
+			const uint32_t tl = g.left, tg = g.right;
+			uint32_t t = tile;
+			if (q == 1) t = tl;
+			if (q == 2) t = tg;
+			s_idoff[tid] = A.idoff[t * A.rows + r];
+		}
+	}
+	/* the grass, requested now and staged in LDS after the records are: 16
+	 * bytes at a time where rows start and end at multiples of that (a cell's
+	 * LDS index is then its cell index), else by words */
+	const TG G(cb + g.y0 * gx + g.x0, gx, g.w, g.h, tr.shift);
+	const uint32_t gwords = G.words();
+	const bool vec = tr.vec != 0;
+	uint4 gq[VIT];
+	uint32_t gw[GIT];
+	if (vec) {
+#pragma unroll
+		for (uint32_t i = 0; i < VIT; i++) {
+			uint32_t cell;
+			gq[i] = make_uint4(0, 0, 0, 0);
+			if (G.chunk(i * NT + tid, cell))
+				gq[i] = *reinterpret_cast<const uint4 *>(&grass[cell]);
+		}
+	} else {
+#pragma unroll
+		for (uint32_t i = 0; i < GIT; i++) {
+			uint32_t cell, at;
+			int32_t lo;
+			const uint32_t q = i * NT + tid;
+			gw[i] = 0;
+			if (q < gwords && G.word(q, cell, lo, at))
+				gw[i] = *reinterpret_cast<const uint32_t *>(&grass[cell]);
+		}
+	}
+	for (uint32_t i = tid; i < CELLS / 8 + 1; i += NT)
+		*reinterpret_cast<uint4 *>(s_cnt + 4 * i) = make_uint4(0, 0, 0, 0);
+	if (tid < WAVE) s_wt[tid] = 0;
+	if (tid == 0) {
+		s_nlist = 0;
+		s_ovf = 0;
+		s_edge[0] = s_edge[1] = 0;
+		/* A replica that is done or has failed no longer moves. Its status
+		 * is that before or after the end of the last tick, written beside
+		 * this: both give the same answer. (One thread decides for the
+		 * group: an energy limit or an error may be noted meanwhile.) */
+		s_go = tile_runs(ctl, tick) & (c_status == RS_ACTIVE) & (step < tr.iters) &
+			((c_ovf == 0) | (c_ovf == tick + 1));
+	}
+	uint32_t idb = 0, idb_up = 0, idb_dn = 0, total_in;
+	if (!D2) {
+		all = wave_sum32(all);
+		bef = wave_sum32(bef);
+		if (lane == 0) {
+			s_sum[2 * w] = all;
+			s_sum[2 * w + 1] = bef;
+		}
+	}
+	__syncthreads();
+	if (!D2) {
+		uint32_t a = 0, c = 0;
+#pragma unroll
+		for (uint32_t i = 0; i < NW; i++) {
+			a += s_sum[2 * i];
+			c += s_sum[2 * i + 1];
+		}
+		total_in = __builtin_amdgcn_readfirstlane(a);
+		idb = __builtin_amdgcn_readfirstlane(c);
+	} else {
+		total_in = __builtin_amdgcn_readfirstlane(A.rtot[k]);
+	}
+	if (!s_go || total_in > tr.cap || total_in > P.cap) return;
+
+	const uint32_t n0 = __builtin_amdgcn_readfirstlane(h_own.x);
+	const uint32_t nup = wrapy ? 0u : __builtin_amdgcn_readfirstlane(h_up.y >> 16);
+	const uint32_t ndn = wrapy ? 0u : __builtin_amdgcn_readfirstlane(h_dn.y & 0xFFFFu);
+	const uint32_t nl = D2 ? __builtin_amdgcn_readfirstlane(h_l.z >> 16) : 0u;
+	const uint32_t nr = D2 ? __builtin_amdgcn_readfirstlane(h_r.z & 0xFFFFu) : 0u;
+	const uint32_t i1 = n0, i2 = i1 + nup, i3 = i2 + ndn, i4 = i3 + nl, i5 = i4 + nr;
+	if (i5 > AG) {
+		/* (the limits set when the records were written exclude this) */
+		if (tid == 0) set_error(ctl, PP_LIBRARY_ERROR, tick, (int32_t)tile);
+		return;
+	}
+	/* positions and ids of the ranges, as offsets from the item index */
+	const uint32_t first_up = __builtin_amdgcn_readfirstlane(h_up.x) - nup;
+	const uint32_t p_own = __builtin_amdgcn_readfirstlane(h_own.w);
+	const uint32_t p_up = __builtin_amdgcn_readfirstlane(h_up.w) + first_up - i1;
+	const uint32_t p_dn = __builtin_amdgcn_readfirstlane(h_dn.w) - i2;
+	uint32_t p_l = 0, p_r = 0;
+	if (!D2) {
+		idb_up = (lt ? idb - __builtin_amdgcn_readfirstlane(h_up.x)
+			: total_in - __builtin_amdgcn_readfirstlane(h_up.x)) + first_up - i1;
+		idb_dn = (lt + 1 < tr.ntiles ? idb + n0 : 0u) - i2;
+	} else {
+		const uint32_t uh = min(tr.by, gy - (g.y0 ? g.y0 - tr.by : (tr.nby - 1) * tr.by));
+		idb_up = __builtin_amdgcn_readfirstlane(A.idoff[g.up * A.rows + uh - 1])
+			+ first_up - i1;
+		idb_dn = __builtin_amdgcn_readfirstlane(A.idoff[g.down * A.rows]) - i2;
+		/* the right list of the tile left of this one, and vice versa */
+		p_l = (2 * g.left + 1) * TILE_ECAP - i3;
+		p_r = 2 * g.right * TILE_ECAP - i4;
+	}
+	uint2 rec[IPT];
+	uint32_t pk[IPT], vv[IPT], ids[IPT];
+#pragma unroll
+	for (int j = 0; j < IPT; j++) {
+		rec[j] = make_uint2(0u, 0u);
+		pk[j] = 0xFFFFFFFFu;
+		vv[j] = ids[j] = 0;
+	}
+#pragma unroll
+	for (int j = 0; j < IPT; j++) {
+		if ((uint32_t)j * NT >= i5) break;   /* (uniform: no more rounds) */
+		const uint32_t i = j * NT + tid;
+		if ((uint32_t)(j + 1) * NT <= i1) {
+			rec[j] = A.in[p_own + i];     /* a round of own agents */
+		} else if (i < i5) {
+			uint32_t p = i < i1 ? p_own : i < i2 ? p_up : p_dn;
+			if (D2 && i >= i3) p = i < i4 ? p_l : p_r;
+			const uint2 *src = D2 && i >= i3 ? A.ein : A.in;
+			rec[j] = src[(uint32_t)(p + i)];
+		}
+	}
+	/* grass to LDS: arrived before the records, in issue order */
+	if (vec) {
+#pragma unroll
+		for (uint32_t i = 0; i < VIT; i++)
+			if (VIT * NT * TG::VPC <= CELLS || i * NT + tid < CELLS / TG::VPC)
+				reinterpret_cast<uint4 *>(s_grass)[i * NT + tid] = gq[i];
+	} else {
+#pragma unroll
+		for (uint32_t i = 0; i < GIT; i++) {
+			uint32_t cell, at;
+			int32_t lo;
+			const uint32_t q = i * NT + tid;
+			if (q < gwords && G.word(q, cell, lo, at)) s_grass[at] = gw[i];
+		}
+	}
+
+	/* 1. the moves; an agent that lands is counted in its cell and keeps its
+	 * place among the cell's arrivals */
+#pragma unroll
+	for (int j = 0; j < IPT; j++) {
+		if ((uint32_t)j * NT >= i5) break;
+		const uint32_t i = j * NT + tid;
+		if (i >= i5) continue;
+		int32_t x = (int32_t)(rec[j].x & 0xFFFFu), r = (int32_t)(rec[j].x >> 16);
+		uint32_t id = i + (D2 ? s_idoff[r] : idb);
+		if ((uint32_t)(j + 1) * NT > i1) {
+			/* a round with neighbours' agents */
+			if (!D2) {
+				id = i + (i < i1 ? idb : i < i2 ? idb_up : idb_dn);
+				r = i < i1 ? r : i < i2 ? -1 : (int32_t)g.h;
+			} else if (i >= i3) {
+				/* an edge record's x is its index among its tile's records */
+				id = (uint32_t)x + s_idoff[(i < i4 ? 1u : 2u) * TILE_ROWS + (uint32_t)r];
+				x = i < i4 ? -1 : (int32_t)g.w;
+			} else if (i >= i1) {
+				id = i + (i < i2 ? idb_up : idb_dn);
+				r = i < i2 ? -1 : (int32_t)g.h;
+			}
+		}
+		const uint4 d4 = pp_philox(id, step, PP_STREAM_MOVE, 0, key0, key1);
+		const uint32_t dice = pp_bounded(d4.y, 100);
+		/* the direction's steps along x and y, from tables of 2-bit signed
+		 * entries: 0, 1, -1, 0, 0 and 0, 0, 0, 1, -1 */
+		const uint32_t dir2 = 2 * pp_bounded(d4.x, 5);
+		x += __builtin_amdgcn_sbfe(0x34, dir2, 2);
+		r += __builtin_amdgcn_sbfe(0x340, dir2, 2);
+		if (wrapx) x = x < 0 ? (int32_t)g.w - 1 : x == (int32_t)g.w ? 0 : x;
+		if (wrapy) r = r < 0 ? (int32_t)g.h - 1 : r == (int32_t)g.h ? 0 : r;
+		/* it loses one energy, and dies below one */
+		const uint32_t y = rec[j].y;
+		if (((y & V_ENERGY) < 2) | ((uint32_t)x >= g.w) | ((uint32_t)r >= g.h)) continue;
+		const uint32_t c = __umul24((uint32_t)r, g.pitch) + (uint32_t)x, sh = (c & 1u) * 16;
+		const uint32_t old = atomicAdd(&s_cnt[c >> 1], 1u << sh);
+		pk[j] = c | (((old >> sh) & 0xFFFFu) << 16);
+		vv[j] = (y - 1) | (dice < ((y & V_WOLF) ? tr.wolves_prob : tr.sheep_prob) ?
+			V_REPRO : 0u);
+		ids[j] = id;
+	}
+	__syncthreads();
+
+	/* 2. first slot of every cell, then the agents to their slots */
+	uint32_t L;
+	{
+		uint32_t v[WPT];
+		uint2 *p2 = reinterpret_cast<uint2 *>(s_cnt + WPT * tid);
+#pragma unroll
+		for (uint32_t i = 0; i < WPT / 2; i++) {
+			const uint2 u = p2[i];
+			v[2 * i] = u.x;
+			v[2 * i + 1] = u.y;
+		}
+		uint32_t sum = 0;
+#pragma unroll
+		for (uint32_t i = 0; i < WPT; i++) sum += v[i];
+		sum = (sum & 0xFFFFu) + (sum >> 16);
+		const uint32_t x = wave_incl_scan32(sum);
+		if (lane == WAVE - 1) s_tmp[w] = x;
+		__syncthreads();
+		uint32_t run = x - sum, tot = 0;
+#pragma unroll
+		for (uint32_t i = 0; i < NW; i++) {
+			const uint32_t t = s_tmp[i];
+			run += i < w ? t : 0u;
+			tot += t;
+		}
+		L = __builtin_amdgcn_readfirstlane(tot);
+#pragma unroll
+		for (uint32_t i = 0; i < WPT / 2; i++) {
+			uint32_t o[2];
+#pragma unroll
+			for (uint32_t q = 0; q < 2; q++) {
+				const uint32_t lo = v[2 * i + q] & 0xFFFFu;
+				o[q] = run | ((run + lo) << 16);
+				run += lo + (v[2 * i + q] >> 16);
+			}
+			p2[i] = make_uint2(o[0], o[1]);
+		}
+		if (tid == 0) s_cnt[CELLS / 2] = L;
+	}
+	__syncthreads();
+	const uint16_t *s_start = reinterpret_cast<const uint16_t *>(s_cnt);
+#pragma unroll
+	for (int j = 0; j < IPT; j++) {
+		if ((uint32_t)j * NT >= i5) break;
+		if (pk[j] == 0xFFFFFFFFu) continue;
+		const uint32_t c = pk[j] & 0xFFFFu, q = s_start[c] + (pk[j] >> 16);
+		s_val[q] = vv[j];
+		s_id[q] = ids[j];
+		s_cell[q + 1] = (uint16_t)c;
+	}
+	if (tid == 0) {
+		s_cell[0] = 0xFFFFu;
+		s_cell[L + 1] = 0xFFFFu;
+	}
+	__syncthreads();
+
+	/* 3. actions: cells of one agent in place, the others listed and then
+	 * acted on by consecutive lanes */
+	const uint32_t sheep_gain = tr.sheep_gain, wolves_gain = tr.wolves_gain;
+	const uint32_t sheep_thr = tr.sheep_thr, wolves_thr = tr.wolves_thr, R = tr.R;
+	GT *s_g = reinterpret_cast<GT *>(s_grass);
+	/* x and row of a cell index */
+	auto cell_xr = [&](uint32_t c, uint32_t &x, uint32_t &r) {
+		if (D2) {
+			r = c >> tr.shift;
+			x = c & (g.pitch - 1);
+		} else {
+			r = div_by(c, tr.gxm, tr.gxs);
+			x = c - r * gx;
+		}
+	};
+	/* (this loop and those below are not unrolled: a group runs through the
+	 * code about once, and fetching instructions is then what takes the time) */
+	uint32_t eaten = 0, ovf = 0;
+#pragma unroll 1
+	for (uint32_t p = tid; p < L; p += NT) {
+		const uint32_t c = s_cell[p + 1];
+		if (s_cell[p] == c) continue;
+		eaten += 1u << 16;     /* high half: occupied cells */
+		if (s_cell[p + 2] == c) {
+			/* slot, cell and agents (63: that many or more) */
+			const uint32_t kk = s_start[c + 1] - p;
+			s_list[atomicAdd(&s_nlist, 1u)] = p | (c << 12) | (min(kk, 63u) << 26);
+			continue;
+		}
+		const uint32_t v = s_val[p];
+		int32_t e = (int32_t)(v & V_ENERGY);
+		uint32_t thr = wolves_thr;
+		if (!(v & V_WOLF)) {
+			thr = sheep_thr;
+			uint32_t gi = c;
+			if (D2 && !vec) {
+				uint32_t x, r;
+				cell_xr(c, x, r);
+				gi = G.index(c, x, r);
+			} else if (!vec) {
+				gi = G.index(c, 0, 0);
+			}
+			if (grass_alive_at<GT>(s_g[gi], tick + 1, P.R)) {
+				e += (int32_t)sheep_gain;
+				s_g[gi] = (GT)(tick + 1 + R);
+				eaten++;
+			}
+		}
+		uint32_t nv = v & V_WOLF;
+		if (e > (int32_t)thr && (v & V_REPRO)) {
+			nv |= V_CHILD | ((e & 1) ? V_ODD : 0u);
+			e -= e / 2;
+		}
+		if (e > (int32_t)V_ENERGY) ovf = 1;
+		s_val[p] = nv | ((uint32_t)e & V_ENERGY);
+	}
+	__syncthreads();
+	{
+		const uint32_t nlist = s_nlist;
+#pragma unroll 1
+		for (uint32_t i = tid; i < nlist; i += NT) {
+			const uint32_t en = s_list[i], p = en & 0xFFFu, c = (en >> 12) & 0x3FFFu;
+			uint32_t kk = en >> 26, cl, gi;
+			if (kk == 63) kk = s_start[c + 1] - p;
+			if (D2) {
+				uint32_t x, r;
+				cell_xr(c, x, r);
+				cl = (g.y0 + r) * gx + g.x0 + x;
+				gi = vec ? c : G.index(c, x, r);
+			} else {
+				cl = g.y0 * gx + c;
+				gi = vec ? c : G.index(c, 0, 0);
+			}
+			const bool alive = grass_alive_at<GT>(s_g[gi], tick + 1, P.R);
+			bool ate;
+			if (kk <= 4)
+				ate = tile_cell<4>(s_val, s_id, p, kk, alive, cl, step, key0, key1,
+					sheep_gain, wolves_gain, sheep_thr, wolves_thr, &ovf);
+			else if (kk <= 8)
+				ate = tile_cell<8>(s_val, s_id, p, kk, alive, cl, step, key0, key1,
+					sheep_gain, wolves_gain, sheep_thr, wolves_thr, &ovf);
+			else
+				ate = tile_cell_any(s_val, s_id, p, kk, alive, cl, step, key0, key1,
+					sheep_gain, wolves_gain, sheep_thr, wolves_thr, &ovf);
+			if (ate) {
+				s_g[gi] = (GT)(tick + 1 + R);
+				eaten++;
+			}
+		}
+	}
+	if (ovf) s_ovf = 1;
+	__syncthreads();
+
+	/* 4. the outputs of each slot and their offsets: slot order is (j, wave,
+	 * lane), so ballots give the place in the wave and one scan over the
+	 * waves' counts the rest */
+	uint32_t n_all = 0, n_wolves = 0, e_all = 0, e_wolves = 0, n_birth = 0;
+	const uint32_t rounds = (L + NT - 1) / NT;
+#pragma unroll 1
+	for (uint32_t j = 0; j < rounds; j++) {
+		const uint32_t p = j * NT + tid;
+		const uint32_t v = p < L ? s_val[p] : V_KILLED;
+		const bool surv = !(v & V_KILLED), child = (v & V_CHILD) != 0;
+		const bool wolf = (v & V_WOLF) != 0;
+		const uint64_t bs = __ballot(surv), bc = __ballot(child), bw = __ballot(wolf);
+		const uint32_t nb = (uint32_t)__popcll(bc), n = nb + (uint32_t)__popcll(bs);
+		if (lane == 0) s_wt[j * NW + w] = n;
+		n_all += n;
+		n_birth += nb;
+		n_wolves += (uint32_t)(__popcll(bs & bw) + __popcll(bc & bw));
+		const uint32_t e = v & V_ENERGY;
+		const uint32_t en = (surv ? e : 0u) + (child ? e - ((v & V_ODD) ? 1u : 0u) : 0u);
+		e_all += en;
+		e_wolves += wolf ? en : 0u;
+	}
+	{
+		const uint32_t ne = wave_sum32(eaten);
+		unsigned long long ea, ew;
+		/* (a lane's sums stay below 2^(24 + 5)) */
+		if (__ballot((e_all >> 26) != 0) == 0) {
+			ea = wave_sum32(e_all);
+			ew = wave_sum32(e_wolves);
+		} else {
+			ea = wave_sum((unsigned long long)e_all);
+			ew = wave_sum((unsigned long long)e_wolves);
+		}
+		if (lane == 0) {
+			s_red[w][0] = n_all - n_wolves;
+			s_red[w][1] = n_wolves;
+			s_red[w][2] = ne & 0xFFFFu;
+			s_red[w][3] = ne >> 16;
+			s_red[w][4] = n_birth;
+			s_red[w][5] = w == 0 ? L : 0u;
+			s_red[w][6] = ea - ew;
+			s_red[w][7] = ew;
+		}
+	}
+	__syncthreads();
+	const uint32_t wt = s_wt[lane];
+	const uint32_t wi = wave_incl_scan32(wt);
+	const uint32_t nout = (uint32_t)__builtin_amdgcn_readlane((int)wi, WAVE - 1);
+	uint32_t o_at = tile * A.slot, o_max = nout;
+	if (nout > A.slot) {
+		if (tid == 0) s_tmp[0] = atomicAdd(&A.spare[1 - A.par], nout);
+		__syncthreads();
+		const uint32_t q = s_tmp[0];
+		/* (past the spare records only with more agents than the capacity:
+		 * the batch then fails, and nothing is written) */
+		if (q + nout > P.cap) o_max = 0;
+		o_at = A.spare0 + (o_max ? q : 0u);
+	}
+	o_at = __builtin_amdgcn_readfirstlane(o_at);
+	uint2 *o_rec = A.out + o_at;
+	uint2 *o_edge = D2 ? A.eout + 2 * TILE_ECAP * tile : nullptr;
+#pragma unroll 1
+	for (uint32_t j = 0; j < rounds; j++) {
+		const uint32_t p = j * NT + tid;
+		const bool in = p < L;
+		const uint32_t v = in ? s_val[p] : V_KILLED;
+		const uint64_t bs = __ballot(!(v & V_KILLED)), bc = __ballot((v & V_CHILD) != 0);
+		uint32_t o = __builtin_amdgcn_mbcnt_hi((uint32_t)(bs >> 32),
+			__builtin_amdgcn_mbcnt_lo((uint32_t)bs,
+			__builtin_amdgcn_mbcnt_hi((uint32_t)(bc >> 32),
+			__builtin_amdgcn_mbcnt_lo((uint32_t)bc, 0u))));
+		o += (uint32_t)__builtin_amdgcn_readlane((int)(wi - wt), (int)(j * NW + w));
+		if (!in) continue;
+		s_id[p] = o;   /* (the ids are no longer needed) */
+		uint32_t x, r;
+		cell_xr(s_cell[p + 1], x, r);
+		const uint32_t rx = x | (r << 16);
+		const uint32_t y = v & (V_ENERGY | V_WOLF);
+		auto put = [&](uint32_t y) {
+			if (o < o_max) at32(o_rec, o) = make_uint2(rx, y);
+			if (D2 && !wrapx) {
+				/* edge lists of the neighbours left and right */
+				const uint2 er = make_uint2(o | (r << 16), y);
+				if (x == 0) {
+					const uint32_t q = atomicAdd(&s_edge[0], 1u);
+					if (q < TILE_ECAP) o_edge[q] = er;
+				}
+				if (x == g.w - 1) {
+					const uint32_t q = atomicAdd(&s_edge[1], 1u);
+					if (q < TILE_ECAP) o_edge[TILE_ECAP + q] = er;
+				}
+			}
+			o++;
+		};
+		if (!(v & V_KILLED)) put(y);
+		if (v & V_CHILD) put(y - ((v & V_ODD) ? 1u : 0u));
+	}
+	/* the grass back; alive cells are re-stamped now and then (see REFRESH) */
+	const bool restamp = tick % TILE_RESTAMP == 0;
+	auto stamped = [&](uint32_t v) {
+		GT gv[TG::VPW];
+		__builtin_memcpy(gv, &v, 4);
+#pragma unroll
+		for (uint32_t u = 0; u < TG::VPW; u++)
+			if (grass_alive_at<GT>(gv[u], tick + 1, P.R)) gv[u] = (GT)(tick + 1);
+		__builtin_memcpy(&v, gv, 4);
+		return v;
+	};
+	if (vec) {
+#pragma unroll 1
+		for (uint32_t i = tid; i < CELLS / TG::VPC; i += NT) {
+			uint32_t cell;
+			if (!G.chunk(i, cell)) continue;
+			uint4 v = reinterpret_cast<const uint4 *>(s_grass)[i];
+			if (restamp)
+				v = make_uint4(stamped(v.x), stamped(v.y), stamped(v.z), stamped(v.w));
+			*reinterpret_cast<uint4 *>(&grass[cell]) = v;
+		}
+	} else {
+#pragma unroll 1
+		for (uint32_t q = tid; q < gwords; q += NT) {
+			uint32_t cell, at;
+			int32_t lo;
+			if (!G.word(q, cell, lo, at)) continue;
+			uint32_t v = s_grass[at];
+			if (restamp) v = stamped(v);
+			if (lo >= 0 && (uint32_t)lo + TG::VPW <= G.n) {
+				*reinterpret_cast<uint32_t *>(&grass[cell]) = v;
+			} else {
+				GT gv[TG::VPW];
+				__builtin_memcpy(gv, &v, 4);
+#pragma unroll
+				for (uint32_t u = 0; u < TG::VPW; u++)
+					if (lo + (int32_t)u >= 0 && (uint32_t)(lo + (int32_t)u) < G.n)
+						grass[cell + u] = gv[u];
+			}
+		}
+	}
+	__syncthreads();
+	/* first record of each row (the output offset of the row's first slot) */
+	auto row_first = [&](uint32_t r) {
+		const uint32_t q = s_start[r * g.pitch];
+		return q < L ? s_id[q] : nout;
+	};
+	if (D2)
+		for (uint32_t r = tid; r <= g.h; r += NT)
+			A.rout[(size_t)tile * (A.rows + 1) + r] = r < g.h ? row_first(r) : nout;
+	if (tid < 8) {
+		unsigned long long v = 0;
+#pragma unroll 4
+		for (uint32_t i = 0; i < NW; i++) v += s_red[i][tid];
+		A.sout[tile].v[tid] = v;
+	}
+	if (tid == 0) {
+		const uint32_t nf = g.h > 1 ? row_first(1) : nout;
+		const uint32_t nla = g.h > 1 ? nout - row_first(g.h - 1) : nout;
+		const uint32_t el = D2 ? s_edge[0] : 0u, er = D2 ? s_edge[1] : 0u;
+		A.hout[tile] = make_uint4(nout, nf | (nla << 16), min(el, TILE_ECAP) |
+			(min(er, TILE_ECAP) << 16), o_at);
+		if (nout > A.nmax || nf > A.hmax || nla > A.hmax || el > TILE_ECAP ||
+			er > TILE_ECAP)
+			ctl->stop = tick + 2;
+		if (s_ovf) T.rctl[tr.slot].ovf = tick + 1;
+		if (!SOLO)
+			atomicAdd(&A.tot[(tick % 3) * PART_SLOTS + tile % PART_SLOTS],
+				(unsigned long long)nout);
+		if (D2)
+			atomicAdd(&A.bsum[(1 - A.par) * A.nbands + tr.band0 + lt / tr.nbx], nout);
+	}
+}
+
+/* After an iteration of tiles that cut grid rows (D2): one work-group per
+ * band (row of tiles) turns the agents per tile row into ids: the bands
+ * before it, then a scan over the band's rows, tile by tile; also the band's
+ * statistics, and the replica's agents (last band). */
+__global__ __launch_bounds__(WG) void k_tile_scan(TileArgs A, Ctl *ctl, Tables T,
+	uint32_t nrep) {
+	const bool SOLO = nrep == 1;
+	__shared__ uint32_t s_tmp[NWAVE];
+	/* only after a tick that ran */
+	if (ctl->error || ctl->halt || ctl->tt[1 - A.par] != ctl->tt[A.par] + 1) return;
+	const uint32_t band = blockIdx.x, tid = threadIdx.x;
+	const uint32_t lane = tid & (WAVE - 1), w = tid / WAVE;
+	const uint32_t k = nrep == 1 ? 0u : A.bk[band];
+	const TileRep tr = SOLO ? A.one : tile_rep(A.trep, k);
+	const Rep &rp = T.rep[T.order[k]];
+	const uint32_t ty = band - tr.band0;
+	const uint32_t h = min(tr.by, rp.gy - ty * tr.by);
+	const uint32_t *bs = A.bsum + (1 - A.par) * A.nbands + tr.band0;
+	uint32_t base = 0;
+	for (uint32_t i = tid; i < ty; i += WG) base += bs[i];
+	uint32_t tot;
+	(void)wg_excl_scan<WG>(base, s_tmp, tot);
+	base = tot;
+	const uint32_t t0 = tr.tile0 + ty * tr.nbx;
+	for (uint32_t e0 = 0; e0 < h * tr.nbx; e0 += WG) {
+		const uint32_t e = e0 + tid;
+		uint32_t cnt = 0, first = 0, r = 0, t = 0;
+		if (e < h * tr.nbx) {
+			r = e / tr.nbx;
+			t = t0 + (e - r * tr.nbx);
+			const uint32_t *rs = A.rout + (size_t)t * (A.rows + 1) + r;
+			first = rs[0];
+			cnt = rs[1] - first;
+		}
+		const uint32_t x = wg_excl_scan<WG>(cnt, s_tmp, tot);
+		if (e < h * tr.nbx) A.idoff[t * A.rows + r] = base + x - first;
+		base += tot;
+	}
+	if (tid == 0) {
+		if (ty + 1 == tr.nby) A.rtot[k] = base;
+		A.bsum[A.par * A.nbands + band] = 0;
+	}
+	__shared__ unsigned long long s_f[NWAVE][8];
+	unsigned long long v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+	for (uint32_t i = tid; i < tr.nbx; i += WG) {
+		const TileStat &u = A.sout[t0 + i];
+#pragma unroll
+		for (int q = 0; q < 8; q++) v[q] += u.v[q];
+	}
+#pragma unroll
+	for (int i = 0; i < 8; i++) {
+		v[i] = wave_sum(v[i]);
+		if (lane == 0) s_f[w][i] = v[i];
+	}
+	__syncthreads();
+	if (tid < 8) {
+		unsigned long long a = 0;
+		for (int q = 0; q < NWAVE; q++) a += s_f[q][tid];
+		A.bstat[band].v[tid] = a;
+	}
+}
+
+/* The end of the last tick run, one work-group per replica of the table. A
+ * holds the buffers by parity: in/hin/sin parity 0, out/hout/sout parity 1. */
+template <bool D2>
+__global__ __launch_bounds__(WG) void k_tile_end(TileArgs A, Ctl *ctl, Tables T,
+	Params P, uint32_t nrep) {
+	const bool SOLO = nrep == 1;
+	if (ctl->error) return;
+	const uint32_t cur = tile_cur(ctl), tick = ctl->tt[cur], k = blockIdx.x;
+	const TileRep tr = SOLO ? A.one : tile_rep(A.trep, k);
+	const TileStat *st = cur ? A.sout : A.sin;
+	tile_finish<WG>(D2 ? A.bstat + tr.band0 : st + tr.tile0,
+		D2 ? tr.nby : tr.ntiles, k, tick - 1, A.tot, ctl, T, P, nrep);
+}
+
+/* Batch positions of the replicas' agents, in table order (the SoA state),
+ * and their number. One wave. */
+__global__ __launch_bounds__(WAVE) void k_tile_base(Ctl *ctl, Tables T,
+	uint32_t nrep) {
+	const uint32_t lane = threadIdx.x;
+	uint32_t carry = 0;
+	for (uint32_t k0 = 0; k0 < nrep; k0 += WAVE) {
+		const uint32_t k = k0 + lane;
+		uint32_t n = 0, slot = 0;
+		if (k < nrep) {
+			slot = T.order[k];
+			n = T.rctl[slot].status == RS_ACTIVE ? T.rctl[slot].n : 0u;
+		}
+		const uint32_t x = wave_incl_scan32(n);
+		if (k < nrep) T.rctl[slot].base = carry + x - n;
+		carry += (uint32_t)__builtin_amdgcn_readlane((int)x, WAVE - 1);
+	}
+	if (lane == 0) ctl->n = carry;
+}
+
+/* Before k_tiles_in: no stop, and the bands' sums (both parities) at zero. */
+__global__ __launch_bounds__(WG) void k_tile_clear(TileArgs A, Ctl *ctl) {
+	const uint32_t i = blockIdx.x * WG + threadIdx.x;
+	if (i == 0) ctl->stop = ctl->halt = 0;
+	if (i < 2) A.spare[i] = 0;
+	if (i < 2 * A.nbands) A.bsum[i] = 0;
+}
+
+/* Re-stamps the alive cells of [c0, c1) with the tick (see REFRESH). */
+template <typename GT>
+__device__ __forceinline__ void tile_restamp(GT *grass, uint32_t c0, uint32_t n,
+	uint32_t tick, uint32_t R) {
+	for (uint32_t i = threadIdx.x; i < n; i += WG) {
+		GT &c = grass[(size_t)c0 + i];
+		if (grass_alive_at<GT>(c, tick, R)) c = (GT)tick;
+	}
+}
+
+/* The SoA state (sorted by cell within each replica) into the tiles' slots
+ * (parity 0). */
+template <typename GT, bool D2>
+__global__ __launch_bounds__(WG) void k_tiles_in(TileArgs A, Ctl *ctl, Tables T,
+	Params P, uint32_t nrep, GT *grass, const uint32_t *cell,
+	const int32_t *energy, const uint8_t *type) {
+	const bool SOLO = nrep == 1;
+	__shared__ uint32_t s_lo[D2 ? TILE_ROWS : 1], s_n[D2 ? TILE_ROWS + 1 : 1];
+	__shared__ uint32_t s_b[4], s_edge[2];
+	if (ctl->error) return;
+	const uint32_t tid = threadIdx.x, tile = blockIdx.x, tick = ctl->tick;
+	if (tile == 0) {
+		if (tid == 0) {
+			ctl->tt[0] = tick;
+			ctl->tt[1] = tick - 1;
+			ctl->in_tick = tick;
+		}
+		if (tid < PART_SLOTS)
+			for (uint32_t i = 0; i < 3; i++) A.tot[i * PART_SLOTS + tid] = 0;
+	}
+	const uint32_t k = nrep == 1 ? 0u : A.tk[tile];
+	const uint32_t slot = T.order[k];
+	const Rep &rp = T.rep[slot];
+	const RepCtl &rc = T.rctl[slot];
+	const TileRep tr = SOLO ? A.one : tile_rep(A.trep, k);
+	const TileGeo g = tile_geo<D2>(tr, tile - tr.tile0, rp.gx, rp.gy);
+	const uint32_t base = rc.base, n = rc.status == RS_ACTIVE ? rc.n : 0u;
+	/* agents of the replica before cell c */
+	auto lower = [&](uint32_t c) {
+		uint32_t lo = 0, hi = n;
+		while (lo < hi) {
+			const uint32_t mid = (lo + hi) / 2;
+			if (cell[base + mid] < c) lo = mid + 1;
+			else hi = mid;
+		}
+		return lo;
+	};
+	uint2 *o_edge = D2 ? const_cast<uint2 *>(A.ein) + 2 * TILE_ECAP * tile : nullptr;
+	if (tid < 2) s_edge[tid] = 0;
+	uint32_t nout, nf, nl;
+	/* the slot, or spare records, for nout agents (a tile above the limits
+	 * keeps none of them: the SoA state stays the valid one) */
+	auto place = [&](uint32_t n_) {
+		if (tid == 0) {
+			uint32_t q = tile * A.slot;
+			if (n_ > A.slot && n_ <= A.nmax) q = A.spare0 + atomicAdd(&A.spare[0], n_);
+			s_b[0] = q;
+		}
+		__syncthreads();
+		return s_b[0];
+	};
+	uint32_t o_at;
+	if (!D2) {
+		/* row bounds of the tile, its second and its last row */
+		if (tid < 4) {
+			const uint32_t r = tid == 0 ? 0u : tid == 1 ? 1u : tid == 2 ? g.h - 1 : g.h;
+			s_b[tid] = lower(rp.cb + (g.y0 + r) * rp.gx);
+		}
+		__syncthreads();
+		nout = s_b[3] - s_b[0];
+		nf = s_b[1] - s_b[0];
+		nl = s_b[3] - s_b[2];
+		const uint32_t lo = s_b[0], take = nout > A.nmax ? 0u : nout;
+		__syncthreads();
+		o_at = place(nout);
+		uint2 *o_rec = const_cast<uint2 *>(A.in) + o_at;
+		const uint32_t c0 = rp.cb + g.y0 * rp.gx;
+		for (uint32_t i = tid; i < take; i += WG) {
+			const uint32_t p = base + lo + i, c = cell[p] - c0;
+			const uint32_t r = c / rp.gx, x = c - r * rp.gx;
+			o_rec[i] = make_uint2(x | (r << 16),
+				(uint32_t)energy[p] | (type[p] ? V_WOLF : 0u));
+		}
+		tile_restamp<GT>(grass, c0, g.w * g.h, tick, P.R);
+	} else {
+		for (uint32_t r = tid; r < g.h; r += WG) {
+			const uint32_t c0 = rp.cb + (g.y0 + r) * rp.gx + g.x0;
+			const uint32_t lo = lower(c0);
+			s_lo[r] = lo;
+			s_n[r + 1] = lower(c0 + g.w) - lo;
+		}
+		__syncthreads();
+		if (tid == 0) {
+			s_n[0] = 0;
+			for (uint32_t r = 0; r < g.h; r++) s_n[r + 1] += s_n[r];
+		}
+		__syncthreads();
+		nout = s_n[g.h];
+		nf = s_n[1];
+		nl = nout - s_n[g.h - 1];
+		o_at = place(nout);
+		uint2 *o_rec = const_cast<uint2 *>(A.in) + o_at;
+		for (uint32_t r = tid; r <= g.h; r += WG)
+			const_cast<uint32_t *>(A.rin)[(size_t)tile * (A.rows + 1) + r] = s_n[r];
+		for (uint32_t r = 0; r < g.h; r++) {
+			const uint32_t c0 = rp.cb + (g.y0 + r) * rp.gx + g.x0;
+			for (uint32_t i = tid; i < s_n[r + 1] - s_n[r]; i += WG) {
+				const uint32_t o = s_n[r] + i;
+				if (nout > A.nmax) break;
+				const uint32_t p = base + s_lo[r] + i, x = cell[p] - c0;
+				const uint32_t y = (uint32_t)energy[p] | (type[p] ? V_WOLF : 0u);
+				o_rec[o] = make_uint2(x | (r << 16), y);
+				if (tr.nbx > 1) {
+					const uint2 er = make_uint2(o | (r << 16), y);
+					if (x == 0) {
+						const uint32_t q = atomicAdd(&s_edge[0], 1u);
+						if (q < TILE_ECAP) o_edge[q] = er;
+					}
+					if (x == g.w - 1) {
+						const uint32_t q = atomicAdd(&s_edge[1], 1u);
+						if (q < TILE_ECAP) o_edge[TILE_ECAP + q] = er;
+					}
+				}
+			}
+			tile_restamp<GT>(grass, c0, g.w, tick, P.R);
+		}
+		__syncthreads();
+		if (tid == 0)
+			atomicAdd(&A.bsum[tr.band0 + (tile - tr.tile0) / tr.nbx], nout);
+	}
+	if (tid == 0) {
+		const uint32_t el = D2 ? s_edge[0] : 0u, er = D2 ? s_edge[1] : 0u;
+		const_cast<uint4 *>(A.hin)[tile] = make_uint4(nout, nf | (nl << 16),
+			min(el, TILE_ECAP) | (min(er, TILE_ECAP) << 16), o_at);
+		if (nout > A.nmax || nf > A.hmax || nl > A.hmax || el > TILE_ECAP ||
+			er > TILE_ECAP)
+			ctl->stop = tick + 1;
+	}
+}
+
+/* The tiles' records (current parity) to the SoA state, at the replicas'
+ * batch positions (k_tile_base), and their grass re-stamped. A holds the
+ * buffers by parity, as for k_tile_end. */
+template <typename GT, bool D2>
+__global__ __launch_bounds__(WG) void k_tiles_out(TileArgs A, Ctl *ctl, Tables T,
+	Params P, uint32_t nrep, GT *grass, uint32_t *cell, int32_t *energy,
+	uint8_t *type) {
+	const bool SOLO = nrep == 1;
+	__shared__ uint32_t s_tmp[NWAVE];
+	const uint32_t tid = threadIdx.x, tile = blockIdx.x;
+	const uint32_t cur = tile_cur(ctl), tick = ctl->tt[cur];
+	const uint32_t k = nrep == 1 ? 0u : A.tk[tile];
+	const uint32_t slot = T.order[k];
+	const Rep &rp = T.rep[slot];
+	const RepCtl &rc = T.rctl[slot];
+	if (rc.status != RS_ACTIVE) return;
+	const TileRep tr = SOLO ? A.one : tile_rep(A.trep, k);
+	const uint32_t lt = tile - tr.tile0;
+	const TileGeo g = tile_geo<D2>(tr, lt, rp.gx, rp.gy);
+	const uint4 *hdr = cur ? A.hout : A.hin;
+	uint32_t idb = 0;
+	if (!D2) {
+		uint32_t sum = 0;
+		for (uint32_t i = tid; i < lt; i += WG) sum += hdr[tr.tile0 + i].x;
+		(void)wg_excl_scan<WG>(sum, s_tmp, idb);
+	}
+	const uint2 *recs = (cur ? A.out : A.in) + hdr[tile].w;
+	const uint32_t n = hdr[tile].x;
+	for (uint32_t i = tid; i < n; i += WG) {
+		const uint2 q = recs[i];
+		const uint32_t x = q.x & 0xFFFFu, r = q.x >> 16;
+		const uint32_t id = rc.base + i + (D2 ? A.idoff[tile * A.rows + r] : idb);
+		if (id >= P.cap) continue;
+		cell[id] = rp.cb + (g.y0 + r) * rp.gx + g.x0 + x;
+		energy[id] = (int32_t)(q.y & V_ENERGY);
+		type[id] = (q.y & V_WOLF) ? PP_WOLF : PP_SHEEP;
+	}
+	for (uint32_t r = 0; r < g.h; r++)
+		tile_restamp<GT>(grass, rp.cb + (g.y0 + r) * rp.gx + g.x0, g.w, tick, P.R);
+}

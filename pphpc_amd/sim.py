@@ -346,7 +346,8 @@ class Simulation:
 
     def set_sort(self, mode: int):
         """0: radix sort every iteration; 8..11: row buckets of 2**mode
-        cells; 1: automatic (the default). Results do not depend on it."""
+        cells; 1: automatic (the default: one kernel an iteration, tile by
+        tile). Results do not depend on it."""
         self._check(_lib().pp_sim_set_sort(self._h, mode), "set_sort")
 
     # -- profiling ---------------------------------------------------------
