@@ -197,7 +197,7 @@ struct RepCtl {
 	uint32_t err_step; /* iteration at which it failed */
 	uint32_t ovf;      /* tick + 1 in which an agent of a tile passed the
 	                    * energy limit (0: none) */
-	uint32_t pad;
+	uint32_t pub;      /* rows the host has (k_publish) */
 	unsigned long long dead_cells;  /* grass cells with countdown > 0 */
 	unsigned long long cd_sum;      /* sum of grass countdowns */
 	unsigned long long acc[NACC];   /* this iteration, AC_* */
@@ -732,15 +732,12 @@ __device__ __forceinline__ void wave_bucket_add(uint32_t *s_win,
 
 /* ------------------------------------------------------------------- init */
 
-/* Empties the batch: no agents, no replicas, tick 0, the pass-0 histograms
- * and the partial-sum slots zeroed. */
-__global__ __launch_bounds__(WG) void k_batch_reset(Ctl *ctl, uint32_t *hist,
-	uint32_t hist_words, unsigned long long *part) {
-	const uint32_t gtid = blockIdx.x * WG + threadIdx.x;
-	for (uint32_t i = gtid; i < hist_words; i += gridDim.x * WG) hist[i] = 0;
-	for (uint32_t i = gtid; i < PART_SLOTS * PART_STRIDE; i += gridDim.x * WG)
-		part[i] = 0;
-	if (gtid == 0) memset(ctl, 0, sizeof(Ctl));
+/* Empties the batch: no agents, no replicas, tick 0, the partial-sum slots
+ * zeroed. */
+__global__ __launch_bounds__(WG) void k_batch_reset(Ctl *ctl,
+	unsigned long long *part) {
+	for (uint32_t i = threadIdx.x; i < PART_SLOTS * PART_STRIDE; i += WG) part[i] = 0;
+	if (threadIdx.x == 0) memset(ctl, 0, sizeof(Ctl));
 }
 
 /* Marks the last of the next `ticks` ticks: its emit writes the SoA state
@@ -750,62 +747,87 @@ __global__ void k_state_tick(Ctl *ctl, uint32_t ticks) {
 		ctl->state_tick = ctl->tick + ticks;
 }
 
-/* Clears one replica slot's control words and grass ring. */
-__global__ __launch_bounds__(WG) void k_rep_reset(Tables T, uint32_t slot) {
+/* A replica admitted since the last run: its slot and the batch position of
+ * its first agent. The kernels that follow initialise all of them, a row of
+ * the grid each. */
+struct Admit {
+	uint32_t slot, pos;
+};
+
+/* Clears the replicas' control words and grass rings. */
+__global__ __launch_bounds__(WG) void k_rep_reset(Tables T, const Admit *list) {
+	const uint32_t slot = list[blockIdx.x].slot;
 	const Rep &rp = T.rep[slot];
 	for (uint32_t i = threadIdx.x; i <= rp.R; i += WG) rp.ring[i] = 0;
 	if (threadIdx.x == 0) memset(&T.rctl[slot], 0, sizeof(RepCtl));
 }
 
-/* Cells of one replica: grass alive with probability 1/2 (draw word 0), else
- * countdown 1 + U[0, R) (word 1), Philox counter (local cell, 0, INIT_CELL,
- * 0). Follows init_cell (pp_gpu.cl:368-398) and pphpc.nlogo:27-35. A cell with
- * countdown g at local iteration 0 is stored as regrow tick t0 + g; dead
- * cells are counted in ring slot (t0 + g) mod (R + 1). */
-template <typename GT>
-__global__ __launch_bounds__(WG) void k_init_cells(GT *grass_at, Tables T,
-	uint32_t slot) {
-	__shared__ uint32_t s_hist[4096];
-	__shared__ unsigned long long s_red[NWAVE][2];
-	const Rep rp = T.rep[slot];
-	const uint32_t M = rp.R + 1;
-	const bool lds_hist = M <= 4096;
-	if (lds_hist)
-		for (uint32_t i = threadIdx.x; i < M; i += WG) s_hist[i] = 0;
-	__syncthreads();
-	unsigned long long v[2] = {0, 0};
-	for (uint32_t c = blockIdx.x * WG + threadIdx.x; c < rp.C;
-		c += gridDim.x * WG) {
-		const uint4 r = pp_philox(c, 0, PP_STREAM_INIT_CELL, 0, rp.key0, rp.key1);
-		uint32_t g = 0;
-		if (pp_bounded(r.x, 2) != 1) g = 1 + pp_bounded(r.y, rp.R);
-		grass_at[rp.cb + c] = (GT)(rp.t0 + g);
-		if (g) {
-			v[0] += 1;
-			v[1] += g;
-			const uint32_t k = (rp.t0 + g) % M;
-			if (lds_hist) atomicAdd(&s_hist[k], 1u);
-			else atomicAdd(&rp.ring[k], 1ull);
-		}
-	}
-	wg_add<2>(v, s_red, &T.rctl[slot].dead_cells);
-	if (lds_hist)
-		for (uint32_t i = threadIdx.x; i < M; i += WG)
-			if (s_hist[i]) atomicAdd(&rp.ring[i], (unsigned long long)s_hist[i]);
+/* Cells and agents that one group initialises: at most INIT_GROUPS groups a
+ * replica and kind add to its counters (atomic adds to one address serialise
+ * at about 11 ns: 2048 groups for 2.56 M cells took 29 us, 313 take 9). */
+constexpr uint32_t INIT_CELLS = 8192, INIT_AGENTS = 2048, INIT_GROUPS = 2048;
+__host__ __device__ __forceinline__ uint32_t init_share(uint32_t n, uint32_t least) {
+	const uint32_t per = (n + INIT_GROUPS - 1) / INIT_GROUPS;
+	return per > least ? per : least;
+}
+__host__ __device__ __forceinline__ uint32_t init_groups(uint32_t n, uint32_t least) {
+	const uint32_t per = init_share(n, least);
+	return n ? (n - 1) / per + 1 : 0u;
 }
 
-/* Agents of one replica at batch positions [pos, pos + n0): local ids
- * 0..init_sheep-1 are sheep, the rest wolves; x = U[0,GX) (word 0),
- * y = U[0,GY) (word 1), energy 1 + U[0, 2*gain) (word 2), Philox counter
- * (local id, 0, INIT_AGENT, 0). Follows init_agent (pp_gpu.cl:406-439) and
- * pphpc.nlogo:38-53. */
-__global__ __launch_bounds__(WG) void k_init_agents(uint32_t *cell,
-	int32_t *energy, uint8_t *type, Tables T, uint32_t slot, uint32_t pos) {
+/* The initial state. Cells (the first groups of a replica's row): grass
+ * alive with probability 1/2 (draw word 0), else countdown 1 + U[0, R) (word
+ * 1), Philox counter (local cell, 0, INIT_CELL, 0). Follows init_cell
+ * (pp_gpu.cl:368-398) and pphpc.nlogo:27-35. A cell with countdown g at local
+ * iteration 0 is stored as regrow tick t0 + g; dead cells are counted in ring
+ * slot (t0 + g) mod (R + 1). Agents (the groups after them) at batch positions
+ * [pos, pos + n0): local ids 0..init_sheep-1 are sheep, the rest wolves; x =
+ * U[0,GX) (word 0), y = U[0,GY) (word 1), energy 1 + U[0, 2*gain) (word 2),
+ * Philox counter (local id, 0, INIT_AGENT, 0). Follows init_agent
+ * (pp_gpu.cl:406-439) and pphpc.nlogo:38-53. */
+template <typename GT>
+__global__ __launch_bounds__(WG) void k_init(GT *grass_at, uint32_t *cell,
+	int32_t *energy, uint8_t *type, Tables T, const Admit *list) {
+	__shared__ uint32_t s_hist[4096];
 	__shared__ unsigned long long s_red[NWAVE][4];
+	const uint32_t slot = list[blockIdx.y].slot, pos = list[blockIdx.y].pos;
 	const Rep rp = T.rep[slot];
+	const uint32_t gc = init_groups(rp.C, INIT_CELLS);
+	if (blockIdx.x < gc) {
+		const uint32_t M = rp.R + 1;
+		const bool lds_hist = M <= 4096;
+		if (lds_hist)
+			for (uint32_t i = threadIdx.x; i < M; i += WG) s_hist[i] = 0;
+		__syncthreads();
+		unsigned long long v[2] = {0, 0};
+		const uint32_t per = init_share(rp.C, INIT_CELLS);
+		const uint32_t c0 = blockIdx.x * per, c1 = min(rp.C, c0 + per);
+		for (uint32_t c = c0 + threadIdx.x; c < c1; c += WG) {
+			const uint4 r = pp_philox(c, 0, PP_STREAM_INIT_CELL, 0, rp.key0, rp.key1);
+			uint32_t g = 0;
+			if (pp_bounded(r.x, 2) != 1) g = 1 + pp_bounded(r.y, rp.R);
+			grass_at[(size_t)rp.cb + c] = (GT)(rp.t0 + g);
+			if (g) {
+				v[0] += 1;
+				v[1] += g;
+				const uint32_t k = (rp.t0 + g) % M;
+				if (lds_hist) atomicAdd(&s_hist[k], 1u);
+				else atomicAdd(&rp.ring[k], 1ull);
+			}
+		}
+		wg_add<2>(v, reinterpret_cast<unsigned long long (*)[2]>(s_red),
+			&T.rctl[slot].dead_cells);
+		if (lds_hist)
+			for (uint32_t i = threadIdx.x; i < M; i += WG)
+				if (s_hist[i]) atomicAdd(&rp.ring[i], (unsigned long long)s_hist[i]);
+		return;
+	}
+	const uint32_t per = init_share(rp.n0, INIT_AGENTS);
+	const uint64_t i0 = (uint64_t)(blockIdx.x - gc) * per;
+	if (i0 >= rp.n0) return;
+	const uint32_t i1 = (uint32_t)min((uint64_t)rp.n0, i0 + per);
 	unsigned long long v[4] = {0, 0, 0, 0};
-	for (uint32_t i = blockIdx.x * WG + threadIdx.x; i < rp.n0;
-		i += gridDim.x * WG) {
+	for (uint32_t i = (uint32_t)i0 + threadIdx.x; i < i1; i += WG) {
 		const uint4 r = pp_philox(i, 0, PP_STREAM_INIT_AGENT, 0, rp.key0, rp.key1);
 		const bool wolf = i >= rp.init_sheep;
 		const uint32_t gain = wolf ? rp.wolves_gain : rp.sheep_gain;
@@ -838,35 +860,38 @@ __device__ void write_row(const unsigned long long *acc, const RepCtl &rc,
 	write_row(acc, (unsigned long long)rp.C - rc.dead_cells, rc.cd_sum, row);
 }
 
-/* Row 0 of one replica placed at batch position pos = ctl->n; its agents join
- * the batch state. */
-__global__ void k_rep_init_done(Ctl *ctl, Tables T, uint32_t slot,
-	uint32_t pos) {
-	if (threadIdx.x != 0 || blockIdx.x != 0) return;
+/* Row 0 of the replicas; their agents, the last of which ends at position
+ * end, join the batch state. One thread a replica. */
+__global__ void k_rep_init_done(Ctl *ctl, Tables T, const Admit *list,
+	uint32_t end) {
+	if (threadIdx.x != 0) return;
+	if (blockIdx.x == 0) ctl->n = end;
+	const uint32_t slot = list[blockIdx.x].slot;
 	const Rep &rp = T.rep[slot];
 	RepCtl &rc = T.rctl[slot];
 	write_row(rc.acc, rc, rp, &rp.stats[0]);
 	for (int i = 0; i < NACC; i++) rc.acc[i] = 0;
 	rc.n = rp.iters ? rp.n0 : 0;
-	rc.base = pos;
+	rc.base = list[blockIdx.x].pos;
 	rc.step = 0;
 	rc.status = rp.iters ? RS_ACTIVE : RS_DONE;
-	ctl->n = pos + rp.n0;
 }
 
-/* Move for one replica's freshly initialised agents at batch positions
- * [pos, pos + n0) (SoA in local id order): their pairs and the live count of
- * this tick. They are appended after the agents of the batch, out of cell
- * order, so the next tick sorts with the general radix sort. */
+/* Move for the replicas' freshly initialised agents (SoA in local id order):
+ * their pairs and the survivors, whom the next tick's first kernel counts.
+ * They are appended after the agents of the batch, out of cell order, so that
+ * tick sorts with the general radix sort. */
 __global__ __launch_bounds__(WG) void k_move0(const uint32_t *__restrict__ cell,
 	const int32_t *__restrict__ energy, const uint8_t *__restrict__ type,
 	uint32_t *__restrict__ keys, uint32_t *__restrict__ vals, Ctl *ctl,
-	Tables T, uint32_t slot, uint32_t pos, Params P) {
-	__shared__ unsigned long long s_red[NWAVE];
+	Tables T, const Admit *list, Params P) {
 	if (ctl->error) return;
-	const uint32_t tick = ctl->tick;
+	const uint32_t slot = list[blockIdx.y].slot, pos = list[blockIdx.y].pos;
 	const Rep &rp = T.rep[slot];
-	const RepCtl &rc = T.rctl[slot];
+	const uint32_t per = init_share(rp.n0, INIT_AGENTS);
+	const uint64_t l0 = (uint64_t)blockIdx.x * per;
+	if (l0 >= rp.n0) return;
+	const uint32_t l1 = (uint32_t)min((uint64_t)rp.n0, l0 + per);
 	RM m;
 	m.cb = rp.cb;
 	m.C = rp.C;
@@ -876,15 +901,14 @@ __global__ __launch_bounds__(WG) void k_move0(const uint32_t *__restrict__ cell,
 	m.wolves_prob = rp.wolves_prob;
 	m.key0 = rp.key0;
 	m.key1 = rp.key1;
-	m.step = tick - rp.t0;
+	m.step = ctl->tick - rp.t0;
 	m.base = pos;
 	m.bbase = 0;
 	m.nb = row_blocks(rp.gx, P.bshift);
 	m.h = rows_per_bucket(rp.gx, P.bshift);
-	m.active = rc.status == RS_ACTIVE;
-	const uint32_t n = rp.n0;
+	m.active = rp.iters != 0;
 	unsigned long long live = 0;
-	for (uint32_t l = blockIdx.x * WG + threadIdx.x; l < n; l += gridDim.x * WG) {
+	for (uint32_t l = (uint32_t)l0 + threadIdx.x; l < l1; l += WG) {
 		const uint32_t g = pos + l;
 		uint32_t k = DEAD_KEY, v = 0, bkt;
 		if (m.active) {
@@ -896,15 +920,42 @@ __global__ __launch_bounds__(WG) void k_move0(const uint32_t *__restrict__ cell,
 		vals[g] = v;
 		live += k != DEAD_KEY;
 	}
-	const int tid = threadIdx.x, lane = tid & (WAVE - 1), w = tid / WAVE;
-	const unsigned long long tsum = wave_sum(live);
-	if (lane == 0) s_red[w] = tsum;
-	__syncthreads();
-	if (tid == 0) {
-		unsigned long long sum = 0;
-		for (int i = 0; i < NWAVE; i++) sum += s_red[i];
-		if (sum) atomicAdd(&ctl->live[tick & 1], (uint32_t)sum);
+	live = wave_sum(live);
+	if ((threadIdx.x & (WAVE - 1)) == 0 && live)
+		atomicAdd(&P.part[(blockIdx.x % PART_SLOTS) * PART_STRIDE + PART_LIVE], live);
+}
+
+/* Writes what the host reads after a run to its pinned memory: the control
+ * words, and each replica's and its statistics rows not yet written (at the
+ * ring index they have on the device). One kernel and one wait in place of
+ * copies of the control words, and then, once the host knows how many, of
+ * every replica's rows (one iteration of 100 x 100 with its row: 45 us with
+ * those). */
+__global__ __launch_bounds__(WG) void k_publish(const Ctl *ctl, RepCtl *rctl,
+	const pp_stats64_t *stats, uint32_t stats_rows, Ctl *h_ctl, RepCtl *h_rctl,
+	pp_stats64_t *h_stats) {
+	const uint32_t slot = blockIdx.x, tid = threadIdx.x;
+	static_assert(sizeof(Ctl) % 4 == 0 && sizeof(RepCtl) % 4 == 0, "copied as words");
+	static_assert(sizeof(pp_stats64_t) == 7 * 8, "a row is seven words");
+	if (slot == 0)
+		for (uint32_t i = tid; i < sizeof(Ctl) / 4; i += WG)
+			reinterpret_cast<uint32_t *>(h_ctl)[i] = reinterpret_cast<const uint32_t *>(ctl)[i];
+	RepCtl *rc = rctl + slot;
+	if (rc->status != RS_FREE) {
+		const uint32_t first = rc->pub, n = rc->step + 1 - first;
+		const size_t ring = (size_t)slot * stats_rows;
+		for (uint32_t i = tid; i < n * 7; i += WG) {
+			const uint32_t r = i / 7, q = i - r * 7;
+			const size_t at = (ring + (first + r) % stats_rows) * 7 + q;
+			reinterpret_cast<unsigned long long *>(h_stats)[at] =
+				reinterpret_cast<const unsigned long long *>(stats)[at];
+		}
+		__syncthreads();
+		if (tid == 0) rc->pub = first + n;
 	}
+	for (uint32_t i = tid; i < sizeof(RepCtl) / 4; i += WG)
+		reinterpret_cast<uint32_t *>(h_rctl + slot)[i] =
+			reinterpret_cast<const uint32_t *>(rc)[i];
 }
 
 /* Before k_move_soa: no pairs (positions of replicas that have ended stay
@@ -3195,6 +3246,7 @@ struct Replica {
 	uint32_t rows_have;    /* rows 0 .. rows_have - 1 collected */
 	uint32_t n;            /* agents of its current state */
 	uint64_t agent_steps;
+	int pending;           /* admitted since the last run: not on the device */
 	int keep;              /* keep every row on the host */
 	std::vector<pp_stats64_t> rows;
 	pp_stats64_t *sink;    /* else rows >= sink_from are written here */
@@ -3392,6 +3444,14 @@ struct pp_batch {
 	uint64_t reserved = 0;
 	std::map<uint32_t, Replica> reps;
 	uint32_t next_id = 0;
+	/* admissions that the next run takes to the device (flush_admitted) */
+	std::vector<Admit> admitted;
+	Admit *admit_dev = nullptr;
+	uint32_t next_pos = 0;        /* batch position after their agents */
+	int table_dirty = 0;          /* the device's replica table is not current */
+	/* host copies of the replica table, which asynchronous copies read */
+	std::vector<uint32_t> h_cbs, h_order, h_bbase, h_crep, h_brep;
+	uint32_t h_counts[2] = {0, 0};
 	uint64_t table_version = 0;   /* replica table uploads */
 	uint32_t table_nrep = 0;      /* replicas in the table */
 	std::vector<uint32_t> table_slots;
@@ -4147,10 +4207,9 @@ static int tile_settle(pp_batch_t *b, int *again) {
 }
 
 static int read_ctl(pp_batch_t *b) {
-	HIP_OK(hipMemcpyAsync(b->ctl_host, b->ctl, sizeof(Ctl),
-		hipMemcpyDeviceToHost, b->stream));
-	HIP_OK(hipMemcpyAsync(b->rctl_host, b->rctl_dev,
-		(size_t)b->max_rep * sizeof(RepCtl), hipMemcpyDeviceToHost, b->stream));
+	k_publish<<<b->max_rep, WG, 0, b->stream>>>(b->ctl, b->rctl_dev, b->stats_dev,
+		b->stats_rows, b->ctl_host, b->rctl_host, b->stats_host);
+	HIP_OK(hipGetLastError());
 	HIP_OK(hipStreamSynchronize(b->stream));
 	b->ctl_fresh = 1;
 	return prof_collect(b);
@@ -4159,42 +4218,50 @@ static int read_ctl(pp_batch_t *b) {
 /* Replica table: the slots in use sorted by first cell, and its length. The
  * stream must be idle. */
 static int upload_table(pp_batch_t *b) {
-	if (b->form == FORM_TILES) {
-		PP_TRY(to_soa(b));
-		HIP_OK(hipStreamSynchronize(b->stream));
-	}
+	PP_TRY(to_soa(b));
+	/* (the copies below read vectors that the last upload may still use) */
+	HIP_OK(hipStreamSynchronize(b->stream));
+	b->table_dirty = 0;
 	std::vector<std::pair<uint32_t, uint32_t>> t;
 	for (uint32_t s = 0; s < b->max_rep; s++)
 		if (b->slot_rid[s] >= 0) t.push_back({b->rep_host[s].cb, s});
 	std::sort(t.begin(), t.end());
-	std::vector<uint32_t> cbs(t.size()), order(t.size());
+	std::vector<uint32_t> &cbs = b->h_cbs, &order = b->h_order;
+	cbs.resize(t.size());
+	order.resize(t.size());
 	for (size_t i = 0; i < t.size(); i++) {
 		cbs[i] = t[i].first;
 		order[i] = t[i].second;
 	}
+	auto up = [&](void *dst, const void *src, size_t bytes) {
+		return bytes ? hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, b->stream)
+			: hipSuccess;
+	};
 	if (!t.empty()) {
-		HIP_OK(hipMemcpy(b->cbs_dev, cbs.data(), t.size() * 4,
-			hipMemcpyHostToDevice));
-		HIP_OK(hipMemcpy(b->order_dev, order.data(), t.size() * 4,
-			hipMemcpyHostToDevice));
+		const auto mm = std::minmax_element(order.begin(), order.end());
+		const uint32_t s0 = *mm.first, s1 = *mm.second + 1;
+		HIP_OK(up(b->rep_dev + s0, &b->rep_host[s0], (s1 - s0) * sizeof(Rep)));
+		HIP_OK(up(b->cbs_dev, cbs.data(), t.size() * 4));
+		HIP_OK(up(b->order_dev, order.data(), t.size() * 4));
 	}
 	const uint32_t nrep = (uint32_t)t.size();
 	/* the cell-chunk table of rep_index, for a table of several */
 	if (nrep > 1) {
-		std::vector<uint32_t> crep((size_t)(b->P.C >> CREP_SHIFT) + 1);
+		std::vector<uint32_t> &crep = b->h_crep;
+		crep.resize((size_t)(b->P.C >> CREP_SHIFT) + 1);
 		uint32_t k = 0;
 		for (size_t i = 0; i < crep.size(); i++) {
 			const uint64_t c0 = (uint64_t)i << CREP_SHIFT;
 			while (k + 1 < nrep && cbs[k + 1] <= c0) k++;
 			crep[i] = k;
 		}
-		HIP_OK(hipMemcpy(b->crep_dev, crep.data(), crep.size() * 4,
-			hipMemcpyHostToDevice));
+		HIP_OK(up(b->crep_dev, crep.data(), crep.size() * 4));
 	}
 	/* bucket layout: rows of blocks of 2^bshift cells, replicas in table
 	 * order */
 	const uint32_t shift = b->sort_mode >= 8 ? b->sort_mode : 11u;
-	std::vector<uint32_t> bbase(nrep + 1);
+	std::vector<uint32_t> &bbase = b->h_bbase;
+	bbase.resize(nrep + 1);
 	uint64_t nbk = 0;
 	for (uint32_t i = 0; i < nrep; i++) {
 		bbase[i] = (uint32_t)std::min<uint64_t>(nbk, 0xFFFFFFFFull);
@@ -4203,8 +4270,7 @@ static int upload_table(pp_batch_t *b) {
 		nbk += (uint64_t)((rp.gy + h - 1) / h) * row_blocks(rp.gx, shift);
 	}
 	bbase[nrep] = (uint32_t)std::min<uint64_t>(nbk, 0xFFFFFFFFull);
-	HIP_OK(hipMemcpy(b->bbase_dev, bbase.data(), (nrep + 1) * 4,
-		hipMemcpyHostToDevice));
+	HIP_OK(up(b->bbase_dev, bbase.data(), (nrep + 1) * 4));
 	/* Row buckets when chosen, or automatically: always for one replica,
 	 * for several while the buckets are few or dense enough that their
 	 * per-bucket latency stays below the radix sort's passes. The density
@@ -4221,10 +4287,11 @@ static int upload_table(pp_batch_t *b) {
 	while (top + 1 < (uint32_t)CNT_LEVELS && (nbk >> (6 * (top + 1))) > 0) top++;
 	/* the replica of each bucket, for the bucket sort of several */
 	if (on && nrep > 1) {
-		std::vector<uint32_t> brep(nbk);
+		std::vector<uint32_t> &brep = b->h_brep;
+		brep.resize(nbk);
 		for (uint32_t i = 0; i < nrep; i++)
 			std::fill(brep.begin() + bbase[i], brep.begin() + bbase[i + 1], i);
-		HIP_OK(hipMemcpy(b->brep_dev, brep.data(), nbk * 4, hipMemcpyHostToDevice));
+		HIP_OK(up(b->brep_dev, brep.data(), nbk * 4));
 	}
 	const uint32_t one = nrep == 1 ? order[0] : 0u;
 	const uint32_t solo = nrep == 1 ? 1u : 0u;
@@ -4260,8 +4327,10 @@ static int upload_table(pp_batch_t *b) {
 		drop_graph(b);     /* Params are launch arguments of the graphs */
 	}
 	const uint32_t nb32 = on ? (uint32_t)nbk : 0u;
-	HIP_OK(hipMemcpy(&b->ctl->nrep, &nrep, 4, hipMemcpyHostToDevice));
-	HIP_OK(hipMemcpy(&b->ctl->nbuckets, &nb32, 4, hipMemcpyHostToDevice));
+	static_assert(offsetof(Ctl, nbuckets) == offsetof(Ctl, nrep) + 4, "copied as one");
+	b->h_counts[0] = nrep;
+	b->h_counts[1] = nb32;
+	HIP_OK(up(&b->ctl->nrep, b->h_counts, 8));
 	b->ctl_host->nrep = nrep;
 	b->ctl_host->nbuckets = nb32;
 	b->need_radix = 1;
@@ -4270,6 +4339,68 @@ static int upload_table(pp_batch_t *b) {
 	b->table_slots = order;
 	b->tile_dense = 0;
 	table_plan(b);
+	return PP_SUCCESS;
+}
+
+template <typename GT>
+static void launch_init(pp_batch_t *b, const Admit *list, uint32_t n,
+	uint32_t groups) {
+	k_init<GT><<<dim3(groups, n), WG, 0, b->stream>>>((GT *)b->grass_at, b->cell,
+		b->energy, b->type, b->tables(), list);
+}
+
+/* The initial state of the n replicas listed in admit_dev (cells, agents,
+ * row 0) and the first move of their agents, who end at position `end`;
+ * gc and ga: the most groups for a replica's cells and agents. */
+static int enqueue_init(pp_batch_t *b, uint32_t n, uint32_t end, uint32_t gc,
+	uint32_t ga) {
+	constexpr uint32_t MOST = 32768;   /* rows of a grid */
+	for (uint32_t i = 0; i < n; i += MOST) {
+		const uint32_t m = min_u32(n - i, MOST);
+		const Admit *list = b->admit_dev + i;
+		PendingEvent pe;
+		prof_begin(b, KI_INIT_RESET, pe);
+		k_rep_reset<<<m, WG, 0, b->stream>>>(b->tables(), list);
+		prof_end(b, pe);
+		prof_begin(b, KI_INIT_CELLS, pe);
+		if (b->grass_bytes == 1) launch_init<uint8_t>(b, list, m, gc + ga);
+		else if (b->grass_bytes == 2) launch_init<uint16_t>(b, list, m, gc + ga);
+		else launch_init<uint32_t>(b, list, m, gc + ga);
+		prof_end(b, pe);
+		prof_begin(b, KI_INIT_DONE, pe);
+		k_rep_init_done<<<m, WAVE, 0, b->stream>>>(b->ctl, b->tables(), list, end);
+		prof_end(b, pe);
+		prof_begin(b, KI_MOVE0, pe);
+		k_move0<<<dim3(std::max(ga, 1u), m), WG, 0, b->stream>>>(b->cell, b->energy,
+			b->type, b->keys[0], b->vals[0], b->ctl, b->tables(), list, b->P);
+		prof_end(b, pe);
+	}
+	HIP_OK(hipGetLastError());
+	return PP_SUCCESS;
+}
+
+/* Brings the device up to date before a run or a look at the state: the
+ * replica table, and the replicas admitted since, all with the same few
+ * launches (one admission at a time took 250 us each, mostly copies and
+ * waits: 30 replicas of 1600 x 1600 for 60 iterations, 28 ms in all, 13 of
+ * them for that). */
+static int flush_admitted(pp_batch_t *b) {
+	if (b->table_dirty) PP_TRY(upload_table(b));
+	if (b->admitted.empty()) return PP_SUCCESS;
+	uint32_t gc = 0, ga = 0;
+	for (const Admit &a : b->admitted) {
+		gc = std::max(gc, init_groups(b->rep_host[a.slot].C, INIT_CELLS));
+		ga = std::max(ga, init_groups(b->rep_host[a.slot].n0, INIT_AGENTS));
+	}
+	const uint32_t n = (uint32_t)b->admitted.size();
+	HIP_OK(hipMemcpyAsync(b->admit_dev, b->admitted.data(), n * sizeof(Admit),
+		hipMemcpyHostToDevice, b->stream));
+	PP_TRY(enqueue_init(b, n, b->next_pos, gc, ga));
+	HIP_OK(hipStreamSynchronize(b->stream));   /* (the list has been read) */
+	for (auto &kv : b->reps) kv.second.pending = 0;
+	b->admitted.clear();
+	b->ctl_fresh = 0;
+	b->soa_fresh = 0;    /* the new agents are in no cell order */
 	return PP_SUCCESS;
 }
 
@@ -4317,33 +4448,10 @@ static int collect(pp_batch_t *b) {
 	if (b->ctl_host->error && getenv("PPHPC_DEBUG"))
 		fprintf(stderr, "pphpc: batch error %d at tick %u (detail %d)\n",
 			b->ctl_host->error, b->ctl_host->err_step, b->ctl_host->err_rep);
-	std::vector<Replica *> got;
-	for (auto &kv : b->reps) {
-		Replica &r = kv.second;
-		if (r.slot < 0) continue;
-		const RepCtl &rc = b->rctl_host[r.slot];
-		if (rc.status == RS_FREE) continue;
-		const uint32_t last = rc.step;  /* rows 0..last exist */
-		if (last + 1 > r.rows_have) {
-			const uint32_t first = r.rows_have, nrows = last + 1 - first;
-			const uint32_t R = b->stats_rows;
-			pp_stats64_t *dev = b->stats_dev + (size_t)r.slot * R;
-			pp_stats64_t *host = b->stats_host + (size_t)r.slot * R;
-			const uint32_t a = first % R;
-			const uint32_t n1 = min_u32(nrows, R - a);
-			HIP_OK(hipMemcpyAsync(host + a, dev + a, (size_t)n1 * sizeof(pp_stats64_t),
-				hipMemcpyDeviceToHost, b->stream));
-			if (nrows > n1)
-				HIP_OK(hipMemcpyAsync(host, dev, (size_t)(nrows - n1) *
-					sizeof(pp_stats64_t), hipMemcpyDeviceToHost, b->stream));
-			got.push_back(&r);
-		}
-	}
-	if (!got.empty()) HIP_OK(hipStreamSynchronize(b->stream));
 	int dirty = 0;
 	for (auto &kv : b->reps) {
 		Replica &r = kv.second;
-		if (r.slot < 0) continue;
+		if (r.slot < 0 || r.pending) continue;
 		const RepCtl &rc = b->rctl_host[r.slot];
 		if (rc.status == RS_FREE) continue;
 		const uint32_t R = b->stats_rows;
@@ -4372,7 +4480,7 @@ static int collect(pp_batch_t *b) {
 	}
 	int again = 0;
 	PP_TRY(tile_settle(b, &again));
-	if (dirty) PP_TRY(upload_table(b));
+	if (dirty) b->table_dirty = 1;
 	else if (again) table_plan(b);
 	return PP_SUCCESS;
 }
@@ -4390,6 +4498,7 @@ static int run_ticks(pp_batch_t *b, uint32_t ticks) {
 	const uint32_t target = b->ctl_host->tick + ticks;
 	while (b->ctl_host->tick != target) {
 		const uint32_t t0 = b->ctl_host->tick;
+		PP_TRY(flush_admitted(b));
 		const uint32_t dense0 = b->tile_dense;
 		PP_TRY(enqueue_ticks(b, target - t0));
 		PP_TRY(collect(b));
@@ -4450,6 +4559,7 @@ static void batch_free(pp_batch_t *b) {
 	(void)hipFree(b->cbs_dev);
 	(void)hipFree(b->crep_dev);
 	(void)hipFree(b->order_dev);
+	(void)hipFree(b->admit_dev);
 	(void)hipFree(b->stats_dev);
 	if (b->stats_host) (void)hipHostFree(b->stats_host);
 	if (b->ctl_host) (void)hipHostFree(b->ctl_host);
@@ -4484,7 +4594,7 @@ static uint64_t batch_bytes(uint64_t A, uint64_t C, uint32_t max_rep,
 		const uint64_t tiles = (uint64_t)ceil_div(A, A_TILE) + 1;
 		t += (tiles + (tiles + 63) / 64 + 1) * 4 + tiles * 4;
 	}
-	t += sizeof(Ctl) + PART_SLOTS * PART_STRIDE * 8 + (uint64_t)max_rep * (sizeof(Rep) + sizeof(RepCtl) + 8);
+	t += sizeof(Ctl) + PART_SLOTS * PART_STRIDE * 8 + (uint64_t)max_rep * (sizeof(Rep) + sizeof(RepCtl) + 8 + sizeof(Admit));
 	t += (uint64_t)max_rep * stats_rows * sizeof(pp_stats64_t);
 	return t;
 }
@@ -4544,6 +4654,7 @@ static int batch_buffers(pp_batch_t *b, Take &&take) {
 	HIP_OK(take((void **)&b->cbs_dev, (size_t)b->max_rep * 4));
 	HIP_OK(take((void **)&b->crep_dev, ((size_t)(C >> CREP_SHIFT) + 1) * 4));
 	HIP_OK(take((void **)&b->order_dev, (size_t)b->max_rep * 4));
+	HIP_OK(take((void **)&b->admit_dev, (size_t)b->max_rep * sizeof(Admit)));
 	const size_t srows = (size_t)b->max_rep * b->stats_rows;
 	HIP_OK(take((void **)&b->stats_dev, srows * sizeof(pp_stats64_t)));
 	return PP_SUCCESS;
@@ -4641,16 +4752,12 @@ static int batch_create(uint64_t agents, uint64_t cells, uint32_t max_rep,
 /* Empties the batch (tick 0, no replicas). */
 static int batch_reset(pp_batch_t *b) {
 	HIP_OK(hipSetDevice(b->device));
-	HIP_OK(hipStreamSynchronize(b->stream));
+	HIP_OK(hipStreamSynchronize(b->stream));   /* (the host's copies are free) */
 	PendingEvent pe;
 	prof_begin(b, KI_INIT_RESET, pe);
-	k_batch_reset<<<min_u32(ceil_div(b->hist_alloc_words, WG), 2048), WG, 0,
-		b->stream>>>(b->ctl, b->hist, (uint32_t)b->hist_alloc_words, b->P.part);
+	k_batch_reset<<<1, WG, 0, b->stream>>>(b->ctl, b->P.part);
 	prof_end(b, pe);
 	HIP_OK(hipGetLastError());
-	HIP_OK(hipMemsetAsync(b->rctl_dev, 0, (size_t)b->max_rep * sizeof(RepCtl),
-		b->stream));
-	HIP_OK(hipStreamSynchronize(b->stream));
 	memset(b->ctl_host, 0, sizeof(Ctl));
 	memset(b->rctl_host, 0, (size_t)b->max_rep * sizeof(RepCtl));
 	b->ctl_fresh = 1;
@@ -4662,6 +4769,8 @@ static int batch_reset(pp_batch_t *b) {
 	b->need_radix = 1;
 	b->form = FORM_PAIRS;
 	b->soa_fresh = 0;
+	b->admitted.clear();
+	b->table_dirty = 1;
 	return PP_SUCCESS;
 }
 
@@ -4679,8 +4788,8 @@ static int check_params(const pp_params_t *p) {
 	return PP_SUCCESS;
 }
 
-/* Admits one replica: its slot, cells and agent reservation, its initial
- * state appended to the batch state and moved for its first iteration. */
+/* Admits one replica: its slot, cells and agent reservation. The next run
+ * (flush_admitted) appends its initial state to the batch state. */
 static int admit(pp_batch_t *b, const pp_params_t *p, uint64_t seed,
 	uint64_t reserve, uint32_t iters, int keep, uint32_t *id_out) {
 	PP_TRY(check_params(p));
@@ -4690,10 +4799,14 @@ static int admit(pp_batch_t *b, const pp_params_t *p, uint64_t seed,
 	if (p->grass_restart > b->P.R || C > b->P.C) return PP_INVALID_ARGS;
 	if (reserve == 0) reserve = std::max<uint64_t>(4ull * n0, 1);
 	if (reserve < n0 || reserve > b->P.cap) return PP_INVALID_ARGS;
-	PP_TRY(to_pairs(b));
-	if (!b->ctl_fresh) PP_TRY(read_ctl(b));
+	if (b->admitted.empty()) {
+		/* its agents will be appended to the batch's pairs */
+		PP_TRY(to_pairs(b));
+		if (!b->ctl_fresh) PP_TRY(read_ctl(b));
+		b->next_pos = b->ctl_host->n;
+	}
 	if (b->ctl_host->error) return b->ctl_host->error;
-	const uint32_t tick = b->ctl_host->tick, pos = b->ctl_host->n;
+	const uint32_t tick = b->ctl_host->tick, pos = b->next_pos;
 	/* (a plain simulation runs without a limit; pp_sim_run checks its runs) */
 	if (iters != ITERS_UNLIMITED &&
 		(uint64_t)tick + iters + b->P.R + 1 >= 0xFFFFFFFFull)
@@ -4733,14 +4846,6 @@ static int admit(pp_batch_t *b, const pp_params_t *p, uint64_t seed,
 	rp.stats_rows = b->stats_rows;
 	rp.ring = b->ring + (size_t)slot * b->ring_stride;
 	rp.stats = b->stats_dev + (size_t)slot * b->stats_rows;
-	int rc = PP_SUCCESS;
-	if (hipMemcpy(&b->rep_dev[slot], &rp, sizeof(Rep), hipMemcpyHostToDevice)
-			!= hipSuccess)
-		rc = PP_LIBRARY_ERROR;
-	if (rc) {
-		release_cells(b, (uint32_t)cb, C);
-		return rc;
-	}
 	b->rep_host[slot] = rp;
 	const uint32_t id = b->next_id++;
 	b->slot_rid[slot] = id;
@@ -4765,41 +4870,10 @@ static int admit(pp_batch_t *b, const pp_params_t *p, uint64_t seed,
 	r.keep = keep;
 	r.sink = nullptr;
 	r.sink_from = 0;
-	PP_TRY(upload_table(b));
-
-	const Tables T = b->tables();
-	const uint32_t cu = (uint32_t)b->num_cu;
-	PendingEvent pe;
-	prof_begin(b, KI_INIT_RESET, pe);
-	k_rep_reset<<<1, WG, 0, b->stream>>>(T, (uint32_t)slot);
-	prof_end(b, pe);
-	prof_begin(b, KI_INIT_CELLS, pe);
-	const uint32_t gc = min_u32(ceil_div(C, WG), 8 * cu);
-	if (b->grass_bytes == 1)
-		k_init_cells<uint8_t><<<gc, WG, 0, b->stream>>>((uint8_t *)b->grass_at, T,
-			(uint32_t)slot);
-	else if (b->grass_bytes == 2)
-		k_init_cells<uint16_t><<<gc, WG, 0, b->stream>>>((uint16_t *)b->grass_at,
-			T, (uint32_t)slot);
-	else
-		k_init_cells<uint32_t><<<gc, WG, 0, b->stream>>>((uint32_t *)b->grass_at,
-			T, (uint32_t)slot);
-	prof_end(b, pe);
-	prof_begin(b, KI_INIT_AGENTS, pe);
-	k_init_agents<<<min_u32(ceil_div(n0 ? n0 : 1, WG), 8 * cu), WG, 0,
-		b->stream>>>(b->cell, b->energy, b->type, T, (uint32_t)slot, pos);
-	prof_end(b, pe);
-	prof_begin(b, KI_INIT_DONE, pe);
-	k_rep_init_done<<<1, 64, 0, b->stream>>>(b->ctl, T, (uint32_t)slot, pos);
-	prof_end(b, pe);
-	prof_begin(b, KI_MOVE0, pe);
-	k_move0<<<min_u32(ceil_div(n0 ? n0 : 1, WG), 8 * cu), WG, 0,
-		b->stream>>>(b->cell, b->energy, b->type, b->keys[0], b->vals[0],
-		b->ctl, T, (uint32_t)slot, pos, b->P);
-	prof_end(b, pe);
-	HIP_OK(hipGetLastError());
-	b->ctl_fresh = 0;
-	b->soa_fresh = 0;    /* the new agents are in no cell order */
+	r.pending = 1;
+	b->admitted.push_back(Admit{(uint32_t)slot, pos});
+	b->next_pos = pos + n0;
+	b->table_dirty = 1;
 	if (id_out) *id_out = id;
 	return PP_SUCCESS;
 }
@@ -4993,10 +5067,8 @@ static int simulate_noalloc(const pp_params_t *p, uint64_t seed,
 	 * zero (control block, partial sums, histograms, the replica's control
 	 * words, the bucket counts). */
 	const hipStream_t st = b->stream;
-	k_batch_reset<<<min_u32(ceil_div(b->hist_alloc_words, WG), 2048), WG, 0,
-		st>>>(b->ctl, b->hist, (uint32_t)b->hist_alloc_words, b->P.part);
+	k_batch_reset<<<1, WG, 0, st>>>(b->ctl, b->P.part);
 	HIP_OK(hipGetLastError());
-	HIP_OK(hipMemsetAsync(b->rctl_dev, 0, sizeof(RepCtl), st));
 	const size_t nbw = cnt_words(b->P.nb_cap);
 	HIP_OK(hipMemsetAsync(b->ocnt, 0, nbw * 4, st));
 	HIP_OK(hipMemsetAsync(b->ncnt, 0, nbw * 4, st));
@@ -5050,22 +5122,10 @@ static int simulate_noalloc(const pp_params_t *p, uint64_t seed,
 	const TileGrid tg{&rp, 0, n0};
 	tile_plan(b, &tg, 1);
 
-	const Tables T = b->tables();
-	const uint32_t cu = (uint32_t)b->num_cu;
-	k_rep_reset<<<1, WG, 0, st>>>(T, 0);
-	const uint32_t gc = min_u32(ceil_div(C, WG), 8 * cu);
-	if (b->grass_bytes == 1)
-		k_init_cells<uint8_t><<<gc, WG, 0, st>>>((uint8_t *)b->grass_at, T, 0);
-	else if (b->grass_bytes == 2)
-		k_init_cells<uint16_t><<<gc, WG, 0, st>>>((uint16_t *)b->grass_at, T, 0);
-	else
-		k_init_cells<uint32_t><<<gc, WG, 0, st>>>((uint32_t *)b->grass_at, T, 0);
-	const uint32_t ga = min_u32(ceil_div(n0 ? n0 : 1, WG), 8 * cu);
-	k_init_agents<<<ga, WG, 0, st>>>(b->cell, b->energy, b->type, T, 0, 0);
-	k_rep_init_done<<<1, 64, 0, st>>>(b->ctl, T, 0, 0);
-	k_move0<<<ga, WG, 0, st>>>(b->cell, b->energy, b->type, b->keys[0],
-		b->vals[0], b->ctl, T, 0, 0, b->P);
-	HIP_OK(hipGetLastError());
+	const Admit ad{0, 0};
+	HIP_OK(hipMemcpy(b->admit_dev, &ad, sizeof(Admit), hipMemcpyHostToDevice));
+	PP_TRY(enqueue_init(b, 1, rp.n0, init_groups(rp.C, INIT_CELLS),
+		init_groups(rp.n0, INIT_AGENTS)));
 	HIP_OK(hipMemcpy(&rows[0], b->stats_dev, sizeof(pp_stats64_t),
 		hipMemcpyDeviceToHost));
 
@@ -5081,9 +5141,14 @@ static int simulate_noalloc(const pp_params_t *p, uint64_t seed,
 		if (b->ctl_host->error) return b->ctl_host->error;
 		const RepCtl &rc = *b->rctl_host;
 		const uint32_t last = rc.step;   /* rows 0..last exist */
-		for (uint32_t i = done + 1; i <= last; i++)
-			HIP_OK(hipMemcpy(&rows[i], b->stats_dev + i % b->stats_rows,
-				sizeof(pp_stats64_t), hipMemcpyDeviceToHost));
+		/* (the ring holds them in one or two pieces) */
+		for (uint32_t i = done + 1; i <= last;) {
+			const uint32_t at = i % b->stats_rows;
+			const uint32_t n = min_u32(last + 1 - i, b->stats_rows - at);
+			HIP_OK(hipMemcpy(&rows[i], b->stats_dev + at, n * sizeof(pp_stats64_t),
+				hipMemcpyDeviceToHost));
+			i += n;
+		}
 		if (rc.status == RS_FAILED) return rc.error;
 		int again = 0;
 		PP_TRY(tile_settle(b, &again));
@@ -5164,7 +5229,8 @@ int pp_sim_init(pp_sim_t *s, pp_stats64_t *stats0) {
 		Replica *r = sim_rep(s);
 		r->sink = stats0;
 		r->sink_from = 0;
-		const int rc = collect(s->b);
+		int rc = flush_admitted(s->b);
+		if (!rc) rc = collect(s->b);
 		r->sink = nullptr;
 		if (rc) return rc;
 		if (s->b->ctl_host->error) return s->b->ctl_host->error;
@@ -5415,6 +5481,7 @@ int pp_batch_get_state(pp_batch_t *b, uint32_t id, uint32_t *n_agents,
 		auto it = b->reps.find(id);
 		if (it == b->reps.end()) return PP_INVALID_ARGS;
 		HIP_OK(hipSetDevice(b->device));
+		PP_TRY(flush_admitted(b));
 		PP_TRY(tiles_out(b));
 		PP_TRY(read_ctl(b));
 		const Replica &r = it->second;
@@ -5523,6 +5590,7 @@ int pp_batch_set_sort(pp_batch_t *b, uint32_t mode) {
 		HIP_OK(hipSetDevice(b->device));
 		if (mode == b->sort_mode) return PP_SUCCESS;
 		if (!b->ctl_fresh) PP_TRY(read_ctl(b));
+		PP_TRY(flush_admitted(b));
 		b->sort_mode = mode;
 		return upload_table(b);    /* new layout; the next tick re-sorts */
 	});
@@ -5534,6 +5602,7 @@ int pp_batch_tune(pp_batch_t *b, uint32_t trial_ticks, uint32_t *bucket_shift,
 		if (!b || trial_ticks == 0 || trial_ticks + 8 > b->stats_rows / 2)
 			return PP_INVALID_ARGS;
 		HIP_OK(hipSetDevice(b->device));
+		PP_TRY(flush_admitted(b));
 		/* candidates: the automatic mode's tile step, the bucket sort at each
 		 * block width, then the radix sort at each shape */
 		struct Cand { uint32_t shift; SortShape sh; };
@@ -5552,10 +5621,13 @@ int pp_batch_tune(pp_batch_t *b, uint32_t trial_ticks, uint32_t *bucket_shift,
 		 * more. */
 		auto trial = [&](double &t) -> int {
 			for (int attempt = 0; attempt < 2; attempt++) {
+				PP_TRY(flush_admitted(b));
 				PP_TRY(enqueue_ticks(b, 8));
 				PP_TRY(collect(b));
+				PP_TRY(flush_admitted(b));
 				const uint64_t v0 = b->table_version;
 				PP_TRY(time_ticks(b, trial_ticks, &t));
+				PP_TRY(flush_admitted(b));
 				if (b->table_version == v0 || active_count(b) == 0) break;
 			}
 			return PP_SUCCESS;

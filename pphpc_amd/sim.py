@@ -206,12 +206,21 @@ def simulate_noalloc(params: Params, seed: int = 0, capacity: int = 0,
     """pp_sim_simulate_noalloc: rows 0..iters of one simulation run in the
     library's fixed device scratch (no device allocation), as an (iters+1, 7)
     uint64 array."""
-    out = (Stats * (params.iters + 1))()
+    out = _row_array(params.iters + 1)
     rc = _lib().pp_sim_simulate_noalloc(ctypes.byref(params), seed, capacity,
-                                        device, out)
+                                        device, _row_ptr(out))
     if rc:
         raise PPError(rc, "simulate_noalloc")
-    return stats_rows_to_array(out)
+    return out
+
+
+def _row_array(n: int) -> np.ndarray:
+    """n statistics rows for the library to fill, as (n, 7) uint64."""
+    return np.empty((n, len(STAT_FIELDS)), np.uint64)
+
+
+def _row_ptr(rows: np.ndarray):
+    return rows.ctypes.data_as(ctypes.POINTER(Stats))
 
 
 def stats_rows_to_array(rows) -> np.ndarray:
@@ -277,7 +286,12 @@ class Simulation:
         return list(rows) if rows is not None else []
 
     def run_array(self, iters: int) -> np.ndarray:
-        return stats_rows_to_array(self.run(iters))
+        out = _row_array(iters)
+        rc = _lib().pp_sim_run(self._h, iters, _row_ptr(out) if iters else None)
+        if rc:
+            raise PPError(rc, f"run({iters}) stopped at iteration "
+                              f"{self.error_step}")
+        return out
 
     def simulate(self):
         """init + ITERS iterations: rows 0..ITERS (pp_gpu.c:1857-1866)."""
@@ -464,7 +478,11 @@ class Batch:
         return list(out)
 
     def rows_array(self, rid: int) -> np.ndarray:
-        return stats_rows_to_array(self.rows(rid))
+        n = self.replica(rid)["steps"] + 1
+        out = _row_array(n)
+        self._check(_lib().pp_batch_rows(self._h, rid, 0, n, _row_ptr(out)),
+                    "rows")
+        return out
 
     def state(self, rid: int):
         """(cell, energy, type, grass) of a running replica, cells local to
