@@ -3351,7 +3351,7 @@ constexpr uint32_t TILE_WIDE = 2048, TILE_MIN = 400;
 struct TileShape {
 	uint32_t nt, ipt, cells;
 };
-const TileShape tile_shapes[] = {{256, 8, 4096}, {512, 8, 8192}};
+const TileShape tile_shapes[] = {{256, 7, 4096}, {512, 8, 8192}};
 
 } /* namespace */
 
@@ -3802,7 +3802,7 @@ static void launch_tile(pp_batch_t *b) {
 	const uint32_t grid = a.nfin + ceil_div(a.ntiles, NXCD) * NXCD;
 	GT *g = (GT *)b->grass_at;
 	if (b->plan.cfg == 0)
-		k_tile<GT, 256, 8, 4096, D2, SOLO><<<grid, 256, 0, b->stream>>>(a, b->ctl,
+		k_tile<GT, 256, 7, 4096, D2, SOLO><<<grid, 256, 0, b->stream>>>(a, b->ctl,
 			b->tables(), b->P, b->table_nrep, g);
 	else
 		k_tile<GT, 512, 8, 8192, D2, SOLO><<<grid, 512, 0, b->stream>>>(a, b->ctl,
@@ -3992,7 +3992,8 @@ struct TileGrid {
  * rows' counts after each iteration); wider grids are cut into 256 columns.
  * One replica takes about as many tiles as run at once: four groups of 256
  * threads a CU hold up to 1024, of which 256 are taken (400 x 400: 10.3 us
- * with tiles of 2 or 4 rows, 11.2 of 8), else two groups of 512 (1600 x 1600:
+ * with tiles of 2 or 4 rows, 11.2 of 8; 7 slots a thread, which 32 KB of LDS
+ * hold with four groups, 1013 x 487 10.8 us, 11.4 with 8), else two groups of 512 (1600 x 1600:
  * 18.6 us with 400 tiles of 4 rows, 20.4 with 320 of 5, 23.7 with 534 of 3, a
  * second round). Several replicas fill the GPU with tiles as large as fit,
  * which move fewer neighbours' agents twice (30 x 1600 x 1600: 248 us with 5
@@ -4021,13 +4022,16 @@ static void tile_layout(const pp_batch_t *b, const TileGrid *grid, uint32_t n,
 	if (ecfg == -1) return;
 	if (ebx) p.d2 = true;
 	/* rows of a tile (at most) in shape c: its cells, and most of the agents
-	 * it may hold */
-	const double fill = n > 1 ? 0.85 : 0.75;
+	 * it may hold (with rows filled further than 0.87, or border rows of less
+	 * than 1.25 times the mean and 64, tiles would outgrow their limits by
+	 * chance and stop the run; 0.75 for one replica's few tiles, whose largest
+	 * ends each iteration) */
+	const double fill = n > 1 || p.d2 ? 0.87 : 0.75;
 	auto limits = [&](int c) {
 		const uint32_t ag = tile_shapes[c].nt * tile_shapes[c].ipt;
 		const uint32_t wide = p.d2 ? std::min<uint32_t>(ebx ? ebx : 256, width) : width;
 		p.cfg = c;
-		p.hmax = std::min<uint32_t>(ag / 3, (uint32_t)(1.4 * dens * wide) + 64);
+		p.hmax = std::min<uint32_t>(ag / 3, (uint32_t)(1.25 * dens * wide) + 64);
 		p.nmax = ag - 2 * p.hmax - (p.d2 ? 2 * TILE_ECAP : 0);
 	};
 	auto rows_max = [&](uint32_t w) {
@@ -4072,7 +4076,6 @@ static void tile_layout(const pp_batch_t *b, const TileGrid *grid, uint32_t n,
 		t.wolves_prob = rp.wolves_prob;
 		t.gxm = rp.gx_magic;
 		t.gxs = rp.gx_shift;
-		const uint64_t gb = b->grass_bytes;
 		if (!p.d2) {
 			t.bx = gx;
 			const double most = rows_max(gx);
@@ -4084,12 +4087,6 @@ static void tile_layout(const pp_batch_t *b, const TileGrid *grid, uint32_t n,
 				const uint32_t round = p.cfg == 0 ? 256 : 512;
 				by = min_u32(by, std::max(ceil_div(gy, round), ceil_div(TILE_MIN, gx)));
 			}
-			/* whole 16-byte chunks of grass where a few rows more give them */
-			uint32_t m = 1;
-			while (m < 16 && (uint64_t)m * gx * gb % 16) m *= 2;
-			const uint32_t up = ceil_div(by, m) * m;
-			if (up <= most) by = up;
-			else if (by >= m) by -= by % m;
 			t.by = by;
 		} else {
 			t.bx = min_u32(ebx ? ebx : 256, gx);
@@ -4103,10 +4100,6 @@ static void tile_layout(const pp_batch_t *b, const TileGrid *grid, uint32_t n,
 		t.by = min_u32(t.by, gy);
 		t.nbx = ceil_div(gx, t.bx);
 		t.nby = ceil_div(gy, t.by);
-		/* rows (or, in one piece, tiles) of whole 16-byte chunks of grass */
-		t.vec = rp.cb * gb % 16 == 0 && (p.d2
-			? gx * gb % 16 == 0 && t.bx * gb % 16 == 0
-			: t.by * (uint64_t)gx * gb % 16 == 0 && rp.C * gb % 16 == 0);
 		t.tile0 = (uint32_t)tiles;
 		t.band0 = (uint32_t)bands;
 		t.ntiles = t.nbx * t.nby;
@@ -4586,7 +4579,7 @@ static uint64_t batch_bytes(uint64_t A, uint64_t C, uint32_t max_rep,
 	t += 4ull * (brec_off(nb_cap_for(C)) - cnt_words(nb_cap_for(C)))
 		+ 4ull * BR_WORDS * nb_cap_for(C);
 	t += 4ull * ((C >> CREP_SHIFT) + 1);   /* the cell-chunk table */
-	t += (C * grass_bytes_for(R) + 3) & ~3ull;
+	t += C * grass_bytes_for(R) + 16;
 	t += (uint64_t)max_rep * (R + 1) * 8;
 	t += hist_words * 4 + RADIX_MAX * 4;
 	{
@@ -4628,8 +4621,8 @@ static int batch_buffers(pp_batch_t *b, Take &&take) {
 		b->keys[i] = b->keys[0] + 2 * i * A4;
 		b->vals[i] = b->keys[i] + A4;
 	}
-	/* (the tile step reads the grass as 32-bit words) */
-	HIP_OK(take((void **)&b->grass_at, ((size_t)C * b->grass_bytes + 3) & ~(size_t)3));
+	/* (the tile step reads the grass in chunks of 16 bytes) */
+	HIP_OK(take((void **)&b->grass_at, (size_t)C * b->grass_bytes + 16));
 	b->ring_stride = b->P.R + 1;
 	HIP_OK(take((void **)&b->ring, (size_t)b->max_rep * b->ring_stride * 8));
 	HIP_OK(take((void **)&b->hist, (size_t)b->hist_alloc_words * 4));

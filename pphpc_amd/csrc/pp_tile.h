@@ -25,9 +25,9 @@
  * What bounds it: on small grids the chain of one group's phases (two round
  * trips to memory, eight barriers, and fetching some 20 KB of instructions
  * that each wave runs through about once); on large ones the vector units.
- * Per iteration, against the three staged kernels: 100 x 100 24.5 -> 8.2 us,
- * 400 x 400 27.5 -> 10.5, 1600 x 1600 41 -> 18.6, 12800 x 12800 768 -> 564;
- * 30 replicas of 1600 x 1600 402 -> 250.
+ * Per iteration, against the three staged kernels: 100 x 100 24.5 -> 7.9 us,
+ * 400 x 400 27.5 -> 10.0, 1600 x 1600 41 -> 18.5, 12800 x 12800 768 -> 576;
+ * 30 replicas of 1600 x 1600 402 -> 249.
  *
  * A tile that outgrows its LDS or border lists sets Ctl::stop; the tick
  * after it is then not run (every group of a later launch returns), and the
@@ -45,7 +45,6 @@ struct TileRep {
 	uint32_t slot, gx, gy, cb, t0, iters, cap, R;
 	uint32_t key0, key1, sheep_gain, wolves_gain, sheep_thr, wolves_thr;
 	uint32_t sheep_prob, wolves_prob, gxm, gxs;
-	uint32_t vec;     /* its tiles' grass is read and written 16 bytes at a time */
 };
 /* ... in the constant address space: scalar loads, placed where they are used */
 typedef __attribute__((address_space(4))) const TileRep TileRepC;
@@ -61,7 +60,7 @@ __device__ __forceinline__ TileRep tile_rep(const TileRep *p, uint32_t k) {
 	r.sheep_gain = c->sheep_gain; r.wolves_gain = c->wolves_gain;
 	r.sheep_thr = c->sheep_thr; r.wolves_thr = c->wolves_thr;
 	r.sheep_prob = c->sheep_prob; r.wolves_prob = c->wolves_prob;
-	r.gxm = c->gxm; r.gxs = c->gxs; r.vec = c->vec;
+	r.gxm = c->gxm; r.gxs = c->gxs;
 	return r;
 }
 
@@ -412,59 +411,42 @@ __device__ __forceinline__ TileGeo tile_geo(const TileRep &tr, uint32_t lt,
 	return g;
 }
 
-/* The tile's grass as rows of 32-bit words: one row of w * h cells (D2 false:
- * the tile's cells are contiguous), or h rows of w cells. A row starts at any
- * cell, so its first word may begin with cells of a neighbour (`phase`). */
+/* 16 bytes of grass at any address (the hardware takes unaligned vectors). */
+struct __attribute__((packed, aligned(1))) Grass16 {
+	uint32_t v[4];
+};
+
+/* The tile's grass as rows of 16-byte chunks: one row of w * h cells (D2
+ * false: the tile's cells are contiguous), or h rows of w cells, 2^csh chunks
+ * apart in LDS. A cell's place in LDS is its cell index. Rows start at any
+ * address: loading and storing 32-bit words at multiples of four, with each
+ * row's first cell anywhere in its first word, was a quarter of the kernel's
+ * instructions where rows are not whole chunks (4001 x 2999: 55 -> 49 us an
+ * iteration, 48 replicas of mixed sizes 102 -> 92, 1013 x 487 11.4 -> 10.8). */
 template <typename GT, bool D2>
 struct TileGrass {
-	static constexpr uint32_t VPW = 4 / sizeof(GT);
-	uint32_t start, gx, n, wpr, wsh, rows;   /* first cell, row stride, cells a row */
+	static constexpr uint32_t VPC = 16 / sizeof(GT);   /* cells of a chunk */
+	uint32_t start, gx, n, csh, rows;
 	__device__ __forceinline__ TileGrass(uint32_t cell0, uint32_t gx_, uint32_t w,
 		uint32_t h, uint32_t shift) {
 		start = cell0;
 		gx = gx_;
 		n = D2 ? w : w * h;
-		rows = D2 ? h : 1u;
-		wsh = D2 ? shift - (VPW == 4 ? 2u : VPW == 2 ? 1u : 0u) : 0u;
-		wpr = 1u << wsh;
+		rows = h;
+		csh = shift - (VPC == 16 ? 4u : VPC == 8 ? 3u : 2u);
 	}
-	/* words in all, and word i: its row and place; false past the row's end */
-	__device__ __forceinline__ uint32_t words() const {
-		return D2 ? rows * (wpr + 1) : (n + VPW - 1) / VPW + 1;
-	}
-	__device__ __forceinline__ bool word(uint32_t i, uint32_t &cell, int32_t &lo,
-		uint32_t &at) const {
-		uint32_t r = 0, c = i;
+	/* chunk i (in LDS order): its first cell and how many of its cells the
+	 * tile has; false: none */
+	__device__ __forceinline__ bool chunk(uint32_t i, uint32_t &cell,
+		uint32_t &cells) const {
+		uint32_t r = 0, x = i * VPC;
 		if (D2) {
-			if (i < rows * wpr) {
-				r = i >> wsh;
-				c = i & (wpr - 1);
-			} else {
-				r = i - rows * wpr;
-				c = wpr;
-			}
+			r = i >> csh;
+			x = (i & ((1u << csh) - 1)) * VPC;
 		}
-		const uint32_t s = start + r * gx, ph = s & (VPW - 1);
-		cell = (s & ~(VPW - 1)) + c * VPW;    /* global cell of the word */
-		lo = (int32_t)(c * VPW) - (int32_t)ph;  /* row cell of its first */
-		at = D2 ? r * (wpr + 1) + c : c;
-		return lo < (int32_t)n;
-	}
-	/* 16-byte chunk i of the tile (rows of 2^csh chunks): its first cell */
-	static constexpr uint32_t VPC = 16 / sizeof(GT);
-	__device__ __forceinline__ bool chunk(uint32_t i, uint32_t &cell) const {
-		if (!D2) {
-			cell = start + i * VPC;
-			return i * VPC < n;
-		}
-		const uint32_t csh = wsh - 2, r = i >> csh, x = (i & ((1u << csh) - 1)) * VPC;
 		cell = start + r * gx + x;
-		return r < rows && x < n;
-	}
-	/* LDS index (in cells) of cell (x, r); c its linear index (D2 false) */
-	__device__ __forceinline__ uint32_t index(uint32_t c, uint32_t x, uint32_t r) const {
-		if (!D2) return (start & (VPW - 1)) + c;
-		return r * (wpr + 1) * VPW + ((start + r * gx) & (VPW - 1)) + x;
+		cells = n - x;
+		return x < n && (!D2 || r < rows);
 	}
 };
 
@@ -476,9 +458,7 @@ __global__ __launch_bounds__(NT) void k_tile(TileArgs A, Ctl *ctl, Tables T,
 	constexpr uint32_t AG = NT * IPT, NW = NT / WAVE;
 	constexpr uint32_t WPT = CELLS / 2 / NT;   /* counter words a thread scans */
 	using TG = TileGrass<GT, D2>;
-	constexpr uint32_t GWORDS = CELLS / TG::VPW + (D2 ? TILE_ROWS : 0u) + 1;
-	constexpr uint32_t GIT = (GWORDS + NT - 1) / NT;
-	constexpr uint32_t VIT = (CELLS / TG::VPC + NT - 1) / NT;
+	constexpr uint32_t CHUNKS = CELLS / TG::VPC, VIT = (CHUNKS + NT - 1) / NT;
 	static_assert(AG <= 4096 && CELLS <= 16384, "list entries");
 	static_assert(NW * IPT <= WAVE, "one wave scans the waves' counts");
 	static_assert(WPT * NT * 2 == CELLS && WPT % 2 == 0, "counter words");
@@ -486,8 +466,12 @@ __global__ __launch_bounds__(NT) void k_tile(TileArgs A, Ctl *ctl, Tables T,
 	__shared__ uint32_t s_val[AG + 8];
 	__shared__ uint32_t s_id[AG + 8];
 	__shared__ uint16_t s_cell[AG + 2];
-	__shared__ uint32_t s_list[AG / 2];
-	__shared__ __align__(16) uint32_t s_grass[GWORDS];
+	/* the list of cells with several agents, over the counters (which the
+	 * agents' places no longer need then) */
+	uint32_t *const s_list = s_cnt;
+	static_assert(AG / 2 <= CELLS / 2, "the list fits");
+	__shared__ uint32_t s_row[D2 ? TILE_ROWS + 1 : 2];   /* first slots of rows */
+	__shared__ uint4 s_grass[CHUNKS];
 	__shared__ uint32_t s_tmp[NW], s_sum[2 * NW], s_wt[WAVE];
 	__shared__ uint32_t s_idoff[D2 ? 3 * TILE_ROWS : 1];
 	__shared__ unsigned long long s_red[NW][8];   /* in TileStat's order */
@@ -555,32 +539,17 @@ __global__ __launch_bounds__(NT) void k_tile(TileArgs A, Ctl *ctl, Tables T,
 			s_idoff[tid] = A.idoff[t * A.rows + r];
 		}
 	}
-	/* the grass, requested now and staged in LDS after the records are: 16
-	 * bytes at a time where rows start and end at multiples of that (a cell's
-	 * LDS index is then its cell index), else by words */
+	/* the grass, requested now and staged in LDS after the records are (a last
+	 * chunk may run on into the next row or replica: those cells are not
+	 * used) */
 	const TG G(cb + g.y0 * gx + g.x0, gx, g.w, g.h, tr.shift);
-	const uint32_t gwords = G.words();
-	const bool vec = tr.vec != 0;
-	uint4 gq[VIT];
-	uint32_t gw[GIT];
-	if (vec) {
+	Grass16 gq[VIT];
 #pragma unroll
-		for (uint32_t i = 0; i < VIT; i++) {
-			uint32_t cell;
-			gq[i] = make_uint4(0, 0, 0, 0);
-			if (G.chunk(i * NT + tid, cell))
-				gq[i] = *reinterpret_cast<const uint4 *>(&grass[cell]);
-		}
-	} else {
-#pragma unroll
-		for (uint32_t i = 0; i < GIT; i++) {
-			uint32_t cell, at;
-			int32_t lo;
-			const uint32_t q = i * NT + tid;
-			gw[i] = 0;
-			if (q < gwords && G.word(q, cell, lo, at))
-				gw[i] = *reinterpret_cast<const uint32_t *>(&grass[cell]);
-		}
+	for (uint32_t i = 0; i < VIT; i++) {
+		uint32_t cell, cells;
+		gq[i] = Grass16{{0, 0, 0, 0}};
+		if (G.chunk(i * NT + tid, cell, cells))
+			gq[i] = *reinterpret_cast<const Grass16 *>(grass + cell);
 	}
 	for (uint32_t i = tid; i < CELLS / 8 + 1; i += NT)
 		*reinterpret_cast<uint4 *>(s_cnt + 4 * i) = make_uint4(0, 0, 0, 0);
@@ -672,20 +641,10 @@ __global__ __launch_bounds__(NT) void k_tile(TileArgs A, Ctl *ctl, Tables T,
 		}
 	}
 	/* grass to LDS: arrived before the records, in issue order */
-	if (vec) {
 #pragma unroll
-		for (uint32_t i = 0; i < VIT; i++)
-			if (VIT * NT * TG::VPC <= CELLS || i * NT + tid < CELLS / TG::VPC)
-				reinterpret_cast<uint4 *>(s_grass)[i * NT + tid] = gq[i];
-	} else {
-#pragma unroll
-		for (uint32_t i = 0; i < GIT; i++) {
-			uint32_t cell, at;
-			int32_t lo;
-			const uint32_t q = i * NT + tid;
-			if (q < gwords && G.word(q, cell, lo, at)) s_grass[at] = gw[i];
-		}
-	}
+	for (uint32_t i = 0; i < VIT; i++)
+		if (VIT * NT == CHUNKS || i * NT + tid < CHUNKS)
+			s_grass[i * NT + tid] = make_uint4(gq[i].v[0], gq[i].v[1], gq[i].v[2], gq[i].v[3]);
 
 	/* 1. the moves; an agent that lands is counted in its cell and keeps its
 	 * place among the cell's arrivals */
@@ -781,6 +740,12 @@ __global__ __launch_bounds__(NT) void k_tile(TileArgs A, Ctl *ctl, Tables T,
 		s_id[q] = ids[j];
 		s_cell[q + 1] = (uint16_t)c;
 	}
+	/* first slot of each row (else: of the second and the last) */
+	if (D2) {
+		for (uint32_t r = tid; r < g.h; r += NT) s_row[r] = s_start[r * g.pitch];
+	} else if (tid < 2) {
+		s_row[tid] = s_start[(tid ? g.h - 1 : g.h > 1 ? 1u : 0u) * g.pitch];
+	}
 	if (tid == 0) {
 		s_cell[0] = 0xFFFFu;
 		s_cell[L + 1] = 0xFFFFu;
@@ -812,7 +777,8 @@ __global__ __launch_bounds__(NT) void k_tile(TileArgs A, Ctl *ctl, Tables T,
 		eaten += 1u << 16;     /* high half: occupied cells */
 		if (s_cell[p + 2] == c) {
 			/* slot, cell and agents (63: that many or more) */
-			const uint32_t kk = s_start[c + 1] - p;
+			uint32_t kk = 2;
+			while (s_cell[p + 1 + kk] == c) kk++;
 			s_list[atomicAdd(&s_nlist, 1u)] = p | (c << 12) | (min(kk, 63u) << 26);
 			continue;
 		}
@@ -821,17 +787,9 @@ __global__ __launch_bounds__(NT) void k_tile(TileArgs A, Ctl *ctl, Tables T,
 		uint32_t thr = wolves_thr;
 		if (!(v & V_WOLF)) {
 			thr = sheep_thr;
-			uint32_t gi = c;
-			if (D2 && !vec) {
-				uint32_t x, r;
-				cell_xr(c, x, r);
-				gi = G.index(c, x, r);
-			} else if (!vec) {
-				gi = G.index(c, 0, 0);
-			}
-			if (grass_alive_at<GT>(s_g[gi], tick + 1, P.R)) {
+			if (grass_alive_at<GT>(s_g[c], tick + 1, P.R)) {
 				e += (int32_t)sheep_gain;
-				s_g[gi] = (GT)(tick + 1 + R);
+				s_g[c] = (GT)(tick + 1 + R);
 				eaten++;
 			}
 		}
@@ -849,18 +807,17 @@ __global__ __launch_bounds__(NT) void k_tile(TileArgs A, Ctl *ctl, Tables T,
 #pragma unroll 1
 		for (uint32_t i = tid; i < nlist; i += NT) {
 			const uint32_t en = s_list[i], p = en & 0xFFFu, c = (en >> 12) & 0x3FFFu;
-			uint32_t kk = en >> 26, cl, gi;
-			if (kk == 63) kk = s_start[c + 1] - p;
+			uint32_t kk = en >> 26, cl;
+			if (kk == 63)
+				while (s_cell[p + 1 + kk] == c) kk++;
 			if (D2) {
 				uint32_t x, r;
 				cell_xr(c, x, r);
 				cl = (g.y0 + r) * gx + g.x0 + x;
-				gi = vec ? c : G.index(c, x, r);
 			} else {
 				cl = g.y0 * gx + c;
-				gi = vec ? c : G.index(c, 0, 0);
 			}
-			const bool alive = grass_alive_at<GT>(s_g[gi], tick + 1, P.R);
+			const bool alive = grass_alive_at<GT>(s_g[c], tick + 1, P.R);
 			bool ate;
 			if (kk <= 4)
 				ate = tile_cell<4>(s_val, s_id, p, kk, alive, cl, step, key0, key1,
@@ -872,7 +829,7 @@ __global__ __launch_bounds__(NT) void k_tile(TileArgs A, Ctl *ctl, Tables T,
 				ate = tile_cell_any(s_val, s_id, p, kk, alive, cl, step, key0, key1,
 					sheep_gain, wolves_gain, sheep_thr, wolves_thr, &ovf);
 			if (ate) {
-				s_g[gi] = (GT)(tick + 1 + R);
+				s_g[c] = (GT)(tick + 1 + R);
 				eaten++;
 			}
 		}
@@ -979,49 +936,27 @@ __global__ __launch_bounds__(NT) void k_tile(TileArgs A, Ctl *ctl, Tables T,
 	}
 	/* the grass back; alive cells are re-stamped now and then (see REFRESH) */
 	const bool restamp = tick % TILE_RESTAMP == 0;
-	auto stamped = [&](uint32_t v) {
-		GT gv[TG::VPW];
-		__builtin_memcpy(gv, &v, 4);
-#pragma unroll
-		for (uint32_t u = 0; u < TG::VPW; u++)
-			if (grass_alive_at<GT>(gv[u], tick + 1, P.R)) gv[u] = (GT)(tick + 1);
-		__builtin_memcpy(&v, gv, 4);
-		return v;
-	};
-	if (vec) {
 #pragma unroll 1
-		for (uint32_t i = tid; i < CELLS / TG::VPC; i += NT) {
-			uint32_t cell;
-			if (!G.chunk(i, cell)) continue;
-			uint4 v = reinterpret_cast<const uint4 *>(s_grass)[i];
-			if (restamp)
-				v = make_uint4(stamped(v.x), stamped(v.y), stamped(v.z), stamped(v.w));
-			*reinterpret_cast<uint4 *>(&grass[cell]) = v;
+	for (uint32_t i = tid; i < CHUNKS; i += NT) {
+		uint32_t cell, cells;
+		if (!G.chunk(i, cell, cells)) continue;
+		if (restamp) {
+			GT *q = s_g + i * TG::VPC;
+#pragma unroll 1
+			for (uint32_t u = 0; u < TG::VPC; u++)
+				if (grass_alive_at<GT>(q[u], tick + 1, P.R)) q[u] = (GT)(tick + 1);
 		}
-	} else {
-#pragma unroll 1
-		for (uint32_t q = tid; q < gwords; q += NT) {
-			uint32_t cell, at;
-			int32_t lo;
-			if (!G.word(q, cell, lo, at)) continue;
-			uint32_t v = s_grass[at];
-			if (restamp) v = stamped(v);
-			if (lo >= 0 && (uint32_t)lo + TG::VPW <= G.n) {
-				*reinterpret_cast<uint32_t *>(&grass[cell]) = v;
-			} else {
-				GT gv[TG::VPW];
-				__builtin_memcpy(gv, &v, 4);
-#pragma unroll
-				for (uint32_t u = 0; u < TG::VPW; u++)
-					if (lo + (int32_t)u >= 0 && (uint32_t)(lo + (int32_t)u) < G.n)
-						grass[cell + u] = gv[u];
-			}
+		if (cells >= TG::VPC) {
+			const uint4 v = s_grass[i];
+			*reinterpret_cast<Grass16 *>(grass + cell) = Grass16{{v.x, v.y, v.z, v.w}};
+		} else {
+			for (uint32_t u = 0; u < cells; u++) grass[cell + u] = s_g[i * TG::VPC + u];
 		}
 	}
 	__syncthreads();
 	/* first record of each row (the output offset of the row's first slot) */
 	auto row_first = [&](uint32_t r) {
-		const uint32_t q = s_start[r * g.pitch];
+		const uint32_t q = s_row[D2 ? r : r == 1 && g.h > 2 ? 0u : 1u];
 		return q < L ? s_id[q] : nout;
 	};
 	if (D2)
