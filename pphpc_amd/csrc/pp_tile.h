@@ -25,9 +25,9 @@
  * What bounds it: on small grids the chain of one group's phases (two round
  * trips to memory, eight barriers, and fetching some 20 KB of instructions
  * that each wave runs through about once); on large ones the vector units.
- * Per iteration, against the three staged kernels: 100 x 100 24.5 -> 7.9 us,
- * 400 x 400 27.5 -> 10.0, 1600 x 1600 41 -> 18.5, 12800 x 12800 768 -> 576;
- * 30 replicas of 1600 x 1600 402 -> 249.
+ * Per iteration, against the three staged kernels: 100 x 100 24.5 -> 7.3 us,
+ * 400 x 400 27.5 -> 9.6, 1600 x 1600 41 -> 18.4, 12800 x 12800 768 -> 561;
+ * 30 replicas of 1600 x 1600 402 -> 242.
  *
  * A tile that outgrows its LDS or border lists sets Ctl::stop; the tick
  * after it is then not run (every group of a later launch returns), and the
@@ -118,10 +118,8 @@ __device__ __forceinline__ uint32_t tile_cur(const Ctl *ctl) {
  * during tick t names tick t + 1 (as t + 2: 0 is none), so it does not touch
  * the groups of tick t that start later; the first launch that does not run
  * halts the others, which would find the tick before in their buffers. */
-__device__ __forceinline__ bool tile_runs(const Ctl *ctl, uint32_t t) {
-	/* (all loads at once, not one after another) */
-	const uint32_t stop = ctl->stop, halt = ctl->halt;
-	const int32_t error = ctl->error;
+__device__ __forceinline__ bool tile_runs(uint32_t error, uint32_t stop,
+	uint32_t halt, uint32_t t) {
 	return (error == 0) & (halt == 0) & ((stop == 0) | ((int32_t)(t + 1 - stop) < 0));
 }
 
@@ -466,10 +464,7 @@ __global__ __launch_bounds__(NT) void k_tile(TileArgs A, Ctl *ctl, Tables T,
 	__shared__ uint32_t s_val[AG + 8];
 	__shared__ uint32_t s_id[AG + 8];
 	__shared__ uint16_t s_cell[AG + 2];
-	/* the list of cells with several agents, over the counters (which the
-	 * agents' places no longer need then) */
-	uint32_t *const s_list = s_cnt;
-	static_assert(AG / 2 <= CELLS / 2, "the list fits");
+	__shared__ uint32_t s_list[AG / 2];   /* the cells with several agents */
 	__shared__ uint32_t s_row[D2 ? TILE_ROWS + 1 : 2];   /* first slots of rows */
 	__shared__ uint4 s_grass[CHUNKS];
 	__shared__ uint32_t s_tmp[NW], s_sum[2 * NW], s_wt[WAVE];
@@ -479,12 +474,34 @@ __global__ __launch_bounds__(NT) void k_tile(TileArgs A, Ctl *ctl, Tables T,
 
 	const uint32_t tid = threadIdx.x, lane = tid & (WAVE - 1);
 	const uint32_t w = __builtin_amdgcn_readfirstlane(tid / WAVE);
-	const uint32_t tick = __builtin_amdgcn_readfirstlane(ctl->tt[A.par]);
+	/* A group that has its CU to itself waits for each of its first loads, and
+	 * a scalar load is waited for together with every other one, so that a
+	 * chain of six round trips stood before the first barrier (1.5 us): all
+	 * arguments that they need are taken at once, and the uniform values come
+	 * as vector loads, a word a lane (100 x 100: 7.9 -> 7.7 us). In tiles of
+	 * 256 columns, where other groups fill the wait, scalar loads are the
+	 * faster (12800 x 12800: 577 us, 620 with vector loads, which queue behind
+	 * the records). */
+	if (!D2)
+		asm volatile("" :: "s"(A.in), "s"(A.hin), "s"(grass), "s"(ctl), "s"(T.rctl),
+			"s"(A.slot), "s"(A.ntiles), "s"(A.nfin), "s"(A.par));
+	if (SOLO && !D2)
+		asm volatile("" :: "s"(A.one.tile0), "s"(A.one.ntiles), "s"(A.one.gx),
+			"s"(A.one.gy), "s"(A.one.cb), "s"(A.one.slot), "s"(A.one.by), "s"(A.one.nby));
+	uint32_t cw = 0;
+	if (!D2) cw = reinterpret_cast<const uint32_t *>(ctl)[lane & 15u];
+	static_assert(offsetof(Ctl, error) == 4 * 4 && offsetof(Ctl, tt) == 12 * 4 &&
+		offsetof(Ctl, stop) == 14 * 4 && offsetof(Ctl, halt) == 15 * 4, "words of Ctl");
+	auto ctl_word = [&](uint32_t i) {
+		return D2 ? reinterpret_cast<const uint32_t *>(ctl)[i]
+			: (uint32_t)__builtin_amdgcn_readlane((int)cw, (int)i);
+	};
 	if (blockIdx.x < A.nfin) {
-		const uint32_t k = blockIdx.x;
+		const uint32_t k = blockIdx.x, tick = ctl_word(12 + A.par);
+		const bool runs = tile_runs(ctl_word(4), ctl_word(14), ctl_word(15), tick);
 		if (k == 0) {
 			if (tid == 0) {
-				if (tile_runs(ctl, tick)) {
+				if (runs) {
 					ctl->tt[1 - A.par] = tick + 1;
 					A.spare[A.par] = 0;   /* for the next tick's outputs */
 				} else {
@@ -508,26 +525,41 @@ __global__ __launch_bounds__(NT) void k_tile(TileArgs A, Ctl *ctl, Tables T,
 	if (b / NXCD >= per || tile >= A.ntiles) return;
 	const uint32_t k = SOLO ? 0u : __builtin_amdgcn_readfirstlane(A.tk[tile]);
 	const TileRep tr = SOLO ? A.one : tile_rep(A.trep, k);
-	const uint32_t gx = tr.gx, gy = tr.gy, cb = tr.cb, step = tick - tr.t0;
+	const uint32_t gx = tr.gx, gy = tr.gy, cb = tr.cb;
 	const uint32_t key0 = tr.key0, key1 = tr.key1;
-	const uint32_t c_status = T.rctl[tr.slot].status, c_ovf = T.rctl[tr.slot].ovf;
 	const uint32_t lt = tile - tr.tile0;
 	const TileGeo g = tile_geo<D2>(tr, lt, gx, gy);
 	const bool wrapx = tr.nbx == 1, wrapy = tr.nby == 1;
-	const uint4 h_own = A.hin[tile], h_up = A.hin[g.up], h_dn = A.hin[g.down];
+	/* headers: this tile's, up, down, left, right */
+	uint4 hs[5];
+	uint32_t hw = 0, rw = 0, d2_status = 0, d2_over = 0;
+	if (D2) {
+		hs[0] = A.hin[tile];
+		hs[1] = A.hin[g.up];
+		hs[2] = A.hin[g.down];
+		hs[3] = A.hin[g.left];
+		hs[4] = A.hin[g.right];
+		d2_status = T.rctl[tr.slot].status;
+		d2_over = T.rctl[tr.slot].ovf;
+	} else {
+		uint32_t ht = tile;
+		if (lane >= 4) ht = g.up;
+		if (lane >= 8) ht = g.down;
+		hw = reinterpret_cast<const uint32_t *>(A.hin)[ht * 4 + (lane & 3u)];
+		rw = reinterpret_cast<const uint32_t *>(T.rctl + tr.slot)[lane & 7u];
+	}
+	static_assert(offsetof(RepCtl, status) == 3 * 4 && offsetof(RepCtl, ovf) == 6 * 4,
+		"words of RepCtl");
+	auto header = [&](uint32_t i) {
+		const uint4 h = hs[i >> 2];
+		const uint32_t j = i & 3u;
+		return D2 ? (j == 0 ? h.x : j == 1 ? h.y : j == 2 ? h.z : h.w)
+			: (uint32_t)__builtin_amdgcn_readlane((int)hw, (int)i);
+	};
 	/* the ids: the agents of the replica's tiles before this one */
 	uint32_t bef = 0, all = 0;
 	if (!D2) {
-		for (uint32_t i = tid; i < tr.ntiles; i += NT) {
-			const uint32_t n = A.hin[tr.tile0 + i].x;
-			all += n;
-			bef += i < lt ? n : 0u;
-		}
-	}
-	uint4 h_l = make_uint4(0, 0, 0, 0), h_r = h_l;
-	if (D2 && !wrapx) {
-		h_l = A.hin[g.left];
-		h_r = A.hin[g.right];
+		if (tid < tr.ntiles) all = A.hin[tr.tile0 + tid].x;
 	}
 	if (D2 && tid < 3 * TILE_ROWS) {
 		const uint32_t q = tid / TILE_ROWS, r = tid % TILE_ROWS;
@@ -554,19 +586,34 @@ __global__ __launch_bounds__(NT) void k_tile(TileArgs A, Ctl *ctl, Tables T,
 	for (uint32_t i = tid; i < CELLS / 8 + 1; i += NT)
 		*reinterpret_cast<uint4 *>(s_cnt + 4 * i) = make_uint4(0, 0, 0, 0);
 	if (tid < WAVE) s_wt[tid] = 0;
+	const uint32_t tick = ctl_word(12 + A.par), step = tick - tr.t0;
+	/* (words are taken from their lanes outside of branches, where all lanes
+	 * have loaded) */
+	const uint32_t status = D2 ? d2_status
+		: (uint32_t)__builtin_amdgcn_readlane((int)rw, 3);
+	const uint32_t over = D2 ? d2_over
+		: (uint32_t)__builtin_amdgcn_readlane((int)rw, 6);
+	/* A replica that is done or has failed no longer moves. Its status is
+	 * that before or after the end of the last tick, written beside this:
+	 * both give the same answer. (One thread decides for the group: an energy
+	 * limit or an error may be noted meanwhile.) */
+	const bool go = tile_runs(ctl_word(4), ctl_word(14), ctl_word(15), tick) &
+		(status == RS_ACTIVE) & (step < tr.iters) &
+		((over == 0) | (over == tick + 1));
 	if (tid == 0) {
 		s_nlist = 0;
 		s_ovf = 0;
 		s_edge[0] = s_edge[1] = 0;
-		/* A replica that is done or has failed no longer moves. Its status
-		 * is that before or after the end of the last tick, written beside
-		 * this: both give the same answer. (One thread decides for the
-		 * group: an energy limit or an error may be noted meanwhile.) */
-		s_go = tile_runs(ctl, tick) & (c_status == RS_ACTIVE) & (step < tr.iters) &
-			((c_ovf == 0) | (c_ovf == tick + 1));
+		s_go = go;
 	}
 	uint32_t idb = 0, idb_up = 0, idb_dn = 0, total_in;
 	if (!D2) {
+		bef = tid < lt ? all : 0u;
+		for (uint32_t i = tid + NT; i < tr.ntiles; i += NT) {
+			const uint32_t n = A.hin[tr.tile0 + i].x;
+			all += n;
+			bef += i < lt ? n : 0u;
+		}
 		all = wave_sum32(all);
 		bef = wave_sum32(bef);
 		if (lane == 0) {
@@ -589,11 +636,11 @@ __global__ __launch_bounds__(NT) void k_tile(TileArgs A, Ctl *ctl, Tables T,
 	}
 	if (!s_go || total_in > tr.cap || total_in > P.cap) return;
 
-	const uint32_t n0 = __builtin_amdgcn_readfirstlane(h_own.x);
-	const uint32_t nup = wrapy ? 0u : __builtin_amdgcn_readfirstlane(h_up.y >> 16);
-	const uint32_t ndn = wrapy ? 0u : __builtin_amdgcn_readfirstlane(h_dn.y & 0xFFFFu);
-	const uint32_t nl = D2 ? __builtin_amdgcn_readfirstlane(h_l.z >> 16) : 0u;
-	const uint32_t nr = D2 ? __builtin_amdgcn_readfirstlane(h_r.z & 0xFFFFu) : 0u;
+	const uint32_t n0 = header(0);
+	const uint32_t nup = wrapy ? 0u : header(4 + 1) >> 16;
+	const uint32_t ndn = wrapy ? 0u : header(8 + 1) & 0xFFFFu;
+	const uint32_t nl = D2 && !wrapx ? header(12 + 2) >> 16 : 0u;
+	const uint32_t nr = D2 && !wrapx ? header(16 + 2) & 0xFFFFu : 0u;
 	const uint32_t i1 = n0, i2 = i1 + nup, i3 = i2 + ndn, i4 = i3 + nl, i5 = i4 + nr;
 	if (i5 > AG) {
 		/* (the limits set when the records were written exclude this) */
@@ -601,14 +648,14 @@ __global__ __launch_bounds__(NT) void k_tile(TileArgs A, Ctl *ctl, Tables T,
 		return;
 	}
 	/* positions and ids of the ranges, as offsets from the item index */
-	const uint32_t first_up = __builtin_amdgcn_readfirstlane(h_up.x) - nup;
-	const uint32_t p_own = __builtin_amdgcn_readfirstlane(h_own.w);
-	const uint32_t p_up = __builtin_amdgcn_readfirstlane(h_up.w) + first_up - i1;
-	const uint32_t p_dn = __builtin_amdgcn_readfirstlane(h_dn.w) - i2;
+	const uint32_t first_up = header(4) - nup;
+	const uint32_t p_own = header(3);
+	const uint32_t p_up = header(4 + 3) + first_up - i1;
+	const uint32_t p_dn = header(8 + 3) - i2;
 	uint32_t p_l = 0, p_r = 0;
 	if (!D2) {
-		idb_up = (lt ? idb - __builtin_amdgcn_readfirstlane(h_up.x)
-			: total_in - __builtin_amdgcn_readfirstlane(h_up.x)) + first_up - i1;
+		idb_up = (lt ? idb - header(4)
+			: total_in - header(4)) + first_up - i1;
 		idb_dn = (lt + 1 < tr.ntiles ? idb + n0 : 0u) - i2;
 	} else {
 		const uint32_t uh = min(tr.by, gy - (g.y0 ? g.y0 - tr.by : (tr.nby - 1) * tr.by));
@@ -735,7 +782,16 @@ __global__ __launch_bounds__(NT) void k_tile(TileArgs A, Ctl *ctl, Tables T,
 	for (int j = 0; j < IPT; j++) {
 		if ((uint32_t)j * NT >= i5) break;
 		if (pk[j] == 0xFFFFFFFFu) continue;
-		const uint32_t c = pk[j] & 0xFFFFu, q = s_start[c] + (pk[j] >> 16);
+		const uint32_t c = pk[j] & 0xFFFFu, c0 = s_start[c];
+		const uint32_t q = c0 + (pk[j] >> 16);
+		/* a cell with several agents is listed by the second that came (the
+		 * asm keeps the compiler from first adding up lanes that share an
+		 * atomic, which takes more than the few atomics do) */
+		if (pk[j] >> 16 == 1) {
+			uint32_t z = 0;
+			asm("" : "+v"(z));
+			s_list[atomicAdd(&s_nlist + z, 1u)] = c0 | (c << 12);
+		}
 		s_val[q] = vv[j];
 		s_id[q] = ids[j];
 		s_cell[q + 1] = (uint16_t)c;
@@ -752,8 +808,13 @@ __global__ __launch_bounds__(NT) void k_tile(TileArgs A, Ctl *ctl, Tables T,
 	}
 	__syncthreads();
 
-	/* 3. actions: cells of one agent in place, the others listed and then
-	 * acted on by consecutive lanes */
+	/* 3. actions: the listed cells, dealt out from the last lane on, and
+	 * those of one agent, from the first: where there are few of both,
+	 * different waves act on them at the same time (100 x 100: 7.7 -> 7.3 us,
+	 * 12800 x 12800 576 -> 561, against those of one agent first, listing the
+	 * others, and these after a barrier; with a cell's single agent acting
+	 * from its registers in the loop above 7.5 and 548, 1600 x 1600 18.4 ->
+	 * 18.7) */
 	const uint32_t sheep_gain = tr.sheep_gain, wolves_gain = tr.wolves_gain;
 	const uint32_t sheep_thr = tr.sheep_thr, wolves_thr = tr.wolves_thr, R = tr.R;
 	GT *s_g = reinterpret_cast<GT *>(s_grass);
@@ -767,49 +828,13 @@ __global__ __launch_bounds__(NT) void k_tile(TileArgs A, Ctl *ctl, Tables T,
 			x = c - r * gx;
 		}
 	};
-	/* (this loop and those below are not unrolled: a group runs through the
-	 * code about once, and fetching instructions is then what takes the time) */
 	uint32_t eaten = 0, ovf = 0;
-#pragma unroll 1
-	for (uint32_t p = tid; p < L; p += NT) {
-		const uint32_t c = s_cell[p + 1];
-		if (s_cell[p] == c) continue;
-		eaten += 1u << 16;     /* high half: occupied cells */
-		if (s_cell[p + 2] == c) {
-			/* slot, cell and agents (63: that many or more) */
-			uint32_t kk = 2;
-			while (s_cell[p + 1 + kk] == c) kk++;
-			s_list[atomicAdd(&s_nlist, 1u)] = p | (c << 12) | (min(kk, 63u) << 26);
-			continue;
-		}
-		const uint32_t v = s_val[p];
-		int32_t e = (int32_t)(v & V_ENERGY);
-		uint32_t thr = wolves_thr;
-		if (!(v & V_WOLF)) {
-			thr = sheep_thr;
-			if (grass_alive_at<GT>(s_g[c], tick + 1, P.R)) {
-				e += (int32_t)sheep_gain;
-				s_g[c] = (GT)(tick + 1 + R);
-				eaten++;
-			}
-		}
-		uint32_t nv = v & V_WOLF;
-		if (e > (int32_t)thr && (v & V_REPRO)) {
-			nv |= V_CHILD | ((e & 1) ? V_ODD : 0u);
-			e -= e / 2;
-		}
-		if (e > (int32_t)V_ENERGY) ovf = 1;
-		s_val[p] = nv | ((uint32_t)e & V_ENERGY);
-	}
-	__syncthreads();
 	{
 		const uint32_t nlist = s_nlist;
 #pragma unroll 1
-		for (uint32_t i = tid; i < nlist; i += NT) {
-			const uint32_t en = s_list[i], p = en & 0xFFFu, c = (en >> 12) & 0x3FFFu;
-			uint32_t kk = en >> 26, cl;
-			if (kk == 63)
-				while (s_cell[p + 1 + kk] == c) kk++;
+		for (uint32_t i = NT - 1 - tid; i < nlist; i += NT) {
+			const uint32_t en = s_list[i], p = en & 0xFFFu, c = en >> 12;
+			uint32_t kk = s_start[c + 1] - p, cl;
 			if (D2) {
 				uint32_t x, r;
 				cell_xr(c, x, r);
@@ -833,6 +858,32 @@ __global__ __launch_bounds__(NT) void k_tile(TileArgs A, Ctl *ctl, Tables T,
 				eaten++;
 			}
 		}
+	}
+	/* (this loop and those below are not unrolled: a group runs through the
+	 * code about once, and fetching instructions is then what takes the time) */
+#pragma unroll 1
+	for (uint32_t p = tid; p < L; p += NT) {
+		const uint32_t c = s_cell[p + 1];
+		if (s_cell[p] == c || s_cell[p + 2] == c) continue;
+		eaten += 1u << 16;     /* high half: these cells */
+		const uint32_t v = s_val[p];
+		int32_t e = (int32_t)(v & V_ENERGY);
+		uint32_t thr = wolves_thr;
+		if (!(v & V_WOLF)) {
+			thr = sheep_thr;
+			if (grass_alive_at<GT>(s_g[c], tick + 1, P.R)) {
+				e += (int32_t)sheep_gain;
+				s_g[c] = (GT)(tick + 1 + R);
+				eaten++;
+			}
+		}
+		uint32_t nv = v & V_WOLF;
+		if (e > (int32_t)thr && (v & V_REPRO)) {
+			nv |= V_CHILD | ((e & 1) ? V_ODD : 0u);
+			e -= e / 2;
+		}
+		if (e > (int32_t)V_ENERGY) ovf = 1;
+		s_val[p] = nv | ((uint32_t)e & V_ENERGY);
 	}
 	if (ovf) s_ovf = 1;
 	__syncthreads();
@@ -874,7 +925,7 @@ __global__ __launch_bounds__(NT) void k_tile(TileArgs A, Ctl *ctl, Tables T,
 			s_red[w][0] = n_all - n_wolves;
 			s_red[w][1] = n_wolves;
 			s_red[w][2] = ne & 0xFFFFu;
-			s_red[w][3] = ne >> 16;
+			s_red[w][3] = (ne >> 16) + (w == 0 ? s_nlist : 0u);
 			s_red[w][4] = n_birth;
 			s_red[w][5] = w == 0 ? L : 0u;
 			s_red[w][6] = ea - ew;
