@@ -3351,7 +3351,7 @@ constexpr uint32_t TILE_WIDE = 2048, TILE_MIN = 400;
 struct TileShape {
 	uint32_t nt, ipt, cells;
 };
-const TileShape tile_shapes[] = {{256, 7, 4096}, {512, 8, 8192}};
+const TileShape tile_shapes[] = {{256, 7, 4096}, {512, 8, 8192}, {1024, 8, 16384}};
 
 } /* namespace */
 
@@ -3804,8 +3804,11 @@ static void launch_tile(pp_batch_t *b) {
 	if (b->plan.cfg == 0)
 		k_tile<GT, 256, 7, 4096, D2, SOLO><<<grid, 256, 0, b->stream>>>(a, b->ctl,
 			b->tables(), b->P, b->table_nrep, g);
-	else
+	else if (b->plan.cfg == 1)
 		k_tile<GT, 512, 8, 8192, D2, SOLO><<<grid, 512, 0, b->stream>>>(a, b->ctl,
+			b->tables(), b->P, b->table_nrep, g);
+	else if constexpr (!D2 && sizeof(GT) < 4)
+		k_tile<GT, 1024, 8, 16384, D2, SOLO><<<grid, 1024, 0, b->stream>>>(a, b->ctl,
 			b->tables(), b->P, b->table_nrep, g);
 	if (D2)
 		k_tile_scan<<<a.nbands, WG, 0, b->stream>>>(a, b->ctl, b->tables(),
@@ -3987,17 +3990,22 @@ struct TileGrid {
 /* Chooses the tiles of a replica table (n grids in table order) and places
  * the tile step's arrays in the memory of the bucket sort's tables, which the
  * tile step does not use. Up to TILE_WIDE columns a tile is a run of whole rows
- * (its ids then follow from one sum over the tiles' counts; 1600 x 1600: 18.6
- * us an iteration, against 28 in tiles of 256 x 16 with their scan of the
+ * (its ids then follow from one sum over the tiles' counts; 1600 x 1600: 17 us
+ * an iteration, against 28 in tiles of 256 x 16 with their scan of the
  * rows' counts after each iteration); wider grids are cut into 256 columns.
- * One replica takes about as many tiles as run at once: four groups of 256
- * threads a CU hold up to 1024, of which 256 are taken (400 x 400: 10.3 us
- * with tiles of 2 or 4 rows, 11.2 of 8; 7 slots a thread, which 32 KB of LDS
- * hold with four groups, 1013 x 487 10.8 us, 11.4 with 8), else two groups of 512 (1600 x 1600:
- * 18.6 us with 400 tiles of 4 rows, 20.4 with 320 of 5, 23.7 with 534 of 3, a
- * second round). Several replicas fill the GPU with tiles as large as fit,
- * which move fewer neighbours' agents twice (30 x 1600 x 1600: 248 us with 5
- * rows, 284 with 4). PPHPC_TILE=shape,columns,rows sets them (columns 0: whole
+ * About one tile a CU is taken where tiles can be that large, so that all run
+ * at once, in the smallest shape that gives a thread no more than two agents
+ * (four in the next; the neighbours' border rows count): 400 x 400 9.6 us
+ * (256 threads), 600 x 600 10.7 (512; 11.4 with 256, 11.1 with 1024), 1013 x
+ * 487 9.7 (512; 10.3 with 256), 1600 x 1600 17.0 (1024, 229 tiles of 7 rows;
+ * 18.4 with 400 tiles of 4 rows, two groups of 512 a CU). Several replicas take
+ * no groups of 1024, which cannot overlap with another on their CU. Where the
+ * cells are too many for that, one replica takes two groups of 512 a CU (1500 x
+ * 3000: 27.3 us, 28.6 with two rounds of 1024), several replicas tiles as large
+ * as fit, which move fewer neighbours' agents twice (30 x 1600 x 1600: 242 us
+ * with 5 rows, 284 with 4; 273 with 1024 threads and 10 rows). Small batches
+ * were in tiles as large as fit, too: 10 x 100 x 100 13.8 -> 10.0 us, 30 x 128 x
+ * 128 15.8 -> 12.9. PPHPC_TILE=shape,columns,rows sets them (columns 0: whole
  * rows; shape -1: the staged step); results do not depend on them. */
 static void tile_layout(const pp_batch_t *b, const TileGrid *grid, uint32_t n,
 	TilePlan &p) {
@@ -4019,7 +4027,7 @@ static void tile_layout(const pp_batch_t *b, const TileGrid *grid, uint32_t n,
 	uint32_t ebx = 0, eby = 0;
 	int ecfg = -2;
 	if (const char *e = getenv("PPHPC_TILE")) sscanf(e, "%d,%u,%u", &ecfg, &ebx, &eby);
-	if (ecfg == -1) return;
+	if (ecfg == -1 || ecfg > 2) return;
 	if (ebx) p.d2 = true;
 	/* rows of a tile (at most) in shape c: its cells, and most of the agents
 	 * it may hold (with rows filled further than 0.87, or border rows of less
@@ -4037,14 +4045,38 @@ static void tile_layout(const pp_batch_t *b, const TileGrid *grid, uint32_t n,
 	auto rows_max = [&](uint32_t w) {
 		return std::min((double)tile_shapes[p.cfg].cells / w, fill * p.nmax / (dens * w));
 	};
+	/* cells of a tile, whole rows: of about as many tiles as CUs, and no more
+	 * tiles than that where tiles up to twice as large allow it */
+	const uint32_t cus = (uint32_t)b->num_cu;
+	uint64_t quota = ceil_div(cells, cus);
+	auto rows_for = [&](uint32_t gx, uint64_t q) {
+		return ceil_div(std::max<uint64_t>(q, TILE_MIN), gx);
+	};
+	for (uint64_t q = quota; n > 1 && q < 2 * quota; q += q / 16 + 1) {
+		uint64_t t = 0;
+		for (uint32_t i = 0; i < n; i++)
+			t += ceil_div(grid[i].rep->gy, rows_for(grid[i].rep->gx, q));
+		if (t > cus) continue;
+		quota = q;
+		break;
+	}
+	const int shapes = n == 1 && b->grass_bytes < 4 ? 3 : 2;
+	int c = 0;
+	for (; c < shapes && !p.d2; c++) {
+		limits(c);
+		const uint32_t by = rows_for(width, quota);
+		if (by <= rows_max(width) && dens * width * (by + 2) <=
+				tile_shapes[c].nt * (c + 1 == shapes ? tile_shapes[c].ipt : c ? 4u : 2u))
+			break;
+	}
 	if (p.d2) {
 		limits(0);
-	} else {
-		limits(0);
-		/* one replica: enough tiles to use every CU */
-		const double want = n > 1 ? 1e9 : (double)cells / width / 256;
-		if (want > rows_max(width)) limits(1);
+	} else if (c == shapes) {
+		limits(1);
+		quota = n == 1 ? ceil_div(cells, 2 * cus) : UINT32_MAX;
 	}
+	/* (the largest shape's LDS does not hold four-byte grass) */
+	if (ecfg == 2 && (p.d2 || b->grass_bytes == 4)) return;
 	if (ecfg >= 0) limits(ecfg);
 	const TileShape sh = tile_shapes[p.cfg];
 	uint64_t tiles = 0, bands = 0;
@@ -4081,12 +4113,7 @@ static void tile_layout(const pp_batch_t *b, const TileGrid *grid, uint32_t n,
 			const double most = rows_max(gx);
 			uint32_t by = (uint32_t)std::min(most, 65535.0);
 			if (!by) return;
-			if (n == 1) {
-				/* one round of groups: as many tiles as fit, of at least
-				 * TILE_MIN cells */
-				const uint32_t round = p.cfg == 0 ? 256 : 512;
-				by = min_u32(by, std::max(ceil_div(gy, round), ceil_div(TILE_MIN, gx)));
-			}
+			by = min_u32(by, rows_for(gx, quota));
 			t.by = by;
 		} else {
 			t.bx = min_u32(ebx ? ebx : 256, gx);

@@ -457,17 +457,18 @@ __global__ __launch_bounds__(NT) void k_tile(TileArgs A, Ctl *ctl, Tables T,
 	constexpr uint32_t WPT = CELLS / 2 / NT;   /* counter words a thread scans */
 	using TG = TileGrass<GT, D2>;
 	constexpr uint32_t CHUNKS = CELLS / TG::VPC, VIT = (CHUNKS + NT - 1) / NT;
-	static_assert(AG <= 4096 && CELLS <= 16384, "list entries");
-	static_assert(NW * IPT <= WAVE, "one wave scans the waves' counts");
+	constexpr uint32_t NWT = NW * IPT > WAVE ? 2u : 1u;   /* waves' counts a lane scans */
+	static_assert(AG < 65536 && CELLS < 65536, "16-bit slots and cells");
+	static_assert(NW * IPT <= 2 * WAVE, "one wave scans the waves' counts");
 	static_assert(WPT * NT * 2 == CELLS && WPT % 2 == 0, "counter words");
 	__shared__ __align__(16) uint32_t s_cnt[CELLS / 2 + 4];
 	__shared__ uint32_t s_val[AG + 8];
 	__shared__ uint32_t s_id[AG + 8];
 	__shared__ uint16_t s_cell[AG + 2];
-	__shared__ uint32_t s_list[AG / 2];   /* the cells with several agents */
+	__shared__ uint16_t s_list[AG / 2];   /* first slots of cells with several agents */
 	__shared__ uint32_t s_row[D2 ? TILE_ROWS + 1 : 2];   /* first slots of rows */
 	__shared__ uint4 s_grass[CHUNKS];
-	__shared__ uint32_t s_tmp[NW], s_sum[2 * NW], s_wt[WAVE];
+	__shared__ uint32_t s_tmp[NW], s_sum[2 * NW], s_wt[NWT * WAVE];
 	__shared__ uint32_t s_idoff[D2 ? 3 * TILE_ROWS : 1];
 	__shared__ unsigned long long s_red[NW][8];   /* in TileStat's order */
 	__shared__ uint32_t s_nlist, s_ovf, s_go, s_edge[2];
@@ -585,7 +586,7 @@ __global__ __launch_bounds__(NT) void k_tile(TileArgs A, Ctl *ctl, Tables T,
 	}
 	for (uint32_t i = tid; i < CELLS / 8 + 1; i += NT)
 		*reinterpret_cast<uint4 *>(s_cnt + 4 * i) = make_uint4(0, 0, 0, 0);
-	if (tid < WAVE) s_wt[tid] = 0;
+	if (tid < NWT * WAVE) s_wt[tid] = 0;
 	const uint32_t tick = ctl_word(12 + A.par), step = tick - tr.t0;
 	/* (words are taken from their lanes outside of branches, where all lanes
 	 * have loaded) */
@@ -790,7 +791,7 @@ __global__ __launch_bounds__(NT) void k_tile(TileArgs A, Ctl *ctl, Tables T,
 		if (pk[j] >> 16 == 1) {
 			uint32_t z = 0;
 			asm("" : "+v"(z));
-			s_list[atomicAdd(&s_nlist + z, 1u)] = c0 | (c << 12);
+			s_list[atomicAdd(&s_nlist + z, 1u)] = (uint16_t)c0;
 		}
 		s_val[q] = vv[j];
 		s_id[q] = ids[j];
@@ -833,7 +834,7 @@ __global__ __launch_bounds__(NT) void k_tile(TileArgs A, Ctl *ctl, Tables T,
 		const uint32_t nlist = s_nlist;
 #pragma unroll 1
 		for (uint32_t i = NT - 1 - tid; i < nlist; i += NT) {
-			const uint32_t en = s_list[i], p = en & 0xFFFu, c = en >> 12;
+			const uint32_t p = s_list[i], c = s_cell[p + 1];
 			uint32_t kk = s_start[c + 1] - p, cl;
 			if (D2) {
 				uint32_t x, r;
@@ -933,8 +934,8 @@ __global__ __launch_bounds__(NT) void k_tile(TileArgs A, Ctl *ctl, Tables T,
 		}
 	}
 	__syncthreads();
-	const uint32_t wt = s_wt[lane];
-	const uint32_t wi = wave_incl_scan32(wt);
+	const uint32_t wt = s_wt[NWT * lane], wt2 = NWT == 2 ? s_wt[2 * lane + 1] : 0u;
+	const uint32_t wi = wave_incl_scan32(wt + wt2);
 	const uint32_t nout = (uint32_t)__builtin_amdgcn_readlane((int)wi, WAVE - 1);
 	uint32_t o_at = tile * A.slot, o_max = nout;
 	if (nout > A.slot) {
@@ -959,7 +960,10 @@ __global__ __launch_bounds__(NT) void k_tile(TileArgs A, Ctl *ctl, Tables T,
 			__builtin_amdgcn_mbcnt_lo((uint32_t)bs,
 			__builtin_amdgcn_mbcnt_hi((uint32_t)(bc >> 32),
 			__builtin_amdgcn_mbcnt_lo((uint32_t)bc, 0u))));
-		o += (uint32_t)__builtin_amdgcn_readlane((int)(wi - wt), (int)(j * NW + w));
+		const uint32_t jw = j * NW + w;
+		o += (uint32_t)__builtin_amdgcn_readlane((int)(wi - wt - wt2), (int)(jw / NWT));
+		if (NWT == 2 && (jw & 1u))
+			o += (uint32_t)__builtin_amdgcn_readlane((int)wt, (int)(jw / 2));
 		if (!in) continue;
 		s_id[p] = o;   /* (the ids are no longer needed) */
 		uint32_t x, r;

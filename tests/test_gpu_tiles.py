@@ -130,3 +130,17 @@ def test_batch_of_tiles_admits_and_retires(tile, monkeypatch):
         assert np.array_equal(b.rows_array(rb)[1:], ref[:o.step_count])
         o.close()
     sys.stdout.flush()
+
+
+LARGEST = [
+    ("every cell of the shape", "2,0,128", v2s(128), 40),
+    ("one tile and a last tile of one row", "2,0,40", v2s(gx=150, gy=41), 40),
+    ("most slots in use", "2,0,60", DENSE, 30),
+    ("two-byte grass", "2,0,90", dict(v2s(90), grass_restart=300), 40),
+    ("as laid out", None, v2s(gx=2000, gy=520), 12),
+]
+
+
+@pytest.mark.parametrize("name,tile,d,iters", LARGEST, ids=[c[0] for c in LARGEST])
+def test_largest_shape_matches_oracle(name, tile, d, iters, monkeypatch):
+    test_tiles_match_oracle(name, tile, d, iters, monkeypatch)
