@@ -3347,6 +3347,13 @@ struct TilePlan {
  * replica's tiles of whole rows hold at least TILE_MIN cells. */
 constexpr uint32_t TILE_WIDE = 2048, TILE_MIN = 400;
 
+/* Tile ticks of a graph. Between two graphs the GPU waits for some 5 us, so
+ * that single launches are faster than graphs of 8 (100 x 100, 4000
+ * iterations: 27.7 and 28.8 ms; 16: 27.5, 32: 26.9, 64: 26.6); building a graph
+ * takes longer the longer it is (100 iterations of it, of which each pass builds
+ * its own: 0.88 ms with 8 and without, 0.83 with 32, 0.85 with 64). */
+constexpr uint32_t TILE_GRAPH = 32;
+
 /* Shapes of k_tile: threads, slots a thread, cells a tile. */
 struct TileShape {
 	uint32_t nt, ipt, cells;
@@ -3429,7 +3436,7 @@ struct pp_batch {
 
 	hipGraphExec_t graph_exec = nullptr;   /* 8 bucket-sort ticks */
 	hipGraphExec_t graph_radix = nullptr;  /* 8 radix-sort ticks */
-	hipGraphExec_t graph_tile = nullptr;   /* 8 tile ticks from parity 0 */
+	hipGraphExec_t graph_tile = nullptr;   /* TILE_GRAPH ticks from parity 0 */
 	int graph_steps = 0;
 
 	int profiling = 0;
@@ -3921,8 +3928,8 @@ static int to_pairs(pp_batch_t *b) {
 
 /* Enqueue `ticks` ticks. The tile step runs where the plan allows it, from
  * the state the staged step left (one staged tick after a change of the
- * replica table: new agents are in no cell order yet), in graphs of 8 ticks
- * and single launches. Otherwise the staged step: after a change of the
+ * replica table: new agents are in no cell order yet), in graphs and single
+ * launches. Otherwise the staged step: after a change of the
  * replica table the first tick sorts with the radix sort (the moved order is
  * not the cell order yet, or the bucket layout changed); then whole graphs of
  * 8, then single launches; the last tick's emit writes the SoA state that
@@ -3953,9 +3960,10 @@ static int enqueue_ticks(pp_batch_t *b, uint32_t ticks) {
 			PP_TRY(enqueue_tile(b));
 			i++;
 		}
-		if (use_graph && ticks - i >= 8) {
-			if (!b->graph_tile) PP_TRY(build_graph(b, 8, 2, &b->graph_tile));
-			for (; i + 8 <= ticks; i += 8)
+		if (use_graph && ticks - i >= TILE_GRAPH) {
+			if (!b->graph_tile)
+				PP_TRY(build_graph(b, TILE_GRAPH, 2, &b->graph_tile));
+			for (; i + TILE_GRAPH <= ticks; i += TILE_GRAPH)
 				HIP_OK(hipGraphLaunch(b->graph_tile, b->stream));
 		}
 		for (; i < ticks; i++) PP_TRY(enqueue_tile(b));
