@@ -1020,16 +1020,26 @@ __global__ __launch_bounds__(WG) void k_move_soa(const uint32_t *__restrict__ ce
  *   k_sort_scan  per digit, exclusive prefix over tiles and the digit total
  *   k_sort_down  per tile: rank in LDS, scatter to bucket start + tile prefix
  * Tile t covers positions [t * sort_tile, (t + 1) * sort_tile). The table
- * hist[d * hist_cols + t] holds tile counts, then tile offsets. */
+ * hist[t * radix + d] holds tile counts, then tile offsets: a tile's row is
+ * written and read whole (with a row a digit, every 4-byte count went to
+ * another line, which all XCDs wrote to). What bounds a pass: up to some
+ * million agents, where a CU holds one or two tiles, the chain of a tile's
+ * steps, hence groups of 512 threads with 8 keys each; beyond, memory (42 M
+ * agents: 20 bytes each in 0.24 ms). 2400 x 1200, 662 K agents, two passes of
+ * 11 bits, a pass: up 13.6 -> 4.8 us, scan 4.7 -> 4.5, down 21.5 -> 14.4. */
+
+constexpr uint32_t NXCD = 8;    /* accelerator dies (XCDs) of the GPU */
+constexpr int SORT_NT = 512;    /* threads of k_sort_up and k_sort_down */
+constexpr int SCAN_NT = 1024;   /* of k_sort_scan */
 
 __device__ __forceinline__ uint32_t pass_len(const Ctl *ctl, uint32_t pass) {
 	return pass == 0 ? ctl->n : ctl->live[ctl->tick & 1];
 }
 
 template <int KPT>
-__global__ __launch_bounds__(WG) void k_sort_up(const uint32_t *__restrict__ kin,
-	uint32_t *__restrict__ hist, Ctl *ctl, uint32_t pass, Params P) {
-	constexpr uint32_t TILE = WG * KPT;
+__global__ __launch_bounds__(SORT_NT) void k_sort_up(const uint32_t *__restrict__ kin,
+	uint32_t *__restrict__ hist, Ctl *ctl, uint32_t pass, uint32_t pairs, Params P) {
+	constexpr uint32_t TILE = SORT_NT * KPT;
 	__shared__ uint32_t s_hist[RADIX_MAX];
 	if (ctl->error) return;
 	/* the tick's first kernel: the last move's survivors into live, which
@@ -1042,36 +1052,43 @@ __global__ __launch_bounds__(WG) void k_sort_up(const uint32_t *__restrict__ kin
 	const uint32_t radix = 1u << P.digit_bits, dmask = radix - 1u;
 	const int tid = threadIdx.x, lane = tid & (WAVE - 1), w = tid / WAVE;
 	for (uint32_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-		for (uint32_t i = tid; i < radix; i += WG) s_hist[i] = 0;
-		__syncthreads();
 		const uint32_t base = tile * TILE + w * (WAVE * KPT);
+		uint32_t key[KPT];
 #pragma unroll
 		for (int j = 0; j < KPT; j++) {
 			const uint32_t idx = base + j * WAVE + lane;
-			const uint32_t k = idx < n ? kin[idx] : DEAD_KEY;
-			wave_hist_add(s_hist, k == DEAD_KEY ? NO_DIGIT : ((k >> shift) & dmask));
+			key[j] = idx < n ? kin[idx << (pairs & 1u)] : DEAD_KEY;
 		}
+		for (uint32_t i = tid; i < radix; i += SORT_NT) s_hist[i] = 0;
 		__syncthreads();
-		for (uint32_t d = tid; d < radix; d += WG)
-			hist[(size_t)d * P.hist_cols + tile] = s_hist[d];
+#pragma unroll
+		for (int j = 0; j < KPT; j++)
+			wave_hist_add(s_hist, key[j] == DEAD_KEY ? NO_DIGIT
+				: ((key[j] >> shift) & dmask));
+		__syncthreads();
+		uint32_t *row = hist + (size_t)tile * radix;
+		for (uint32_t d = tid; d < radix; d += SORT_NT) row[d] = s_hist[d];
 		__syncthreads();
 	}
 }
 
-/* One work-group per digit: hist[d][0..ntiles) -> exclusive prefix, and the
- * digit's total. Each thread sums a contiguous run of tiles. The pass-0 scan
- * also clears the action tiles' counters for this iteration and re-stamps
- * one grass slice. */
-template <typename GT>
-__global__ __launch_bounds__(WG) void k_sort_scan(uint32_t *__restrict__ hist,
+/* A work-group for DG digits: hist[0 .. ntiles)[d] -> exclusive prefix, and
+ * the digits' totals. The tiles are cut into SCAN_NT / DG runs, a thread for
+ * each and digit, so that a wave reads whole sectors of the table's rows. The
+ * pass-0 scan also clears the action tiles' counters for this iteration and
+ * re-stamps one grass slice. */
+template <typename GT, int DG>
+__global__ __launch_bounds__(SCAN_NT) void k_sort_scan(uint32_t *__restrict__ hist,
 	uint32_t *__restrict__ totals, const Ctl *ctl, uint32_t pass, Params P,
 	uint32_t *__restrict__ act_cnt, uint32_t act_words, GT *grass_at) {
-	__shared__ uint32_t s_tmp[NWAVE];
+	constexpr uint32_t RUNS = SCAN_NT / DG, RPL = RUNS / WAVE;
+	__shared__ uint32_t s_sum[RUNS * DG];
 	if (ctl->error) return;
+	const uint32_t tid = threadIdx.x, lane = tid & (WAVE - 1), w = tid / WAVE;
 	if (pass == 0) {
 		/* The action tiles' counters of this iteration start at zero. */
-		for (uint32_t i = blockIdx.x * WG + threadIdx.x; i < act_words;
-			i += gridDim.x * WG)
+		for (uint32_t i = blockIdx.x * SCAN_NT + tid; i < act_words;
+			i += gridDim.x * SCAN_NT)
 			act_cnt[i] = 0;
 		/* Re-stamp the alive cells of slice (t mod REFRESH) with t, which
 		 * keeps their stored regrow tick within the modular window; the
@@ -1081,8 +1098,8 @@ __global__ __launch_bounds__(WG) void k_sort_scan(uint32_t *__restrict__ hist,
 		const uint32_t per = (P.C + REFRESH - 1) / REFRESH;
 		const uint32_t c0 = (s % REFRESH) * per;
 		const uint32_t c1 = min(c0 + per, P.C);
-		for (uint32_t c = c0 + blockIdx.x * WG + threadIdx.x; c < c1;
-			c += gridDim.x * WG) {
+		for (uint32_t c = c0 + blockIdx.x * SCAN_NT + tid; c < c1;
+			c += gridDim.x * SCAN_NT) {
 			const GT g = grass_at[c];
 			if (grass_alive_at<GT>(g, s, P.R) && g != (GT)s) grass_at[c] = (GT)s;
 		}
@@ -1090,21 +1107,54 @@ __global__ __launch_bounds__(WG) void k_sort_scan(uint32_t *__restrict__ hist,
 	const uint32_t n = pass_len(ctl, pass);
 	const uint32_t ntiles = (n + P.sort_tile - 1) / P.sort_tile;
 	const uint32_t radix = 1u << P.digit_bits;
-	const uint32_t per = (ntiles + WG - 1) / WG;
-	const uint32_t t0 = threadIdx.x * per;
-	const uint32_t t1 = min(t0 + per, ntiles);
-	for (uint32_t d = blockIdx.x; d < radix; d += gridDim.x) {
-		uint32_t *col = hist + (size_t)d * P.hist_cols;
-		uint32_t sum = 0;
-		for (uint32_t t = t0; t < t1; t++) sum += col[t];
-		uint32_t total;
-		uint32_t run = wg_excl_scan<WG>(sum, s_tmp, total);
-		for (uint32_t t = t0; t < t1; t++) {
-			const uint32_t v = col[t];
-			col[t] = run;
-			run += v;
+	const uint32_t per = (ntiles + RUNS - 1) / RUNS;
+	/* (groups of neighbouring digits, which share sectors, on one XCD) */
+	const uint32_t dgs = (radix + DG - 1) / DG;
+	const uint32_t dg = blockIdx.x >= dgs || dgs % NXCD ? blockIdx.x
+		: (blockIdx.x % NXCD) * (dgs / NXCD) + blockIdx.x / NXCD;
+	const uint32_t d = dg * DG + tid % DG;
+	const uint32_t t0 = min(tid / DG * per, ntiles);
+	const uint32_t t1 = d < radix ? min(t0 + per, ntiles) : t0;
+	uint32_t *col = hist + d;
+	/* (CH rows requested at a time) */
+	constexpr uint32_t CH = 8;
+	uint32_t sum = 0;
+	for (uint32_t t = t0; t < t1; t += CH) {
+#pragma unroll
+		for (uint32_t i = 0; i < CH; i++)
+			sum += t + i < t1 ? col[(size_t)(t + i) * radix] : 0u;
+	}
+	s_sum[tid] = sum;
+	__syncthreads();
+	if (w < DG) {
+		/* the runs of digit w, RPL a lane */
+		uint32_t v[RPL], all = 0;
+#pragma unroll
+		for (uint32_t i = 0; i < RPL; i++) {
+			v[i] = s_sum[(lane * RPL + i) * DG + w];
+			all += v[i];
 		}
-		if (threadIdx.x == 0) totals[d] = total;
+		const uint32_t x = wave_incl_scan32(all);
+		uint32_t run = x - all;
+#pragma unroll
+		for (uint32_t i = 0; i < RPL; i++) {
+			s_sum[(lane * RPL + i) * DG + w] = run;
+			run += v[i];
+		}
+		if (lane == WAVE - 1 && dg * DG + w < radix) totals[dg * DG + w] = x;
+	}
+	__syncthreads();
+	uint32_t run = s_sum[tid];
+	for (uint32_t t = t0; t < t1; t += CH) {
+		uint32_t v[CH];
+#pragma unroll
+		for (uint32_t i = 0; i < CH; i++)
+			v[i] = t + i < t1 ? col[(size_t)(t + i) * radix] : 0u;
+#pragma unroll
+		for (uint32_t i = 0; i < CH; i++) {
+			if (t + i < t1) col[(size_t)(t + i) * radix] = run;
+			run += v[i];
+		}
 	}
 }
 
@@ -1114,135 +1164,151 @@ __global__ __launch_bounds__(WG) void k_sort_scan(uint32_t *__restrict__ hist,
  * ranking is stable), combine the waves, stage the tile in digit order in
  * LDS and write it to bucket start + tile prefix. */
 template <int KPT, int RBITS>
-__global__ __launch_bounds__(WG) void k_sort_down(
+__global__ __launch_bounds__(SORT_NT) void k_sort_down(
 	const uint32_t *__restrict__ kin, const uint32_t *__restrict__ vin,
 	uint32_t *__restrict__ kout, uint32_t *__restrict__ vout,
 	const uint32_t *__restrict__ hist, const uint32_t *__restrict__ totals,
-	Ctl *ctl, uint32_t pass, Params P) {
-	constexpr uint32_t TILE = WG * KPT;
+	Ctl *ctl, uint32_t pass, uint32_t pairs, Params P) {
+	constexpr uint32_t TILE = SORT_NT * KPT, NW = SORT_NT / WAVE;
 	constexpr uint32_t R = 1u << RBITS;
-	constexpr uint32_t DPT = R / WG < 1 ? 1 : R / WG;  /* digits per thread */
+	constexpr uint32_t DPT = R / SORT_NT < 1 ? 1 : R / SORT_NT;  /* digits per thread */
 	__shared__ uint32_t s_keys[TILE];
 	__shared__ uint32_t s_vals[TILE];
-	__shared__ uint32_t s_wh[NWAVE][R + 1];
-	__shared__ uint32_t s_bstart[R];
+	__shared__ __align__(16) uint16_t s_wh[NW][R];
+	static_assert(TILE < 65536, "16-bit counts and places");
 	__shared__ int32_t s_dst[R];
-	__shared__ uint32_t s_tstart[R];
-	__shared__ uint32_t s_tmp[NWAVE];
+	__shared__ uint32_t s_tmp[NW];
 
 	if (ctl->error) return;
 	const uint32_t n = pass_len(ctl, pass);
 	const uint32_t ntiles = (n + TILE - 1) / TILE;
-	const uint32_t shift = pass * P.digit_bits;
-	const uint32_t radix = 1u << P.digit_bits, dmask = radix - 1u;
+	const uint32_t shift = pass * P.digit_bits, bits = P.digit_bits;
+	const uint32_t radix = 1u << bits, dmask = radix - 1u;
 	const int tid = threadIdx.x, lane = tid & (WAVE - 1), w = tid / WAVE;
-	const uint64_t lt_mask = (1ull << lane) - 1ull;
 	bool bad = false;
 
 	/* Bucket starts: exclusive scan over digits of the digit totals. Thread
 	 * tid owns digits [tid*DPT, tid*DPT + DPT). */
+	uint32_t bstart[DPT];
 	{
-		uint32_t loc[DPT], sum = 0;
+		uint32_t sum = 0;
 #pragma unroll
 		for (uint32_t i = 0; i < DPT; i++) {
 			const uint32_t d = tid * DPT + i;
-			loc[i] = d < radix ? totals[d] : 0u;
-			sum += loc[i];
+			bstart[i] = d < radix ? totals[d] : 0u;
+			sum += bstart[i];
 		}
 		uint32_t tot;
-		uint32_t run = wg_excl_scan<WG>(sum, s_tmp, tot);
+		uint32_t run = wg_excl_scan<SORT_NT>(sum, s_tmp, tot);
 #pragma unroll
 		for (uint32_t i = 0; i < DPT; i++) {
-			const uint32_t d = tid * DPT + i;
-			if (d < R) s_bstart[d] = run;
-			run += loc[i];
+			const uint32_t t = bstart[i];
+			bstart[i] = run;
+			run += t;
 		}
 	}
 
 	for (uint32_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-		for (uint32_t i = tid; i < NWAVE * (R + 1); i += WG) (&s_wh[0][0])[i] = 0;
-		__syncthreads();
 		const uint32_t base = tile * TILE + w * (WAVE * KPT);
-		uint32_t key[KPT], val[KPT], dig[KPT], loc[KPT];
+		uint32_t key[KPT], val[KPT], loc[KPT], off[DPT];
 #pragma unroll
 		for (int j = 0; j < KPT; j++) {
 			const uint32_t idx = base + j * WAVE + lane;
-			uint32_t k = DEAD_KEY, v = 0;
+			key[j] = DEAD_KEY;
+			val[j] = 0;
 			if (idx < n) {
-				k = kin[idx];
-				v = vin[idx];
+				if (pairs & 1u) {
+					const uint2 q = reinterpret_cast<const uint2 *>(kin)[idx];
+					key[j] = q.x;
+					val[j] = q.y;
+				} else {
+					key[j] = kin[idx];
+					val[j] = vin[idx];
+				}
 			}
-			key[j] = k;
-			val[j] = v;
-			dig[j] = (k == DEAD_KEY) ? R : ((k >> shift) & dmask);
 		}
 #pragma unroll
-		for (int j = 0; j < KPT; j++) {
-			const uint32_t d = dig[j];
-			uint64_t peers = ~0ull;
+		for (uint32_t i = 0; i < DPT; i++) {
+			const uint32_t d = tid * DPT + i;
+			off[i] = d < radix ? hist[(size_t)tile * radix + d] : 0u;
+		}
+		for (uint32_t i = tid; i < NW * R / 8; i += SORT_NT)
+			reinterpret_cast<uint4 *>(&s_wh[0][0])[i] = make_uint4(0, 0, 0, 0);
+		__syncthreads();
 #pragma unroll
-			for (int b = 0; b <= RBITS; b++) {
-				const bool bit = (d >> b) & 1u;
-				const uint64_t bal = __ballot(bit);
-				peers &= bit ? bal : ~bal;
+		for (int j = 0; j < KPT; j++) {
+			const uint32_t d = (key[j] >> shift) & dmask;
+			const bool live = key[j] != DEAD_KEY;
+			const uint64_t alive = __ballot(live);
+			uint32_t lo = (uint32_t)alive, hi = (uint32_t)(alive >> 32);
+#pragma unroll
+			for (uint32_t b = 0; b < RBITS; b++) {
+				/* all ones where the lane's bit b is set */
+				const uint32_t m = (uint32_t)((int32_t)(d << (31 - b)) >> 31);
+				const uint64_t bal = __ballot(m != 0);
+				lo &= ~((uint32_t)bal ^ m);
+				hi &= ~((uint32_t)(bal >> 32) ^ m);
 			}
-			const uint32_t rank = __popcll(peers & lt_mask);
-			const uint32_t cnt = __popcll(peers);
+			const uint32_t rank = __builtin_amdgcn_mbcnt_hi(hi,
+				__builtin_amdgcn_mbcnt_lo(lo, 0u));
 			const uint32_t prev = s_wh[w][d];
-			if (rank == 0) s_wh[w][d] = prev + cnt;
+			if (live && rank == 0)
+				s_wh[w][d] = (uint16_t)(prev + (uint32_t)(__popc(lo) + __popc(hi)));
 			loc[j] = prev + rank;
 		}
 		__syncthreads();
 
-		/* Per digit: exclusive offsets of the waves, tile count; then the
-		 * tile-local start of each digit (exclusive scan over digits). */
-		uint32_t cnt_d[DPT], sum = 0;
+		/* Per digit: tile-local start (exclusive scan over digits), and from
+		 * it that of each wave's keys. */
+		uint32_t cnt[DPT], sum = 0;
 #pragma unroll
 		for (uint32_t i = 0; i < DPT; i++) {
 			const uint32_t d = tid * DPT + i;
-			uint32_t acc = 0;
+			cnt[i] = 0;
+			if (d < R)
 #pragma unroll
-			for (int ww = 0; ww < NWAVE; ww++) {
-				const uint32_t c = s_wh[ww][d];
-				s_wh[ww][d] = acc;
-				acc += c;
-			}
-			cnt_d[i] = acc;
-			sum += acc;
+				for (uint32_t ww = 0; ww < NW; ww++) cnt[i] += s_wh[ww][d];
+			sum += cnt[i];
 		}
 		uint32_t tile_live;
-		uint32_t run = wg_excl_scan<WG>(sum, s_tmp, tile_live);
+		uint32_t run = wg_excl_scan<SORT_NT>(sum, s_tmp, tile_live);
 #pragma unroll
 		for (uint32_t i = 0; i < DPT; i++) {
 			const uint32_t d = tid * DPT + i;
-			s_tstart[d] = run;
-			const uint32_t off = d < radix ? hist[(size_t)d * P.hist_cols + tile] : 0u;
-			s_dst[d] = (int32_t)(s_bstart[d] + off) - (int32_t)run;
-			run += cnt_d[i];
+			if (d >= R) continue;
+			s_dst[d] = (int32_t)(bstart[i] + off[i]) - (int32_t)run;
+			uint32_t at = run;
+#pragma unroll
+			for (uint32_t ww = 0; ww < NW; ww++) {
+				const uint32_t c = s_wh[ww][d];
+				s_wh[ww][d] = (uint16_t)at;
+				at += c;
+			}
+			run += cnt[i];
 		}
 		__syncthreads();
 #pragma unroll
 		for (int j = 0; j < KPT; j++) {
-			const uint32_t d = dig[j];
-			if (d < R) {
-				const uint32_t q = s_tstart[d] + s_wh[w][d] + loc[j];
-				s_keys[q] = key[j];
-				s_vals[q] = val[j];
-			}
+			if (key[j] == DEAD_KEY) continue;
+			const uint32_t q = s_wh[w][(key[j] >> shift) & dmask] + loc[j];
+			s_keys[q] = key[j];
+			s_vals[q] = val[j];
 		}
 		__syncthreads();
-		for (uint32_t q = tid; q < tile_live; q += WG) {
+		for (uint32_t q = tid; q < tile_live; q += SORT_NT) {
 			const uint32_t k = s_keys[q];
 			const uint32_t d = (k >> shift) & dmask;
 			const uint32_t dst = (uint32_t)(s_dst[d] + (int32_t)q);
 			/* dst < n whenever the histograms describe the input; the guard
 			 * turns an inconsistent table into an error, never a stray
 			 * write */
-			if (dst < n) {
+			if (dst >= n) {
+				bad = true;
+			} else if (pairs & 2u) {
+				reinterpret_cast<uint2 *>(kout)[dst] = make_uint2(k, s_vals[q]);
+			} else {
 				kout[dst] = k;
 				vout[dst] = s_vals[q];
-			} else {
-				bad = true;
 			}
 		}
 		__syncthreads();
@@ -1272,7 +1338,6 @@ __global__ __launch_bounds__(WG) void k_sort_down(
  * radix sort gives. */
 
 constexpr uint32_t BCAP = 1024;  /* agents of one bucket sorted in LDS */
-constexpr uint32_t NXCD = 8;     /* accelerator dies (XCDs) of the GPU */
 constexpr uint32_t W_MAX = 2048; /* cells of a bucket block: 2^S, S <= 11 */
 static_assert(W_MAX <= 2 * BCAP, "a dense bucket's counters reuse the staging");
 constexpr uint32_t BG_IPT = 6;   /* source positions per thread per round (1536: the three bucket rows of 12800^2) */
@@ -3541,18 +3606,34 @@ static int pass_dst(uint32_t p) { return 1 + (int)(p & 1); }
 
 template <typename GT>
 static void launch_sort_scan(pp_batch_t *b, uint32_t pass) {
-	k_sort_scan<GT><<<1u << b->P.digit_bits, WG, 0, b->stream>>>(b->hist,
-		b->totals, b->ctl, pass, b->P, b->act_cnt, b->act_words,
-		(GT *)b->grass_at);
+	const uint32_t radix = 1u << b->P.digit_bits;
+	/* (pass 0: enough groups for the grass slice, too) */
+	const uint32_t slice = pass ? 0u
+		: min_u32(2 * (uint32_t)b->num_cu, ceil_div(b->P.C, REFRESH * 4 * SCAN_NT));
+	if (b->rbits == 11)
+		k_sort_scan<GT, 16><<<std::max(ceil_div(radix, 16), slice), SCAN_NT, 0, b->stream>>>(b->hist,
+			b->totals, b->ctl, pass, b->P, b->act_cnt, b->act_words,
+			(GT *)b->grass_at);
+	else
+		k_sort_scan<GT, 4><<<std::max(ceil_div(radix, 4), slice), SCAN_NT, 0, b->stream>>>(b->hist,
+			b->totals, b->ctl, pass, b->P, b->act_cnt, b->act_words,
+			(GT *)b->grass_at);
 }
 
-template <int KPT, int RBITS>
+template <int TILE, int RBITS>
 static void launch_sort(pp_batch_t *b, uint32_t pass) {
+	constexpr int KPT = TILE / SORT_NT;
 	PendingEvent pe;
 	const int src = pass_src(pass), dst = pass_dst(pass);
+	/* 11-bit digits: pairs side by side between the passes, as a tile has but
+	 * two or three for each digit, which are then one write and not two (2400 x
+	 * 1200: k_sort_down 16.0 -> 14.4 us a pass); 8-bit digits have runs of 16
+	 * and more, and the histogram would read twice as much */
+	const uint32_t pairs = RBITS == 11
+		? (pass > 0 ? 1u : 0u) | (pass + 1 < b->P.passes ? 2u : 0u) : 0u;
 	prof_begin(b, KI_SORT_UP, pe);
-	k_sort_up<KPT><<<b->grid_up, WG, 0, b->stream>>>(b->keys[src], b->hist,
-		b->ctl, pass, b->P);
+	k_sort_up<KPT><<<b->grid_up, SORT_NT, 0, b->stream>>>(b->keys[src], b->hist,
+		b->ctl, pass, pairs, b->P);
 	prof_end(b, pe);
 	prof_begin(b, KI_SORT_SCAN, pe);
 	if (b->grass_bytes == 1) launch_sort_scan<uint8_t>(b, pass);
@@ -3560,19 +3641,19 @@ static void launch_sort(pp_batch_t *b, uint32_t pass) {
 	else launch_sort_scan<uint32_t>(b, pass);
 	prof_end(b, pe);
 	prof_begin(b, KI_SORT_DOWN, pe);
-	k_sort_down<KPT, RBITS><<<b->grid_down, WG, 0, b->stream>>>(b->keys[src],
+	k_sort_down<KPT, RBITS><<<b->grid_down, SORT_NT, 0, b->stream>>>(b->keys[src],
 		b->vals[src], b->keys[dst], b->vals[dst], b->hist, b->totals, b->ctl,
-		pass, b->P);
+		pass, pairs, b->P);
 	prof_end(b, pe);
 }
 
 static void launch_sort_pass(pp_batch_t *b, uint32_t pass) {
 	if (b->shape.kpt == 8) {
-		if (b->rbits == 11) launch_sort<8, 11>(b, pass);
-		else launch_sort<8, 8>(b, pass);
+		if (b->rbits == 11) launch_sort<8 * WG, 11>(b, pass);
+		else launch_sort<8 * WG, 8>(b, pass);
 	} else {
-		if (b->rbits == 11) launch_sort<16, 11>(b, pass);
-		else launch_sort<16, 8>(b, pass);
+		if (b->rbits == 11) launch_sort<16 * WG, 11>(b, pass);
+		else launch_sort<16 * WG, 8>(b, pass);
 	}
 }
 
@@ -3714,9 +3795,9 @@ static void apply_shape(pp_batch_t *b, const SortShape &sh) {
 	 * tiles of a full-capacity population; all loops are grid-strided. */
 	const uint32_t cu = (uint32_t)b->num_cu;
 	b->grid_up = min_u32(P.hist_cols, 8 * cu);
-	/* (8-bit digits: three groups a CU, as many as its LDS holds; 11-bit
-	 * digits: one) */
-	b->grid_down = min_u32(P.hist_cols, (b->rbits == 11 ? 1 : 3) * cu);
+	/* (8-bit digits: three groups a CU, 11-bit digits: two, as many as its
+	 * LDS holds) */
+	b->grid_down = min_u32(P.hist_cols, (b->rbits == 11 ? 2 : 3) * cu);
 	b->grid_emit = min_u32(ceil_div(P.cap, A_TILE), b->tile_rounds *
 		(b->wide ? resident(b, (const void *)k_emit_move<WIDE_WG>, WIDE_WG)
 			: resident(b, (const void *)k_emit_move<WG>)));
