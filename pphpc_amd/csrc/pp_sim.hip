@@ -3899,8 +3899,7 @@ static void launch_tile(pp_batch_t *b) {
 		k_tile<GT, 1024, 8, 16384, D2, SOLO><<<grid, 1024, 0, b->stream>>>(a, b->ctl,
 			b->tables(), b->P, b->table_nrep, g);
 	if (D2)
-		k_tile_scan<<<a.nbands, WG, 0, b->stream>>>(a, b->ctl, b->tables(),
-			b->table_nrep);
+		k_tile_scan<<<a.nbands, WG, 0, b->stream>>>(a, b->ctl, b->table_nrep);
 }
 
 template <typename GT>
@@ -3933,7 +3932,7 @@ static void launch_tiles_in(pp_batch_t *b) {
 	/* the ids of the rows, as after a tick whose output is parity 0 */
 	if (D2)
 		k_tile_scan<<<a.nbands, WG, 0, b->stream>>>(tile_args(b, 1), b->ctl,
-			b->tables(), b->table_nrep);
+			b->table_nrep);
 }
 
 template <typename GT, bool D2>
@@ -4212,8 +4211,12 @@ static void tile_layout(const pp_batch_t *b, const TileGrid *grid, uint32_t n,
 				(double)(sh.cells >> t.shift)), (double)TILE_ROWS);
 			if (!t.by) return;
 		}
-		if (eby) t.by = eby;
+		/* (set sizes: no larger than the shape's cells) */
+		if (eby)
+			t.by = p.d2 ? min_u32(min_u32(eby, TILE_ROWS), sh.cells >> t.shift)
+				: min_u32(eby, sh.cells / gx);
 		t.by = min_u32(t.by, gy);
+		if (!t.by) return;
 		t.nbx = ceil_div(gx, t.bx);
 		t.nby = ceil_div(gy, t.by);
 		t.tile0 = (uint32_t)tiles;
