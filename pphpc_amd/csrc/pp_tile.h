@@ -105,7 +105,7 @@ struct TileArgs {
 };
 
 constexpr uint32_t TILE_ROWS = 64;    /* rows of a tile, D2 */
-constexpr uint32_t TILE_ECAP = 64;    /* records of an edge list */
+constexpr uint32_t TILE_ECAP = 48;    /* records of an edge list */
 constexpr uint32_t TILE_RESTAMP = 32; /* ticks between re-stamps of the grass */
 
 /* The buffers (parity) that hold the current state: the parity whose tick
