@@ -1025,8 +1025,8 @@ __global__ __launch_bounds__(WG) void k_move_soa(const uint32_t *__restrict__ ce
  * another line, which all XCDs wrote to). What bounds a pass: up to some
  * million agents, where a CU holds one or two tiles, the chain of a tile's
  * steps, hence groups of 512 threads with 8 keys each; beyond, memory (42 M
- * agents: 20 bytes each in 0.24 ms). 2400 x 1200, 662 K agents, two passes of
- * 11 bits, a pass: up 13.6 -> 4.8 us, scan 4.7 -> 4.5, down 21.5 -> 14.4. */
+ * agents: 20 bytes each in 0.22 ms). 2400 x 1200, 662 K agents, two passes of
+ * 11 bits, a pass: up 13.6 -> 4.8 us, scan 4.7 -> 4.5, down 21.5 -> 13.4. */
 
 constexpr uint32_t NXCD = 8;    /* accelerator dies (XCDs) of the GPU */
 constexpr int SORT_NT = 512;    /* threads of k_sort_up and k_sort_down */
@@ -1034,6 +1034,13 @@ constexpr int SCAN_NT = 1024;   /* of k_sort_scan */
 
 __device__ __forceinline__ uint32_t pass_len(const Ctl *ctl, uint32_t pass) {
 	return pass == 0 ? ctl->n : ctl->live[ctl->tick & 1];
+}
+
+/* Tiles of an XCD, to whose groups (every NXCD-th) neighbouring tiles go: they
+ * write next to each other, and a line that two XCDs write to is written in
+ * parts (k_sort_down of 49 M agents 188 -> 157 us, of 662 K 14.4 -> 13.4). */
+__device__ __forceinline__ uint32_t xcd_share(uint32_t ntiles) {
+	return (ntiles + NXCD - 1) / NXCD;
 }
 
 template <int KPT>
@@ -1051,7 +1058,10 @@ __global__ __launch_bounds__(SORT_NT) void k_sort_up(const uint32_t *__restrict_
 	const uint32_t shift = pass * P.digit_bits;
 	const uint32_t radix = 1u << P.digit_bits, dmask = radix - 1u;
 	const int tid = threadIdx.x, lane = tid & (WAVE - 1), w = tid / WAVE;
-	for (uint32_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+	const uint32_t per = xcd_share(ntiles);
+	for (uint32_t q = blockIdx.x; q < per * NXCD; q += gridDim.x) {
+		const uint32_t tile = q % NXCD * per + q / NXCD;
+		if (tile >= ntiles) continue;
 		const uint32_t base = tile * TILE + w * (WAVE * KPT);
 		uint32_t key[KPT];
 #pragma unroll
@@ -1208,7 +1218,10 @@ __global__ __launch_bounds__(SORT_NT) void k_sort_down(
 		}
 	}
 
-	for (uint32_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+	const uint32_t per = xcd_share(ntiles);
+	for (uint32_t q = blockIdx.x; q < per * NXCD; q += gridDim.x) {
+		const uint32_t tile = q % NXCD * per + q / NXCD;
+		if (tile >= ntiles) continue;
 		const uint32_t base = tile * TILE + w * (WAVE * KPT);
 		uint32_t key[KPT], val[KPT], loc[KPT], off[DPT];
 #pragma unroll
@@ -3794,10 +3807,11 @@ static void apply_shape(pp_batch_t *b, const SortShape &sh) {
 	/* Enough groups to fill every CU several times, never more than the
 	 * tiles of a full-capacity population; all loops are grid-strided. */
 	const uint32_t cu = (uint32_t)b->num_cu;
-	b->grid_up = min_u32(P.hist_cols, 8 * cu);
+	const uint32_t sort_groups = ceil_div(P.hist_cols, NXCD) * NXCD;
+	b->grid_up = min_u32(sort_groups, 8 * cu);
 	/* (8-bit digits: three groups a CU, 11-bit digits: two, as many as its
 	 * LDS holds) */
-	b->grid_down = min_u32(P.hist_cols, (b->rbits == 11 ? 2 : 3) * cu);
+	b->grid_down = min_u32(sort_groups, (b->rbits == 11 ? 2 : 3) * cu);
 	b->grid_emit = min_u32(ceil_div(P.cap, A_TILE), b->tile_rounds *
 		(b->wide ? resident(b, (const void *)k_emit_move<WIDE_WG>, WIDE_WG)
 			: resident(b, (const void *)k_emit_move<WG>)));
