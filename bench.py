@@ -12,15 +12,18 @@ the K iterations of the agents alive at the start of each, divided by the
 wall time.
 
 Also reported (one JSON line on stdout, progress on stderr):
-  roofline      dominant kernel of a profiled run of the same workload:
-                algorithmic bytes per launch (exact, from the run's event
-                counters) / average launch duration (HIP events on the
-                simulation's stream), against 8 TB/s
-  roofline_12800  the same for the 12800x12800 run (HBM-resident working
-                set), every iteration sorted by the radix sort (the
-                bandwidth-bound path)
-  roofline_12800_auto  the same with the automatic sort (row buckets: fewer
-                bytes, latency-bound), and its time per iteration
+  roofline      the tile step of the same workload: the bytes it cannot do
+                without (8-byte records in and out, the grass in and out,
+                exact, from the run's event counters) / its unprofiled time
+                per iteration (one kernel and what lies between two), against
+                8 TB/s; `staged` holds the kernels of the staged step, which a
+                profiled run takes (HIP events on the simulation's stream),
+                with their bytes and rates
+  roofline_12800  the dominant kernel of the 12800x12800 run (HBM-resident
+                working set) with every iteration sorted by the radix sort
+                (the staged step): algorithmic bytes per launch / average
+                launch duration of a profiled run
+  roofline_12800_auto  the tile step there, as `roofline`
   cpu_baseline  the OpenMP restatement of the step (row bands, as the
                 reference's CPU simulator) on this host's cores, and the
                 single-threaded C oracle: the OpenMP one over the whole
@@ -206,7 +209,7 @@ def measure_roofline(params, capacity, steps, seed=0, sort_mode=None):
             "compulsory_GBps": round(bc / t, 1) if bc and t else None,
             "share": round(t / sum(v[1] for v in step_kernels.values()), 3)}
     achieved = total_bytes / ns  # bytes/ns == GB/s
-    return {
+    staged = {
         "kernel": dom,
         "bound": "hbm",
         "achieved": round(achieved, 1),
@@ -221,6 +224,23 @@ def measure_roofline(params, capacity, steps, seed=0, sort_mode=None):
         "sort": "radix" if radix_all else "row buckets",
         "per_kernel": per_kernel,
         "events_per_iteration": {k: round(v / steps, 1) for k, v in c.items()},
+    }
+    if radix_all:
+        return staged
+    # one grass byte a cell while a countdown fits (grass_restart <= 191)
+    grass = 2 * params["grid_xy"]
+    tile = (8 * (c["agent_steps"] + c["out"]) / steps + grass)
+    return {
+        "kernel": "tile",
+        "bound": "hbm",
+        "achieved": round(tile / ms_tick / 1e6, 1),
+        "peak": HBM_PEAK_GBS,
+        "unit": "GB/s",
+        "frac": round(tile / ms_tick / 1e6 / HBM_PEAK_GBS, 4),
+        "traffic": None,
+        "bytes_per_launch": int(tile),
+        "ms_per_iteration": round(ms_tick, 4),
+        "staged": staged,
     }
 
 

@@ -7,7 +7,7 @@
  *
  *   reference                                this implementation
  *   ---------------------------------------  -----------------------------------
- *   init_cell, init_agent (pp_gpu.cl:368)    k_init_cells, k_init_agents
+ *   init_cell, init_agent (pp_gpu.cl:368)    k_init
  *   grass (pp_gpu.cl:448)                    lazy regrow step per cell plus an
  *                                            O(1) ring update at the end of
  *                                            tick (k_act_scan, or the emit's
@@ -17,9 +17,9 @@
  *   cl_ops sbitonic sort (pp_gpu.c:826)      LSD radix sort of (cell, value)
  *                                            pairs: per pass k_sort_up (tile
  *                                            histograms), k_sort_scan (one
- *                                            work-group per digit), k_sort_down
- *                                            (LDS-staged wave64 ranking and
- *                                            scatter); stable, so the order is
+ *                                            work-group per 4 or 16 digits),
+ *                                            k_sort_down (LDS-staged wave64
+ *                                            ranking and scatter); stable, so the order is
  *                                            that of the key cell<<32 | id
  *   find_cell_idx (pp_gpu.cl:834)            segment heads found in k_act
  *   action_agent (pp_gpu.cl:883)             k_act: one lane per occupied cell,
@@ -30,8 +30,10 @@
  *   reduce_grass1/2, reduce_agent1/2         fused reductions (k_act, then
  *   (pp_gpu.cl:485-736)                      k_act_scan or end_tick_solo) with
  *                                            exact 64-bit sums
- *   stats readback every iteration           device rings of stats rows, one
- *   (pp_gpu.c:766, :840)                     copy per chunk of iterations
+ *   stats readback every iteration           device rings of stats rows; one
+ *   (pp_gpu.c:766, :840)                     kernel (k_publish) writes the new
+ *                                            ones to host memory per chunk of
+ *                                            iterations
  *
  * Replicas. A batch holds independent simulations (replicas, each with its
  * own grid, parameters, seed and iteration count) in one set of buffers:
@@ -1018,6 +1020,7 @@ __global__ __launch_bounds__(WG) void k_move_soa(const uint32_t *__restrict__ ce
  * drops dead agents (DEAD_KEY). A pass is three kernels:
  *   k_sort_up    digit histogram of every tile
  *   k_sort_scan  per digit, exclusive prefix over tiles and the digit total
+ *                (a group for some digits)
  *   k_sort_down  per tile: rank in LDS, scatter to bucket start + tile prefix
  * Tile t covers positions [t * sort_tile, (t + 1) * sort_tile). The table
  * hist[t * radix + d] holds tile counts, then tile offsets: a tile's row is
@@ -1356,14 +1359,15 @@ static_assert(W_MAX <= 2 * BCAP, "a dense bucket's counters reuse the staging");
 constexpr uint32_t BG_IPT = 6;   /* source positions per thread per round (1536: the three bucket rows of 12800^2) */
 static_assert(NWAVE == 4, "the gather reads the waves' counts as one uint4");
 /* The automatic choice (sort mode 1): one replica sorts by buckets at any
- * size (12800 x 12800: 89,600 buckets, 0.28 ms against 1.15 ms for four
+ * size (12800 x 12800: 89,600 buckets, 0.28 ms against 0.85 ms for four
  * radix passes); a batch of several sorts by buckets while it has at most
  * BUCKET_AUTO_MAX buckets, or at least BUCKET_AUTO_DENSITY agents a bucket
  * on average, else by the radix sort. Each bucket costs a few dependent
  * round trips to memory whatever it holds, so sparse buckets (many small
  * replicas, or sparse populations) favour the radix sort; dense ones do not
  * (30 replicas of 1600 x 1600, 48,000 buckets of about 390 agents: 2.48 s
- * against 3.47 s by radix for 4000 iterations). */
+ * against 3.47 s by radix for 4000 iterations, with the radix passes at 1.3
+ * times what they take now). */
 constexpr uint64_t BUCKET_AUTO_MAX = 16384;
 constexpr uint64_t BUCKET_AUTO_DENSITY = 64;
 

@@ -23,11 +23,11 @@
  * more than its four neighbours' border cells.
  *
  * What bounds it: on small grids the chain of one group's phases (two round
- * trips to memory, eight barriers, and fetching some 20 KB of instructions
+ * trips to memory, seven barriers, and fetching some 20 KB of instructions
  * that each wave runs through about once); on large ones the vector units.
- * Per iteration, against the three staged kernels: 100 x 100 24.5 -> 7.3 us,
- * 400 x 400 27.5 -> 9.6, 1600 x 1600 41 -> 18.4, 12800 x 12800 768 -> 561;
- * 30 replicas of 1600 x 1600 402 -> 242.
+ * Per iteration, against the three staged kernels: 100 x 100 24.5 -> 6.8 us,
+ * 400 x 400 27.5 -> 9.5, 1600 x 1600 41 -> 17.2, 12800 x 12800 768 -> 540;
+ * 30 replicas of 1600 x 1600 402 -> 240.
  *
  * A tile that outgrows its LDS or border lists sets Ctl::stop; the tick
  * after it is then not run (every group of a later launch returns), and the
