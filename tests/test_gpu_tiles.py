@@ -144,3 +144,13 @@ LARGEST = [
 @pytest.mark.parametrize("name,tile,d,iters", LARGEST, ids=[c[0] for c in LARGEST])
 def test_largest_shape_matches_oracle(name, tile, d, iters, monkeypatch):
     test_tiles_match_oracle(name, tile, d, iters, monkeypatch)
+
+
+@pytest.mark.parametrize("per_cell", [0.25, 0.34, 0.6])
+def test_cut_rows_by_density(per_cell, monkeypatch):
+    """Cut rows in the smaller and, from the density that fills it, the larger
+    shape, as laid out."""
+    d = v2s(gx=2100, gy=40)
+    n0 = int(per_cell * d["grid_x"] * d["grid_y"])
+    d.update(init_wolves=n0 // 10, init_sheep=n0 - n0 // 10)
+    test_tiles_match_oracle(f"density {per_cell}", None, d, 24, monkeypatch)
