@@ -4128,8 +4128,9 @@ static void tile_layout(const pp_batch_t *b, const TileGrid *grid, uint32_t n,
 		width = std::max(width, grid[i].rep->gx);
 		cells += grid[i].rep->C;
 	}
-	/* (by little: a stop costs about a millisecond, tiles of fewer rows than
-	 * need be every iteration: 30 x 1600 x 1600 from iteration 400 on, 311 us
+	/* (by little: a stop costs a few milliseconds at most, as what is enqueued
+	 * of the run returns at once, tiles of fewer rows than need be every
+	 * iteration: 30 x 1600 x 1600 from iteration 400 on, 311 us
 	 * with the 4 rows that 1.1 gives, 369 with 3) */
 	for (uint32_t i = 0; i < b->tile_dense; i++) dens *= 1.1;
 	p.d2 = width > TILE_WIDE;
@@ -4139,18 +4140,21 @@ static void tile_layout(const pp_batch_t *b, const TileGrid *grid, uint32_t n,
 	if (ecfg == -1 || ecfg > 2) return;
 	if (ebx) p.d2 = true;
 	/* rows of a tile (at most) in shape c: its cells, and most of the agents
-	 * it may hold (with rows filled further, or border rows of less than 1.25
+	 * it may hold. With rows filled further, or border rows of less than 1.25
 	 * times the mean and 64, tiles would outgrow their limits by chance and
-	 * stop the run; 0.9 gives cut rows tiles of 16 rows, all of their cells:
-	 * 4001 x 2999 45.3 -> 43.2 us, 15 rows with 0.87; 0.75 for one replica's
-	 * few tiles, whose largest ends each iteration) */
+	 * stop the run (1600 x 1600 with 1.15: 1000 iterations 17.2 -> 19.4 ms).
+	 * Whole rows of several replicas, whose tiles are full, leave the tile what
+	 * 1.15 does not take (48 replicas of mixed sizes, from iteration 400 on,
+	 * 115 -> 104 us a tick). 0.9 gives cut rows tiles of 16 rows, all of their
+	 * cells: 4001 x 2999 45.3 -> 43.2 us, 15 rows with 0.87; 0.75 is for one
+	 * replica's few tiles, whose largest ends each iteration. */
 	const double fill = p.d2 ? 0.9 : n > 1 ? 0.87 : 0.75;
 	const uint32_t bx = min_u32(ebx ? ebx : 256, width);   /* of cut rows */
 	auto limits = [&](int c) {
 		const uint32_t ag = tile_shapes[c].nt * tile_shapes[c].ipt;
 		p.cfg = c;
 		p.hmax = std::min<uint32_t>(ag / 3,
-			(uint32_t)(1.25 * dens * (p.d2 ? bx : width)) + 64);
+			(uint32_t)((p.d2 ? 1.25 * bx : n > 1 ? 1.15 * width : 1.25 * width) * dens) + 64);
 		p.nmax = ag - 2 * p.hmax - (p.d2 ? 2 * TILE_ECAP : 0);
 	};
 	auto rows_max = [&](uint32_t w) {
