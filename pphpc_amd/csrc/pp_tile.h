@@ -141,9 +141,11 @@ __device__ __forceinline__ void stat_sums(const TileStat *units, uint32_t n,
 /* End of tick t for the k-th replica of the table, by one work-group: sums
  * the units' statistics (tiles, or bands of tiles), then does what
  * end_tick_solo and k_act_scan do. Nothing happens when the replica has
- * ended that tick already. */
+ * ended that tick already. Where the outputs of all replicas are more than
+ * the capacity, the batch fails: the tick does not count, no replica ends it,
+ * and thread 0 returns true. */
 template <int NT>
-__device__ void tile_finish(const TileStat *units, uint32_t nunits, uint32_t k,
+__device__ bool tile_finish(const TileStat *units, uint32_t nunits, uint32_t k,
 	uint32_t t, unsigned long long *tot, Ctl *ctl, const Tables &T,
 	const Params &P, uint32_t nrep) {
 	__shared__ unsigned long long s_f[NT / WAVE][8];
@@ -152,9 +154,10 @@ __device__ void tile_finish(const TileStat *units, uint32_t nunits, uint32_t k,
 	RepCtl &rc = T.rctl[slot];
 	const Rep &rp = T.rep[slot];
 	const uint32_t s = t - rp.t0;
-	const bool due = rc.status == RS_ACTIVE && rc.step == s && !ctl->error;
+	const bool failed = ctl->error != 0;
+	const bool due = rc.status == RS_ACTIVE && rc.step == s && !failed;
 	stat_sums<NT>(units, due ? nunits : 0u, s_f);
-	if (w != 0) return;
+	if (w != 0) return false;
 	/* the outputs of all replicas, which the agent buffers bound */
 	unsigned long long total = 0;
 	if (nrep > 1) total = wave_sum(tot[(t % 3) * PART_SLOTS + lane]);
@@ -164,16 +167,17 @@ __device__ void tile_finish(const TileStat *units, uint32_t nunits, uint32_t k,
 		for (int q = 0; q < NT / WAVE; q++) sum += s_f[q][lane];
 #pragma unroll
 	for (int i = 0; i < 8; i++) a[i] = __shfl(sum, i);
-	if (lane != 0) return;
-	/* (the tick counts on when every replica is done) */
-	if (k == 0 && (int32_t)(t + 1 - ctl->tick) > 0) ctl->tick = t + 1;
-	if (!due) return;
+	if (lane != 0) return false;
 	const unsigned long long out64 = a[0] + a[1];
 	if (nrep == 1) total = out64;
-	if (total > P.cap) {
-		if (k == 0) ctl->tick = t;
+	const bool beyond = total > P.cap;
+	/* (the tick counts on when every replica is done) */
+	if (k == 0 && !failed && !beyond && (int32_t)(t + 1 - ctl->tick) > 0)
+		ctl->tick = t + 1;
+	if (!due) return beyond;
+	if (beyond) {
 		set_error(ctl, PP_OUT_OF_RESOURCES, t, -1);
-		return;
+		return true;
 	}
 	const uint32_t out = (uint32_t)out64;
 	atomicAdd(&ctl->sum_live, a[5]);
@@ -184,7 +188,7 @@ __device__ void tile_finish(const TileStat *units, uint32_t nunits, uint32_t k,
 		rc.error = over ? PP_ENERGY_OVERFLOW : PP_OUT_OF_RESOURCES;
 		rc.err_step = s;
 		rc.n = 0;
-		return;
+		return false;
 	}
 	const uint32_t M = rp.R + 1;
 	unsigned long long D = rc.dead_cells, S = rc.cd_sum;
@@ -217,6 +221,7 @@ __device__ void tile_finish(const TileStat *units, uint32_t nunits, uint32_t k,
 		rc.status = RS_DONE;
 		rc.n = 0;
 	}
+	return false;
 }
 
 /* One cell of k agents (2 <= k <= N <= 8) at LDS slots p .. p + k - 1, in
@@ -502,23 +507,21 @@ __global__ __launch_bounds__(NT) void k_tile(TileArgs A, Ctl *ctl, Tables T,
 	if (blockIdx.x < A.nfin) {
 		const uint32_t k = blockIdx.x, tick = ctl_word(12 + A.par);
 		const bool runs = tile_runs(ctl_word(4), ctl_word(14), ctl_word(15), tick);
-		if (k == 0) {
-			if (tid == 0) {
-				if (runs) {
-					ctl->tt[1 - A.par] = tick + 1;
-					A.spare[A.par] = 0;   /* for the next tick's outputs */
-				} else {
-					ctl->halt = 1;
-				}
-			}
-			if (!SOLO && tid < PART_SLOTS)
-				A.tot[((tick + 1) % 3) * PART_SLOTS + tid] = 0;
-		}
 		const TileRep tr = SOLO ? A.one : tile_rep(A.trep, k);
-		if (D2) tile_finish<NT>(A.bstat + tr.band0, tr.nby, k, tick - 1, A.tot, ctl, T,
-				P, nrep);
-		else tile_finish<NT>(A.sin + tr.tile0, tr.ntiles, k, tick - 1, A.tot, ctl, T, P,
+		const bool beyond = D2
+			? tile_finish<NT>(A.bstat + tr.band0, tr.nby, k, tick - 1, A.tot, ctl, T, P, nrep)
+			: tile_finish<NT>(A.sin + tr.tile0, tr.ntiles, k, tick - 1, A.tot, ctl, T, P,
 				nrep);
+		if (k != 0) return;
+		if (tid == 0) {
+			if (!runs) {
+				ctl->halt = 1;
+			} else if (!beyond) {
+				ctl->tt[1 - A.par] = tick + 1;
+				A.spare[A.par] = 0;   /* for the next tick's outputs */
+			}
+		}
+		if (!SOLO && tid < PART_SLOTS) A.tot[((tick + 1) % 3) * PART_SLOTS + tid] = 0;
 		return;
 	}
 	/* groups of one XCD take neighbouring tiles (their borders are then read
@@ -600,8 +603,15 @@ __global__ __launch_bounds__(NT) void k_tile(TileArgs A, Ctl *ctl, Tables T,
 	 * that before or after the end of the last tick, written beside this:
 	 * both give the same answer. (One thread decides for the group: an energy
 	 * limit or an error may be noted meanwhile.) */
+	/* Nor does any replica when the outputs of the last tick are more than the
+	 * capacity (the first groups then fail the batch): the records which that
+	 * tick started from stay, as its outputs may not all have been written.
+	 * (One replica: total_in, below.) */
+	bool fits = true;
+	if (!SOLO && w == 0)
+		fits = wave_sum32((uint32_t)A.tot[((tick + 2) % 3) * PART_SLOTS + lane]) <= P.cap;
 	const bool go = tile_runs(ctl_word(4), ctl_word(14), ctl_word(15), tick) &
-		(status == RS_ACTIVE) & (step < tr.iters) &
+		fits & (status == RS_ACTIVE) & (step < tr.iters) &
 		((over == 0) | (over == tick + 1));
 	if (tid == 0) {
 		s_nlist = 0;
