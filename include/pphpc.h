@@ -155,7 +155,10 @@ int pp_sim_counters(const pp_sim_t *s, uint64_t out[6]);
 /* State dump, the counterpart of PPG_DUMP (pp_gpu.c:438-555): agents in slot
  * order (cell = y * grid_x + x, energy, type) and the grass countdown of every
  * cell. Each pointer may be NULL; arrays hold pp_sim_num_agents() agents and
- * grid_xy cells. */
+ * grid_xy cells. After an iteration that failed for want of capacity this is
+ * the state before it, in which the grass that it ate reads as alive (under a
+ * sort mode of its own or profiling, where no kernel writes the state within a
+ * run, only when that iteration was its run's first). */
 int pp_sim_get_state(pp_sim_t *s, uint32_t *cell, int32_t *energy,
 	uint8_t *type, uint32_t *grass);
 

@@ -229,7 +229,8 @@ struct Ctl {
 	uint32_t stop, halt;
 	uint32_t in_tick;  /* tick at which the records were written from the SoA
 	                    * state */
-	uint32_t pad;
+	uint32_t records;  /* the record buffers hold a state (they do not where an
+	                    * error kept k_tiles_in from writing them) */
 	/* sums over completed ticks of: agents at the start, alive after the
 	 * move, after actions, occupied cells, grass eaten, births */
 	unsigned long long agent_steps, sum_live, sum_out, sum_occ, sum_eaten,
@@ -3917,7 +3918,7 @@ static void launch_tile(pp_batch_t *b) {
 		k_tile<GT, 1024, 8, 16384, D2, SOLO><<<grid, 1024, 0, b->stream>>>(a, b->ctl,
 			b->tables(), b->P, b->table_nrep, g);
 	if (D2)
-		k_tile_scan<<<a.nbands, WG, 0, b->stream>>>(a, b->ctl, b->table_nrep);
+		k_tile_scan<<<a.nbands, WG, 0, b->stream>>>(a, b->ctl, b->table_nrep, 0u);
 }
 
 template <typename GT>
@@ -3950,12 +3951,18 @@ static void launch_tiles_in(pp_batch_t *b) {
 	/* the ids of the rows, as after a tick whose output is parity 0 */
 	if (D2)
 		k_tile_scan<<<a.nbands, WG, 0, b->stream>>>(tile_args(b, 1), b->ctl,
-			b->table_nrep);
+			b->table_nrep, 0u);
 }
 
 template <typename GT, bool D2>
 static void launch_tiles_out(pp_batch_t *b) {
 	const TileArgs a = tile_args(b, 0);
+	if (D2 && b->ctl_host->error) {
+		/* the ids are those of the failed tick's outputs */
+		const TileArgs c = tile_args(b, 1u - tile_cur(b->ctl_host));
+		k_tile_bands<<<c.nbands, WG, 0, b->stream>>>(c, b->ctl, b->table_nrep);
+		k_tile_scan<<<c.nbands, WG, 0, b->stream>>>(c, b->ctl, b->table_nrep, 1u);
+	}
 	k_tile_base<<<1, WAVE, 0, b->stream>>>(b->ctl, b->tables(), b->table_nrep);
 	k_tiles_out<GT, D2><<<a.ntiles, WG, 0, b->stream>>>(a, b->ctl, b->tables(),
 		b->P, b->table_nrep, (GT *)b->grass_at, b->cell, b->energy, b->type);
@@ -3982,7 +3989,8 @@ static int tiles_in(pp_batch_t *b) {
 	return PP_SUCCESS;
 }
 
-/* Tiles -> SoA state (the tiles stay valid). */
+/* Tiles -> SoA state (the tiles stay valid). Also after an error, which every
+ * run has read back: the state is that before the failed iteration. */
 static int tiles_out(pp_batch_t *b) {
 	if (b->form != FORM_TILES || b->soa_fresh) return PP_SUCCESS;
 	{
@@ -4337,8 +4345,17 @@ static void table_plan(pp_batch_t *b) {
  * another plan (returned in *again). */
 static int tile_settle(pp_batch_t *b, int *again) {
 	*again = 0;
-	if (b->form != FORM_TILES || b->ctl_host->error) return PP_SUCCESS;
 	const Ctl *c = b->ctl_host;
+	if (b->form != FORM_TILES) return PP_SUCCESS;
+	if (c->error) {
+		/* (a staged iteration failed, and the tiles were not written: the SoA
+		 * state is the last) */
+		if (!c->records) {
+			b->form = FORM_SOA;
+			b->soa_fresh = 1;
+		}
+		return PP_SUCCESS;
+	}
 	b->tile_par = (int32_t)(c->tt[1] - c->tt[0]) > 0 ? 1u : 0u;
 	if (!c->stop) return PP_SUCCESS;
 	/* (records that did not fit in the first place are not complete: the SoA

@@ -108,10 +108,16 @@ constexpr uint32_t TILE_ROWS = 64;    /* rows of a tile, D2 */
 constexpr uint32_t TILE_ECAP = 48;    /* records of an edge list */
 constexpr uint32_t TILE_RESTAMP = 32; /* ticks between re-stamps of the grass */
 
-/* The buffers (parity) that hold the current state: the parity whose tick
- * is the later. */
-__device__ __forceinline__ uint32_t tile_cur(const Ctl *ctl) {
+/* The buffers (parity) that the last tick wrote: those whose tick is the
+ * later. */
+__device__ __forceinline__ uint32_t tile_last(const Ctl *ctl) {
 	return (int32_t)(ctl->tt[1] - ctl->tt[0]) > 0 ? 1u : 0u;
+}
+
+/* The buffers that hold the state of Ctl::tick: those it wrote, or, when its
+ * agents were more than the capacity, those it started from. */
+__host__ __device__ __forceinline__ uint32_t tile_cur(const Ctl *ctl) {
+	return ctl->tt[1] == ctl->tick ? 1u : 0u;
 }
 
 /* Whether tick t may run: no error, and not at or past a stop. A stop set
@@ -1059,15 +1065,18 @@ __global__ __launch_bounds__(NT) void k_tile(TileArgs A, Ctl *ctl, Tables T,
  * statistics, and the replica's agents (last band). A chain of memory round
  * trips: what can be requested together is, and a thread takes four tile rows
  * in turn (12800 x 12800: 11.4 -> 9.6 us, 4001 x 2999 5.5 -> 5.0, with its
- * iteration 46.6 -> 45.3). */
+ * iteration 46.6 -> 45.3). again: for a state whose ids the scan after a
+ * failed tick has replaced, its bands' sums by k_tile_bands. */
 __global__ __launch_bounds__(WG) void k_tile_scan(TileArgs A, Ctl *ctl,
-	uint32_t nrep) {
+	uint32_t nrep, uint32_t again) {
 	const bool SOLO = nrep == 1;
 	constexpr uint32_t EPT = 4;
 	__shared__ uint32_t s_tmp[NWAVE];
 	__shared__ unsigned long long s_f[NWAVE][8];
 	/* only after a tick that ran */
-	if (ctl->error || ctl->halt || ctl->tt[1 - A.par] != ctl->tt[A.par] + 1) return;
+	if (!again && (ctl->error || ctl->halt || ctl->tt[1 - A.par] != ctl->tt[A.par] + 1))
+		return;
+	if (again && !ctl->records) return;
 	const uint32_t band = blockIdx.x, tid = threadIdx.x;
 	const uint32_t k = nrep == 1 ? 0u : A.bk[band];
 	const TileRep tr = SOLO ? A.one : tile_rep(A.trep, k);
@@ -1115,6 +1124,20 @@ __global__ __launch_bounds__(WG) void k_tile_scan(TileArgs A, Ctl *ctl,
 	}
 }
 
+/* The agents of each band, of the tiles in A.hout. */
+__global__ __launch_bounds__(WG) void k_tile_bands(TileArgs A, const Ctl *ctl,
+	uint32_t nrep) {
+	__shared__ uint32_t s_tmp[NWAVE];
+	if (!ctl->records) return;
+	const uint32_t band = blockIdx.x, tid = threadIdx.x;
+	const TileRep tr = nrep == 1 ? A.one : tile_rep(A.trep, A.bk[band]);
+	const uint32_t t0 = tr.tile0 + (band - tr.band0) * tr.nbx;
+	uint32_t sum = 0, tot;
+	for (uint32_t i = tid; i < tr.nbx; i += WG) sum += A.hout[t0 + i].x;
+	(void)wg_excl_scan<WG>(sum, s_tmp, tot);
+	if (tid == 0) A.bsum[(1 - A.par) * A.nbands + band] = tot;
+}
+
 /* The end of the last tick run, one work-group per replica of the table. A
  * holds the buffers by parity: in/hin/sin parity 0, out/hout/sout parity 1. */
 template <bool D2>
@@ -1122,7 +1145,7 @@ __global__ __launch_bounds__(WG) void k_tile_end(TileArgs A, Ctl *ctl, Tables T,
 	Params P, uint32_t nrep) {
 	const bool SOLO = nrep == 1;
 	if (ctl->error) return;
-	const uint32_t cur = tile_cur(ctl), tick = ctl->tt[cur], k = blockIdx.x;
+	const uint32_t cur = tile_last(ctl), tick = ctl->tt[cur], k = blockIdx.x;
 	const TileRep tr = SOLO ? A.one : tile_rep(A.trep, k);
 	const TileStat *st = cur ? A.sout : A.sin;
 	tile_finish<WG>(D2 ? A.bstat + tr.band0 : st + tr.tile0,
@@ -1135,6 +1158,7 @@ __global__ __launch_bounds__(WAVE) void k_tile_base(Ctl *ctl, Tables T,
 	uint32_t nrep) {
 	const uint32_t lane = threadIdx.x;
 	uint32_t carry = 0;
+	if (!ctl->records) return;
 	for (uint32_t k0 = 0; k0 < nrep; k0 += WAVE) {
 		const uint32_t k = k0 + lane;
 		uint32_t n = 0, slot = 0;
@@ -1149,10 +1173,11 @@ __global__ __launch_bounds__(WAVE) void k_tile_base(Ctl *ctl, Tables T,
 	if (lane == 0) ctl->n = carry;
 }
 
-/* Before k_tiles_in: no stop, and the bands' sums (both parities) at zero. */
+/* Before k_tiles_in: no records, no stop, and the bands' sums (both parities)
+ * at zero. */
 __global__ __launch_bounds__(WG) void k_tile_clear(TileArgs A, Ctl *ctl) {
 	const uint32_t i = blockIdx.x * WG + threadIdx.x;
-	if (i == 0) ctl->stop = ctl->halt = 0;
+	if (i == 0) ctl->stop = ctl->halt = ctl->records = 0;
 	if (i < 2) A.spare[i] = 0;
 	if (i < 2 * A.nbands) A.bsum[i] = 0;
 }
@@ -1218,6 +1243,7 @@ __global__ __launch_bounds__(WG) void k_tiles_in(TileArgs A, Ctl *ctl, Tables T,
 			ctl->tt[0] = tick;
 			ctl->tt[1] = tick - 1;
 			ctl->in_tick = tick;
+			ctl->records = 1;
 		}
 		if (tid < PART_SLOTS)
 			for (uint32_t i = 0; i < 3; i++) A.tot[i * PART_SLOTS + tid] = 0;
@@ -1327,9 +1353,9 @@ __global__ __launch_bounds__(WG) void k_tiles_in(TileArgs A, Ctl *ctl, Tables T,
 	}
 }
 
-/* The tiles' records (current parity) to the SoA state, at the replicas'
- * batch positions (k_tile_base), and their grass re-stamped. A holds the
- * buffers by parity, as for k_tile_end. */
+/* The tiles' records (of Ctl::tick, also after an iteration that failed the
+ * batch) to the SoA state, at the replicas' batch positions (k_tile_base), and
+ * their grass re-stamped. A holds the buffers by parity, as for k_tile_end. */
 template <typename GT, bool D2>
 __global__ __launch_bounds__(WG) void k_tiles_out(TileArgs A, Ctl *ctl, Tables T,
 	Params P, uint32_t nrep, GT *grass, uint32_t *cell, int32_t *energy,
@@ -1337,7 +1363,8 @@ __global__ __launch_bounds__(WG) void k_tiles_out(TileArgs A, Ctl *ctl, Tables T
 	const bool SOLO = nrep == 1;
 	__shared__ uint32_t s_tmp[NWAVE];
 	const uint32_t tid = threadIdx.x, tile = blockIdx.x;
-	const uint32_t cur = tile_cur(ctl), tick = ctl->tt[cur];
+	if (!ctl->records) return;
+	const uint32_t cur = tile_cur(ctl), tick = ctl->tick;
 	const uint32_t k = nrep == 1 ? 0u : A.tk[tile];
 	const uint32_t slot = T.order[k];
 	const Rep &rp = T.rep[slot];

@@ -1,10 +1,11 @@
 """What is left after an iteration whose agents are more than the capacity:
 the run ends with PP_OUT_OF_RESOURCES at that iteration, which does not count,
-with the tiles laid out and forced (PPHPC_TILE=shape,columns,rows)."""
+and the state that can be read is the one before it, with the tiles laid out
+and forced (PPHPC_TILE=shape,columns,rows)."""
 import numpy as np
 import pytest
 
-from helpers import gpu_params, v2ref, v2s
+from helpers import assert_state_equal, gpu_params, v2ref, v2s
 
 pytestmark = pytest.mark.gpu
 
@@ -31,6 +32,16 @@ def _states(d, seed, upto):
         rows.append(o.stats())
     o.close()
     return states, np.array(rows, np.uint64)
+
+
+def _left(d, states, t):
+    """The state that iteration t leaves when it fails: the one before it, in
+    which the grass that it ate reads as alive (it is eaten in place; a cell
+    so marked may have had a countdown of 1)."""
+    cell, energy, typ, grass = states[t]
+    ate = states[t + 1][3] == d["grass_restart"]
+    assert (grass[ate] <= 1).all()
+    return cell, energy, typ, np.where(ate, 0, grass).astype(np.uint32)
 
 
 def _failing_batch():
@@ -70,3 +81,50 @@ def test_a_failed_iteration_does_not_count(tile, pieces, monkeypatch):
         for rid, (_, rows) in zip(ids, ref):
             assert b.replica(rid)["steps"] == FAILS
             assert np.array_equal(b.rows_array(rid), rows[:FAILS + 1])
+
+
+@pytest.mark.parametrize("pieces", [[1] * 20, [60]], ids=["stepped", "one run"])
+@pytest.mark.parametrize("fails", [0, 2, 9])
+@pytest.mark.parametrize("tile", TILES, ids=TILE_IDS)
+def test_state_before_the_failed_iteration(tile, fails, pieces, monkeypatch):
+    """fails 0: the staged iteration before the first of tiles; 2: a tile that
+    is given no spare records in the iteration that fails. Changing the sort
+    brings the agents into other forms; init starts anew."""
+    from pphpc_amd import Simulation
+    if tile:
+        monkeypatch.setenv("PPHPC_TILE", tile)
+    print(f"[case] state after failure: {tile} {fails} {pieces[:2]}", flush=True)
+    states, rows = _states(GROWS, 1, fails + 1)
+    cap = len(states[fails][0])
+    assert len(states[fails + 1][0]) > cap
+    left = _left(GROWS, states, fails)
+    with Simulation(gpu_params(GROWS), seed=1, capacity=cap, device=0) as sim:
+        for _ in range(2):
+            sim.init()
+            _run_to_failure(sim.run, pieces)
+            assert sim.step_count == fails
+            assert_state_equal(sim.state(), left, "failed")
+            for mode in (0, 1):
+                sim.set_sort(mode)
+                assert_state_equal(sim.state(), left, f"sort {mode}")
+                _run_to_failure(sim.run, [2])
+            assert_state_equal(sim.state(), left, "run again")
+        sim.init()
+        assert np.array_equal(sim.run_array(fails), rows[1:fails + 1])
+        assert_state_equal(sim.state(), states[fails], "up to the failure")
+
+
+@pytest.mark.parametrize("pieces", [[1] * 20, [60]], ids=["stepped", "one run"])
+@pytest.mark.parametrize("tile", TILES, ids=TILE_IDS)
+def test_states_of_a_failed_batch(tile, pieces, monkeypatch):
+    if tile:
+        monkeypatch.setenv("PPHPC_TILE", tile)
+    print(f"[case] states of a failed batch: {tile} {pieces[:2]}", flush=True)
+    b, ids, ref = _failing_batch()
+    with b:
+        _run_to_failure(b.run, pieces)
+        for _ in range(2):
+            for rid, d, (states, _) in zip(ids, (GROWS, STAYS), ref):
+                assert_state_equal(b.state(rid), _left(d, states, FAILS),
+                                   f"replica {rid}")
+            b.set_sort(0)
