@@ -1007,7 +1007,8 @@ __global__ __launch_bounds__(NT) void k_tile(TileArgs A, Ctl *ctl, Tables T,
 		if (!(v & V_KILLED)) put(y);
 		if (v & V_CHILD) put(y - ((v & V_ODD) ? 1u : 0u));
 	}
-	/* the grass back; alive cells are re-stamped now and then (see REFRESH) */
+	/* the grass back; alive cells are re-stamped now and then (see REFRESH),
+	 * with this tick, so that they are alive in it also where it fails */
 	const bool restamp = tick % TILE_RESTAMP == 0;
 #pragma unroll 1
 	for (uint32_t i = tid; i < CHUNKS; i += NT) {
@@ -1017,7 +1018,8 @@ __global__ __launch_bounds__(NT) void k_tile(TileArgs A, Ctl *ctl, Tables T,
 			GT *q = s_g + i * TG::VPC;
 #pragma unroll 1
 			for (uint32_t u = 0; u < TG::VPC; u++)
-				if (grass_alive_at<GT>(q[u], tick + 1, P.R)) q[u] = (GT)(tick + 1);
+				if (grass_alive_at<GT>(q[u], tick + 1, P.R) && q[u] != (GT)(tick + 1))
+					q[u] = (GT)tick;
 		}
 		if (cells >= TG::VPC) {
 			const uint4 v = s_grass[i];

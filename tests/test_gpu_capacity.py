@@ -128,3 +128,23 @@ def test_states_of_a_failed_batch(tile, pieces, monkeypatch):
                 assert_state_equal(b.state(rid), _left(d, states, FAILS),
                                    f"replica {rid}")
             b.set_sort(0)
+
+
+@pytest.mark.parametrize("tile", [None, "0,16,8"], ids=["as laid out", "cut rows"])
+def test_grass_when_the_failed_iteration_renews_its_ticks(tile, monkeypatch):
+    """The tiles store the tick anew in live cells at every 32nd iteration:
+    also of these the state before stays readable."""
+    from pphpc_amd import Simulation
+    if tile:
+        monkeypatch.setenv("PPHPC_TILE", tile)
+    print(f"[case] renewed grass: {tile}", flush=True)
+    d = v2ref(60, iters=100)
+    for fails in (31, 32, 33, 64):
+        states, _ = _states(d, 17, fails + 1)
+        cap = len(states[fails][0])
+        assert max(len(s[0]) for s in states[:-1]) == cap < len(states[-1][0])
+        with Simulation(gpu_params(d), seed=17, capacity=cap, device=0) as sim:
+            sim.init()
+            _run_to_failure(sim.run, [90])
+            assert sim.step_count == fails
+            assert_state_equal(sim.state(), _left(d, states, fails), f"{fails}")
