@@ -354,7 +354,8 @@ int pp_batch_get_launch(const pp_batch_t *b, uint32_t *tile_rounds,
  * pp_batch_set_sort / pp_batch_set_shape. Then, under a sort of its own, each
  * launch shape (tile_rounds 1, 2, 4, 8; bucket_eighths 4, 8) is timed and
  * the fastest kept (pp_batch_get_launch reports it). A trial during which
- * replicas finish is timed again. */
+ * replicas finish, or tiles outgrow their limits and are laid out anew, is
+ * timed again. */
 int pp_batch_tune(pp_batch_t *b, uint32_t trial_ticks, uint32_t *bucket_shift,
 	uint32_t *keys_per_thread, uint32_t *max_digit_bits, double *sec_per_tick);
 

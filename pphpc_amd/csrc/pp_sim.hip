@@ -4653,15 +4653,29 @@ static uint32_t active_count(const pp_batch_t *b) {
 	return n;
 }
 
+static double now_s() {
+	struct timespec ts;
+	clock_gettime(CLOCK_MONOTONIC, &ts);
+	return (double)ts.tv_sec + 1e-9 * (double)ts.tv_nsec;
+}
+
 /* Runs `ticks` ticks and collects; where the tiles stop short (tile_settle),
- * the rest with the new plan. The control words must be fresh. */
-static int run_ticks(pp_batch_t *b, uint32_t ticks) {
+ * the rest with the new plan. The control words must be fresh. sec: the time
+ * until the last of the ticks has run, with new plans, without the last
+ * collection. */
+static int run_ticks(pp_batch_t *b, uint32_t ticks, double *sec = nullptr) {
 	const uint32_t target = b->ctl_host->tick + ticks;
+	if (sec) HIP_OK(hipStreamSynchronize(b->stream));
+	const double start = sec ? now_s() : 0.0;
 	while (b->ctl_host->tick != target) {
 		const uint32_t t0 = b->ctl_host->tick;
 		PP_TRY(flush_admitted(b));
 		const uint32_t dense0 = b->tile_dense;
 		PP_TRY(enqueue_ticks(b, target - t0));
+		if (sec) {
+			HIP_OK(hipStreamSynchronize(b->stream));
+			*sec = now_s() - start;
+		}
 		PP_TRY(collect(b));
 		if (b->ctl_host->error) break;
 		/* (a plan can stop at its first tick; the next one is finer) */
@@ -5096,22 +5110,6 @@ static int prof_export(pp_batch_t *b, const char *path) {
 			total > 0 ? b->prof_ns[i] / total : 0.0);
 	fclose(fp);
 	return PP_SUCCESS;
-}
-
-static double now_s() {
-	struct timespec ts;
-	clock_gettime(CLOCK_MONOTONIC, &ts);
-	return (double)ts.tv_sec + 1e-9 * (double)ts.tv_nsec;
-}
-
-/* Times `ticks` ticks of the current shape (graph replay, then collect). */
-static int time_ticks(pp_batch_t *b, uint32_t ticks, double *sec) {
-	HIP_OK(hipStreamSynchronize(b->stream));
-	const double t0 = now_s();
-	PP_TRY(enqueue_ticks(b, ticks));
-	HIP_OK(hipStreamSynchronize(b->stream));
-	*sec = now_s() - t0;
-	return collect(b);
 }
 
 /* ------------------------------------------------ allocation-free runs */
@@ -5778,18 +5776,19 @@ int pp_batch_tune(pp_batch_t *b, uint32_t trial_ticks, uint32_t *bucket_shift,
 		double best_t = -1.0;
 		/* One trial of the current shapes: 8 untimed ticks re-sort if
 		 * needed, build the graph, warm caches; a trial during which
-		 * replicas finished (the table changed) is settled and timed once
-		 * more. */
+		 * replicas finished (the table changed) or tiles outgrew their
+		 * limits is settled and timed once more. */
 		auto trial = [&](double &t) -> int {
 			for (int attempt = 0; attempt < 2; attempt++) {
-				PP_TRY(flush_admitted(b));
-				PP_TRY(enqueue_ticks(b, 8));
-				PP_TRY(collect(b));
+				PP_TRY(run_ticks(b, 8));
 				PP_TRY(flush_admitted(b));
 				const uint64_t v0 = b->table_version;
-				PP_TRY(time_ticks(b, trial_ticks, &t));
+				const uint32_t stops0 = b->tile_dense;
+				PP_TRY(run_ticks(b, trial_ticks, &t));
 				PP_TRY(flush_admitted(b));
-				if (b->table_version == v0 || active_count(b) == 0) break;
+				if ((b->table_version == v0 && b->tile_dense == stops0) ||
+					active_count(b) == 0)
+					break;
 			}
 			return PP_SUCCESS;
 		};
