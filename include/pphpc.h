@@ -212,6 +212,9 @@ int pp_sim_prof_export(pp_sim_t *s, const char *path);
 int pp_sim_info(const pp_sim_t *s, uint32_t *sort_passes, uint32_t *sort_tile,
 	uint32_t *action_tile, uint32_t *grid_move);
 
+/* The tile step's layout, as pp_batch_tiles. */
+int pp_sim_tiles(const pp_sim_t *s, uint32_t out[6]);
+
 /* Sort of the agents by cell, as pp_batch_set_sort. */
 int pp_sim_set_sort(pp_sim_t *s, uint32_t mode);
 
@@ -318,6 +321,13 @@ int pp_batch_counters(const pp_batch_t *b, uint64_t out[6]);
 /* Sort passes, sort tile, action tile and emit grid in use. */
 int pp_batch_info(const pp_batch_t *b, uint32_t *sort_passes,
 	uint32_t *sort_tile, uint32_t *action_tile, uint32_t *grid_move);
+
+/* The tile step as it is laid out: [0] 1 when the agents are in the tiles'
+ * records (the last iteration was the tile step's), [1] threads of a tile's
+ * group, [2] 1 when grid rows are cut into several tiles, [3] tiles, [4]
+ * records of a tile's slot, [5] stops since the replicas last changed (tiles
+ * that outgrew their limits). [1] to [4] are 0 where the staged step runs. */
+int pp_batch_tiles(const pp_batch_t *b, uint32_t out[6]);
 
 /* Sort of the agents by cell: mode 0 = the radix sort every iteration;
  * 8..11 = from the second iteration after a change of the replicas, row

@@ -5544,6 +5544,10 @@ int pp_sim_info(const pp_sim_t *s, uint32_t *sort_passes, uint32_t *sort_tile,
 	return pp_batch_info(s->b, sort_passes, sort_tile, action_tile, grid_move);
 }
 
+int pp_sim_tiles(const pp_sim_t *s, uint32_t out[6]) {
+	return s ? pp_batch_tiles(s->b, out) : PP_INVALID_ARGS;
+}
+
 int pp_sim_set_sort(pp_sim_t *s, uint32_t bucket_shift) {
 	return guarded([&]() -> int {
 		if (!s) return PP_INVALID_ARGS;
@@ -5699,6 +5703,18 @@ int pp_batch_info(const pp_batch_t *b, uint32_t *sort_passes,
 	if (sort_tile) *sort_tile = b->P.sort_tile;
 	if (action_tile) *action_tile = A_TILE;
 	if (grid_move) *grid_move = b->grid_emit;
+	return PP_SUCCESS;
+}
+
+int pp_batch_tiles(const pp_batch_t *b, uint32_t out[6]) {
+	if (!b || !out) return PP_INVALID_ARGS;
+	const TilePlan &p = b->plan;
+	out[0] = b->form == FORM_TILES;
+	out[1] = p.on ? tile_shapes[p.cfg].nt : 0;
+	out[2] = p.on && p.d2;
+	out[3] = p.on ? p.ntiles : 0;
+	out[4] = p.on ? p.slot : 0;
+	out[5] = b->tile_dense;
 	return PP_SUCCESS;
 }
 

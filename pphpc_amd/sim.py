@@ -27,6 +27,11 @@ PP_ENERGY_OVERFLOW = -9   # no counterpart in the reference: energy limit
 # cells eaten, births.
 COUNTER_FIELDS = ("agent_steps", "live", "out", "occupied", "eaten", "births")
 
+# pp_sim_tiles / pp_batch_tiles: the agents are in the tiles' records, threads
+# of a tile's group, rows cut into several tiles, tiles, records of a tile's
+# slot, stops since the replicas last changed.
+TILE_FIELDS = ("in_use", "threads", "cut", "tiles", "slot", "stops")
+
 # Field order of PPParameters (opencl/pp/pp_common.in.h:129-157) and the keys
 # of the parameter file that fill them (pp_common.c:55-167).
 PARAM_FIELDS = (
@@ -128,6 +133,7 @@ def _lib():
         "pp_sim_prof_reset": (i32, [vp]),
         "pp_sim_prof_export": (i32, [vp, ctypes.c_char_p]),
         "pp_sim_info": (i32, [vp, P(u32), P(u32), P(u32), P(u32)]),
+        "pp_sim_tiles": (i32, [vp, P(u32)]),
         "pp_sim_destroy": (None, [vp]),
         "pp_sim_sync": (i32, [vp]),
         "pp_sim_set_sort": (i32, [vp, u32]),
@@ -149,6 +155,7 @@ def _lib():
         "pp_batch_tick": (u32, [vp]),
         "pp_batch_counters": (i32, [vp, P(u64)]),
         "pp_batch_info": (i32, [vp, P(u32), P(u32), P(u32), P(u32)]),
+        "pp_batch_tiles": (i32, [vp, P(u32)]),
         "pp_batch_set_shape": (i32, [vp, u32, u32]),
         "pp_batch_tune": (i32, [vp, u32, P(u32), P(u32), P(u32),
                                 P(ctypes.c_double)]),
@@ -337,6 +344,12 @@ class Simulation:
                                        ctypes.byref(d)), "info")
         return {"sort_passes": a.value, "sort_tile": b.value,
                 "action_tile": c.value, "grid_move": d.value}
+
+    def tiles(self) -> dict:
+        """The tile step's layout (TILE_FIELDS)."""
+        out = (ctypes.c_uint32 * 6)()
+        self._check(_lib().pp_sim_tiles(self._h, out), "tiles")
+        return dict(zip(TILE_FIELDS, tuple(out)))
 
     def state(self):
         """(cell u32[n], energy i32[n], type u8[n], grass u32[C])."""
@@ -532,6 +545,12 @@ class Batch:
                                          ctypes.byref(d)), "info")
         return {"sort_passes": a.value, "sort_tile": b.value,
                 "action_tile": c.value, "grid_move": d.value}
+
+    def tiles(self) -> dict:
+        """The tile step's layout (TILE_FIELDS)."""
+        out = (ctypes.c_uint32 * 6)()
+        self._check(_lib().pp_batch_tiles(self._h, out), "tiles")
+        return dict(zip(TILE_FIELDS, tuple(out)))
 
     def set_shape(self, keys_per_thread: int, max_digit_bits: int):
         self._check(_lib().pp_batch_set_shape(self._h, keys_per_thread,
