@@ -4974,20 +4974,14 @@ static int admit(pp_batch_t *b, const pp_params_t *p, uint64_t seed,
 	if (p->grass_restart > b->P.R || C > b->P.C) return PP_INVALID_ARGS;
 	if (reserve == 0) reserve = std::max<uint64_t>(4ull * n0, 1);
 	if (reserve < n0 || reserve > b->P.cap) return PP_INVALID_ARGS;
-	if (b->admitted.empty()) {
-		/* its agents will be appended to the batch's pairs */
-		PP_TRY(to_pairs(b));
-		if (!b->ctl_fresh) PP_TRY(read_ctl(b));
-		b->next_pos = b->ctl_host->n;
-	}
+	if (b->admitted.empty() && !b->ctl_fresh) PP_TRY(read_ctl(b));
 	if (b->ctl_host->error) return b->ctl_host->error;
-	const uint32_t tick = b->ctl_host->tick, pos = b->next_pos;
+	const uint32_t tick = b->ctl_host->tick;
 	/* (a plain simulation runs without a limit; pp_sim_run checks its runs) */
 	if (iters != ITERS_UNLIMITED &&
 		(uint64_t)tick + iters + b->P.R + 1 >= 0xFFFFFFFFull)
 		return PP_INVALID_ARGS;
-	if (b->reserved + reserve > b->P.cap || (uint64_t)pos + n0 > b->P.cap)
-		return PP_OUT_OF_RESOURCES;
+	if (b->reserved + reserve > b->P.cap) return PP_OUT_OF_RESOURCES;
 	int slot = -1;
 	for (uint32_t s = 0; s < b->max_rep; s++)
 		if (b->slot_rid[s] < 0) {
@@ -4997,6 +4991,21 @@ static int admit(pp_batch_t *b, const pp_params_t *p, uint64_t seed,
 	if (slot < 0) return PP_OUT_OF_RESOURCES;
 	const int64_t cb = take_cells(b, C);
 	if (cb < 0) return PP_OUT_OF_RESOURCES;
+	/* Its agents will be appended to the batch's pairs. (Only now: a caller
+	 * may ask again and again for room that there is not, while the others
+	 * run in their tiles.) */
+	int rc = PP_SUCCESS;
+	if (b->admitted.empty()) {
+		rc = to_pairs(b);
+		if (!rc && !b->ctl_fresh) rc = read_ctl(b);
+		b->next_pos = b->ctl_host->n;
+	}
+	const uint32_t pos = b->next_pos;
+	if (!rc && (uint64_t)pos + n0 > b->P.cap) rc = PP_OUT_OF_RESOURCES;
+	if (rc) {
+		release_cells(b, (uint32_t)cb, C);
+		return rc;
+	}
 
 	Rep rp{};
 	rp.cb = (uint32_t)cb;

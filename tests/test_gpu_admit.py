@@ -1,0 +1,35 @@
+"""Admissions while replicas hold their agents in tiles."""
+import numpy as np
+import pytest
+
+from helpers import gpu_params, v1, v2s
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("short", ["agents", "cells", "slots"])
+def test_a_refused_admission_leaves_the_tiles(short):
+    """A batch without room for another replica stays in its tiles, and its
+    replicas' rows are the oracle's."""
+    from oracle.pp_oracle import simulate
+    from pphpc_amd import Batch
+    print(f"[case] refused admission: {short}", flush=True)
+    ds = [(v2s(64, iters=60), 1), (v1(gx=50, gy=70, iters=50), 2)]
+    room = [3 * d["grid_xy"] for d, _ in ds]
+    cells = sum(d["grid_xy"] for d, _ in ds)
+    more = v2s(32, iters=40)
+    want = 3 * more["grid_xy"]
+    with Batch(sum(room) + (want - 1 if short == "agents" else want),
+               cells + (more["grid_xy"] - 1 if short == "cells" else 4096),
+               2 if short == "slots" else 3, 15, device=0) as b:
+        ids = [b.add(gpu_params(d), s, r) for (d, s), r in zip(ds, room)]
+        for n in (7, 1, 12, 25, 60):
+            b.run(n)
+            if b.replica(ids[0])["state"] == b.replica(ids[1])["state"] == 1:
+                assert b.add(gpu_params(more), 9, want) is None
+                assert b.tiles()["in_use"] == 1
+        for rid, (d, s), r in zip(ids, ds, room):
+            assert np.array_equal(b.rows_array(rid), simulate(d, seed=s, capacity=r))
+        rid = b.add(gpu_params(more), 9, want)
+        b.run(40)
+        assert np.array_equal(b.rows_array(rid), simulate(more, seed=9, capacity=want))
