@@ -33,3 +33,29 @@ def test_a_refused_admission_leaves_the_tiles(short):
         rid = b.add(gpu_params(more), 9, want)
         b.run(40)
         assert np.array_equal(b.rows_array(rid), simulate(more, seed=9, capacity=want))
+
+
+@pytest.mark.parametrize("sort", [1, 0])
+def test_running_replicas_are_moved_by_one_launch(sort):
+    """Twelve replicas of different sides in tiles, of which some end, then
+    one more: one launch moves all agents for the iteration that sorts them."""
+    from oracle.pp_oracle import simulate
+    from pphpc_amd import Batch
+    print(f"[case] one launch moves all: sort {sort}", flush=True)
+    ds = [(v2s(gx=7 + 9 * i, gy=90 - 7 * i, iters=30 + 5 * (i % 4)), i) for i in range(12)]
+    late = (v1(40, iters=30), 77)
+    room = [3 * d["grid_xy"] + 8 for d, _ in ds + [late]]
+    cells = sum(d["grid_xy"] for d, _ in ds + [late])
+    with Batch(sum(room), cells, 13, 15, device=0) as b:
+        ids = [b.add(gpu_params(d), s, r) for (d, s), r in zip(ds, room)]
+        b.run(37)
+        assert {b.replica(i)["state"] for i in ids} == {1, 2}
+        assert b.tiles()["in_use"] == 1
+        b.set_profiling(True)
+        ids.append(b.add(gpu_params(late[0]), late[1], room[-1]))
+        assert b.profile()["move0"][0] == 1
+        b.set_profiling(False)
+        b.set_sort(sort)
+        b.run(40)
+        for rid, (d, s), r in zip(ids, ds + [late], room):
+            assert np.array_equal(b.rows_array(rid), simulate(d, seed=s, capacity=r)), s
