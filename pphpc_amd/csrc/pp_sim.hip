@@ -5241,8 +5241,8 @@ static int simulate_noalloc(const pp_params_t *p, uint64_t seed,
 	b->rctl_host = &g_na_rctl[dev];
 
 	/* The scratch keeps the last call's contents: clear what must start at
-	 * zero (control block, partial sums, histograms, the replica's control
-	 * words, the bucket counts). */
+	 * zero (control block, partial sums, the bucket counts; the replica's
+	 * control words with its initial state, below). */
 	const hipStream_t st = b->stream;
 	k_batch_reset<<<1, WG, 0, st>>>(b->ctl, b->P.part);
 	HIP_OK(hipGetLastError());
@@ -5286,14 +5286,13 @@ static int simulate_noalloc(const pp_params_t *p, uint64_t seed,
 	b->P.cnt_top = top;
 	b->P.one_slot = 0;
 	b->P.solo = 1;
-	const uint32_t zero = 0, one = 1, nb32 = on ? (uint32_t)nbk : 0u;
+	const uint32_t zero = 0, counts[2] = {1, on ? (uint32_t)nbk : 0u};
 	const uint32_t bbase[2] = {0, (uint32_t)nbk};
 	HIP_OK(hipMemcpy(b->rep_dev, &rp, sizeof(Rep), hipMemcpyHostToDevice));
 	HIP_OK(hipMemcpy(b->cbs_dev, &zero, 4, hipMemcpyHostToDevice));
 	HIP_OK(hipMemcpy(b->order_dev, &zero, 4, hipMemcpyHostToDevice));
 	HIP_OK(hipMemcpy(b->bbase_dev, bbase, 8, hipMemcpyHostToDevice));
-	HIP_OK(hipMemcpy(&b->ctl->nrep, &one, 4, hipMemcpyHostToDevice));
-	HIP_OK(hipMemcpy(&b->ctl->nbuckets, &nb32, 4, hipMemcpyHostToDevice));
+	HIP_OK(hipMemcpy(&b->ctl->nrep, counts, 8, hipMemcpyHostToDevice));
 	b->need_radix = 1;
 	b->table_nrep = 1;
 	const TileGrid tg{&rp, 0, n0};
