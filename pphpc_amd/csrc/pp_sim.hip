@@ -3924,7 +3924,7 @@ static void launch_tile(pp_batch_t *b) {
 		k_tile<GT, 1024, 8, 16384, D2, SOLO><<<grid, 1024, 0, b->stream>>>(a, b->ctl,
 			b->tables(), b->P, b->table_nrep, g);
 	if (D2)
-		k_tile_scan<<<a.nbands, WG, 0, b->stream>>>(a, b->ctl, b->table_nrep, 0u);
+		k_tile_scan<<<a.nbands, WG, 0, b->stream>>>(a, b->ctl, b->P, b->table_nrep, 0u);
 }
 
 template <typename GT>
@@ -3957,7 +3957,7 @@ static void launch_tiles_in(pp_batch_t *b) {
 	/* the ids of the rows, as after a tick whose output is parity 0 */
 	if (D2)
 		k_tile_scan<<<a.nbands, WG, 0, b->stream>>>(tile_args(b, 1), b->ctl,
-			b->table_nrep, 0u);
+			b->P, b->table_nrep, 0u);
 }
 
 template <typename GT, bool D2>
@@ -3967,7 +3967,7 @@ static void launch_tiles_out(pp_batch_t *b) {
 		/* the ids are those of the failed tick's outputs */
 		const TileArgs c = tile_args(b, 1u - tile_cur(b->ctl_host));
 		k_tile_bands<<<c.nbands, WG, 0, b->stream>>>(c, b->ctl, b->table_nrep);
-		k_tile_scan<<<c.nbands, WG, 0, b->stream>>>(c, b->ctl, b->table_nrep, 1u);
+		k_tile_scan<<<c.nbands, WG, 0, b->stream>>>(c, b->ctl, b->P, b->table_nrep, 1u);
 	}
 	k_tile_base<<<1, WAVE, 0, b->stream>>>(b->ctl, b->tables(), b->table_nrep);
 	k_tiles_out<GT, D2><<<a.ntiles, WG, 0, b->stream>>>(a, b->ctl, b->tables(),

@@ -114,10 +114,11 @@ __device__ __forceinline__ uint32_t tile_last(const Ctl *ctl) {
 	return (int32_t)(ctl->tt[1] - ctl->tt[0]) > 0 ? 1u : 0u;
 }
 
-/* The buffers that hold the state of Ctl::tick: those it wrote, or, when its
- * agents were more than the capacity, those it started from. */
+/* The buffers that hold the state of Ctl::tick: those written last, or, when
+ * the tick that wrote them failed the batch, those it started from (of which
+ * the launch behind it may have counted on two ticks already). */
 __host__ __device__ __forceinline__ uint32_t tile_cur(const Ctl *ctl) {
-	return ctl->tt[1] == ctl->tick ? 1u : 0u;
+	return (ctl->tt[1] ^ ctl->tick) & 1u ? 0u : 1u;
 }
 
 /* Whether tick t may run: no error, and not at or past a stop. A stop set
@@ -148,10 +149,10 @@ __device__ __forceinline__ void stat_sums(const TileStat *units, uint32_t n,
  * the units' statistics (tiles, or bands of tiles), then does what
  * end_tick_solo and k_act_scan do. Nothing happens when the replica has
  * ended that tick already. Where the outputs of all replicas are more than
- * the capacity, the batch fails: the tick does not count, no replica ends it,
- * and thread 0 returns true. */
+ * the capacity, the batch fails: the tick does not count, and no replica ends
+ * it. */
 template <int NT>
-__device__ bool tile_finish(const TileStat *units, uint32_t nunits, uint32_t k,
+__device__ void tile_finish(const TileStat *units, uint32_t nunits, uint32_t k,
 	uint32_t t, unsigned long long *tot, Ctl *ctl, const Tables &T,
 	const Params &P, uint32_t nrep) {
 	__shared__ unsigned long long s_f[NT / WAVE][8];
@@ -163,7 +164,7 @@ __device__ bool tile_finish(const TileStat *units, uint32_t nunits, uint32_t k,
 	const bool failed = ctl->error != 0;
 	const bool due = rc.status == RS_ACTIVE && rc.step == s && !failed;
 	stat_sums<NT>(units, due ? nunits : 0u, s_f);
-	if (w != 0) return false;
+	if (w != 0) return;
 	/* the outputs of all replicas, which the agent buffers bound */
 	unsigned long long total = 0;
 	if (nrep > 1) total = wave_sum(tot[(t % 3) * PART_SLOTS + lane]);
@@ -173,17 +174,17 @@ __device__ bool tile_finish(const TileStat *units, uint32_t nunits, uint32_t k,
 		for (int q = 0; q < NT / WAVE; q++) sum += s_f[q][lane];
 #pragma unroll
 	for (int i = 0; i < 8; i++) a[i] = __shfl(sum, i);
-	if (lane != 0) return false;
+	if (lane != 0) return;
 	const unsigned long long out64 = a[0] + a[1];
 	if (nrep == 1) total = out64;
 	const bool beyond = total > P.cap;
 	/* (the tick counts on when every replica is done) */
 	if (k == 0 && !failed && !beyond && (int32_t)(t + 1 - ctl->tick) > 0)
 		ctl->tick = t + 1;
-	if (!due) return beyond;
+	if (!due) return;
 	if (beyond) {
 		set_error(ctl, PP_OUT_OF_RESOURCES, t, -1);
-		return true;
+		return;
 	}
 	const uint32_t out = (uint32_t)out64;
 	atomicAdd(&ctl->sum_live, a[5]);
@@ -194,7 +195,7 @@ __device__ bool tile_finish(const TileStat *units, uint32_t nunits, uint32_t k,
 		rc.error = over ? PP_ENERGY_OVERFLOW : PP_OUT_OF_RESOURCES;
 		rc.err_step = s;
 		rc.n = 0;
-		return false;
+		return;
 	}
 	const uint32_t M = rp.R + 1;
 	unsigned long long D = rc.dead_cells, S = rc.cd_sum;
@@ -227,7 +228,6 @@ __device__ bool tile_finish(const TileStat *units, uint32_t nunits, uint32_t k,
 		rc.status = RS_DONE;
 		rc.n = 0;
 	}
-	return false;
 }
 
 /* One cell of k agents (2 <= k <= N <= 8) at LDS slots p .. p + k - 1, in
@@ -513,21 +513,23 @@ __global__ __launch_bounds__(NT) void k_tile(TileArgs A, Ctl *ctl, Tables T,
 	if (blockIdx.x < A.nfin) {
 		const uint32_t k = blockIdx.x, tick = ctl_word(12 + A.par);
 		const bool runs = tile_runs(ctl_word(4), ctl_word(14), ctl_word(15), tick);
-		const TileRep tr = SOLO ? A.one : tile_rep(A.trep, k);
-		const bool beyond = D2
-			? tile_finish<NT>(A.bstat + tr.band0, tr.nby, k, tick - 1, A.tot, ctl, T, P, nrep)
-			: tile_finish<NT>(A.sin + tr.tile0, tr.ntiles, k, tick - 1, A.tot, ctl, T, P,
-				nrep);
-		if (k != 0) return;
-		if (tid == 0) {
-			if (!runs) {
-				ctl->halt = 1;
-			} else if (!beyond) {
-				ctl->tt[1 - A.par] = tick + 1;
-				A.spare[A.par] = 0;   /* for the next tick's outputs */
+		if (k == 0) {
+			if (tid == 0) {
+				if (runs) {
+					ctl->tt[1 - A.par] = tick + 1;
+					A.spare[A.par] = 0;   /* for the next tick's outputs */
+				} else {
+					ctl->halt = 1;
+				}
 			}
+			if (!SOLO && tid < PART_SLOTS)
+				A.tot[((tick + 1) % 3) * PART_SLOTS + tid] = 0;
 		}
-		if (!SOLO && tid < PART_SLOTS) A.tot[((tick + 1) % 3) * PART_SLOTS + tid] = 0;
+		const TileRep tr = SOLO ? A.one : tile_rep(A.trep, k);
+		if (D2) tile_finish<NT>(A.bstat + tr.band0, tr.nby, k, tick - 1, A.tot, ctl, T,
+				P, nrep);
+		else tile_finish<NT>(A.sin + tr.tile0, tr.ntiles, k, tick - 1, A.tot, ctl, T, P,
+				nrep);
 		return;
 	}
 	/* groups of one XCD take neighbouring tiles (their borders are then read
@@ -568,6 +570,14 @@ __global__ __launch_bounds__(NT) void k_tile(TileArgs A, Ctl *ctl, Tables T,
 		return D2 ? (j == 0 ? h.x : j == 1 ? h.y : j == 2 ? h.z : h.w)
 			: (uint32_t)__builtin_amdgcn_readlane((int)hw, (int)i);
 	};
+	/* No replica moves when the outputs of the last tick are more than the
+	 * capacity (the first groups then fail the batch): the records which that
+	 * tick started from stay, as its outputs may not all have been written.
+	 * (One replica: total_in, below; cut rows: k_tile_scan halts. Requested
+	 * before the grass, which would be waited for with it.) */
+	uint32_t outputs = 0;
+	if (!SOLO && !D2 && w == 0)
+		outputs = (uint32_t)A.tot[((ctl_word(12 + A.par) + 2) % 3) * PART_SLOTS + lane];
 	/* the ids: the agents of the replica's tiles before this one */
 	uint32_t bef = 0, all = 0;
 	if (!D2) {
@@ -609,13 +619,7 @@ __global__ __launch_bounds__(NT) void k_tile(TileArgs A, Ctl *ctl, Tables T,
 	 * that before or after the end of the last tick, written beside this:
 	 * both give the same answer. (One thread decides for the group: an energy
 	 * limit or an error may be noted meanwhile.) */
-	/* Nor does any replica when the outputs of the last tick are more than the
-	 * capacity (the first groups then fail the batch): the records which that
-	 * tick started from stay, as its outputs may not all have been written.
-	 * (One replica: total_in, below.) */
-	bool fits = true;
-	if (!SOLO && w == 0)
-		fits = wave_sum32((uint32_t)A.tot[((tick + 2) % 3) * PART_SLOTS + lane]) <= P.cap;
+	const bool fits = SOLO || D2 || w != 0 || wave_sum32(outputs) <= P.cap;
 	const bool go = tile_runs(ctl_word(4), ctl_word(14), ctl_word(15), tick) &
 		fits & (status == RS_ACTIVE) & (step < tr.iters) &
 		((over == 0) | (over == tick + 1));
@@ -1070,7 +1074,7 @@ __global__ __launch_bounds__(NT) void k_tile(TileArgs A, Ctl *ctl, Tables T,
  * iteration 46.6 -> 45.3). again: for a state whose ids the scan after a
  * failed tick has replaced, its bands' sums by k_tile_bands. */
 __global__ __launch_bounds__(WG) void k_tile_scan(TileArgs A, Ctl *ctl,
-	uint32_t nrep, uint32_t again) {
+	Params P, uint32_t nrep, uint32_t again) {
 	const bool SOLO = nrep == 1;
 	constexpr uint32_t EPT = 4;
 	__shared__ uint32_t s_tmp[NWAVE];
@@ -1117,6 +1121,12 @@ __global__ __launch_bounds__(WG) void k_tile_scan(TileArgs A, Ctl *ctl,
 	if (tid == 0) {
 		if (ty + 1 == tr.nby) A.rtot[k] = base;
 		A.bsum[A.par * A.nbands + band] = 0;
+	}
+	/* more agents than the capacity: no tick runs on them (see k_tile) */
+	if (!SOLO && band == 0 && tid < WAVE) {
+		const uint32_t t = ctl->tt[A.par] % 3;
+		if (wave_sum32((uint32_t)A.tot[t * PART_SLOTS + tid]) > P.cap && tid == 0)
+			ctl->halt = 1;
 	}
 	stat_sums<WG>(A.sout + t0, tr.nbx, s_f);
 	if (tid < 8) {
