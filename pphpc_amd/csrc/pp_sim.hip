@@ -3443,6 +3443,9 @@ constexpr uint32_t TILE_WIDE = 2048, TILE_MIN = 400;
  * its own: 0.88 ms with 8 and without, 0.83 with 32, 0.85 with 64). */
 constexpr uint32_t TILE_GRAPH = 32;
 
+/* Ticks enqueued at once after a stop of the tiles (next_piece). */
+constexpr uint32_t PIECE_MIN = 2 * TILE_GRAPH;
+
 /* Shapes of k_tile: threads, slots a thread, cells a tile. */
 struct TileShape {
 	uint32_t nt, ipt, cells;
@@ -3502,6 +3505,7 @@ struct pp_batch {
 	TilePlan plan;        /* the tiles of the replica table */
 	uint32_t tile_par = 0;   /* parity of the record buffers in use */
 	uint32_t tile_dense = 0; /* stops of the tiles: each makes them smaller */
+	uint32_t piece = UINT32_MAX; /* ticks enqueued at once (next_piece) */
 	/* 0: radix sort every tick; 1: automatic; 8..11: row buckets of
 	 * 2^mode cells */
 	uint32_t sort_mode = 1;
@@ -4349,6 +4353,19 @@ static void table_plan(pp_batch_t *b) {
 	tile_plan(b, g.data(), (uint32_t)g.size());
 }
 
+/* Ticks to enqueue at once of the next `ticks`: all, but few after a stop and
+ * then twice as many each time. Where a tile outgrows its limits, every launch
+ * behind it still takes 2 to 3 us, and a population that grows stops several
+ * times. Runs of 2000 iterations of the reference's v2 set: 400 x 400 (5
+ * stops) 56.5 -> 37.6 ms, 1600 x 1600 (3) 274 -> 256 (the staged step 251),
+ * without graphs 200 x 200 183 -> 38. A wait takes some 25 us. */
+static uint32_t next_piece(pp_batch_t *b, uint32_t ticks) {
+	if (ticks <= b->piece) return ticks;
+	const uint32_t n = b->piece;
+	b->piece *= 2;
+	return n;
+}
+
 /* After a run, with the control words read back: the parity of the records,
  * and, where a tile has outgrown its limits, the SoA state and the need for
  * another plan (returned in *again). */
@@ -4372,6 +4389,7 @@ static int tile_settle(pp_batch_t *b, int *again) {
 	if (c->tick == c->in_tick) b->soa_fresh = 1;
 	PP_TRY(to_soa(b));
 	b->tile_dense++;
+	b->piece = PIECE_MIN;
 	*again = 1;
 	return PP_SUCCESS;
 }
@@ -4508,6 +4526,7 @@ static int upload_table(pp_batch_t *b) {
 	b->table_nrep = nrep;
 	b->table_slots = order;
 	b->tile_dense = 0;
+	b->piece = UINT32_MAX;
 	table_plan(b);
 	return PP_SUCCESS;
 }
@@ -4680,7 +4699,7 @@ static int run_ticks(pp_batch_t *b, uint32_t ticks, double *sec = nullptr) {
 		const uint32_t t0 = b->ctl_host->tick;
 		PP_TRY(flush_admitted(b));
 		const uint32_t dense0 = b->tile_dense;
-		PP_TRY(enqueue_ticks(b, target - t0));
+		PP_TRY(enqueue_ticks(b, next_piece(b, target - t0)));
 		if (sec) {
 			HIP_OK(hipStreamSynchronize(b->stream));
 			*sec = now_s() - start;
@@ -5309,7 +5328,7 @@ static int simulate_noalloc(const pp_params_t *p, uint64_t seed,
 	 * than a chunk where the tiles stop short). */
 	uint32_t done = 0;
 	while (done < p->iters) {
-		const uint32_t chunk = min_u32(p->iters - done, b->stats_rows / 2);
+		const uint32_t chunk = next_piece(b, min_u32(p->iters - done, b->stats_rows / 2));
 		PP_TRY(enqueue_ticks(b, chunk));
 		HIP_OK(hipMemcpy(b->ctl_host, b->ctl, sizeof(Ctl), hipMemcpyDeviceToHost));
 		HIP_OK(hipMemcpy(b->rctl_host, b->rctl_dev, sizeof(RepCtl),

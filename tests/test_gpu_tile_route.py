@@ -81,3 +81,23 @@ def test_dense_populations_are_staged():
         sim.run(3)
         assert sim.tiles() == dict(in_use=0, threads=0, cut=0, tiles=0, slot=0,
                                    stops=0)
+
+
+@pytest.mark.parametrize("noalloc", [False, True], ids=["run", "without allocating"])
+def test_runs_in_pieces_after_stops(noalloc):
+    """A population that grows through several stops within one run: the
+    iterations after each are enqueued piece by piece, to the last."""
+    from oracle.pp_oracle import simulate
+    from pphpc_amd import Simulation, simulate_noalloc
+    d = v2ref(70, iters=500)
+    room = 4 * d["grid_xy"]
+    ref = simulate(d, seed=6, capacity=room)
+    print(f"[case] tile route: pieces {noalloc}", flush=True)
+    if noalloc:
+        assert np.array_equal(simulate_noalloc(gpu_params(d), 6, room, device=0), ref)
+        return
+    with Simulation(gpu_params(d), seed=6, capacity=room, device=0) as sim:
+        for _ in range(2):
+            assert sim.init().as_tuple() == tuple(ref[0])
+            assert np.array_equal(sim.run_array(500), ref[1:])
+            assert sim.tiles()["stops"] > 1
