@@ -3287,8 +3287,7 @@ __global__ __launch_bounds__(NT) void k_emit_move(
 
 enum KernelId {
 	KI_INIT_RESET,
-	KI_INIT_CELLS,
-	KI_INIT_AGENTS,
+	KI_INIT,
 	KI_INIT_DONE,
 	KI_MOVE0,
 	KI_SORT_UP,
@@ -3303,7 +3302,7 @@ enum KernelId {
 };
 
 const char *const kernel_names[KI_COUNT] = {
-	"init_reset", "init_cells", "init_agents", "init_done", "move0",
+	"init_reset", "init", "init_done", "move0",
 	"sort_up", "sort_scan", "sort_down", "act", "act_scan", "emit_move",
 	"bucket_scan", "bucket_sort",
 };
@@ -4551,7 +4550,7 @@ static int enqueue_init(pp_batch_t *b, uint32_t n, uint32_t end, uint32_t gc,
 		prof_begin(b, KI_INIT_RESET, pe);
 		k_rep_reset<<<m, WG, 0, b->stream>>>(b->tables(), list);
 		prof_end(b, pe);
-		prof_begin(b, KI_INIT_CELLS, pe);
+		prof_begin(b, KI_INIT, pe);
 		if (b->grass_bytes == 1) launch_init<uint8_t>(b, list, m, gc + ga);
 		else if (b->grass_bytes == 2) launch_init<uint16_t>(b, list, m, gc + ga);
 		else launch_init<uint32_t>(b, list, m, gc + ga);

@@ -59,3 +59,14 @@ def test_running_replicas_are_moved_by_one_launch(sort):
         b.run(40)
         for rid, (d, s), r in zip(ids, ds + [late], room):
             assert np.array_equal(b.rows_array(rid), simulate(d, seed=s, capacity=r)), s
+
+
+def test_the_profile_names_what_is_launched():
+    """Cells and agents are initialised by one kernel: one entry, no empty
+    one."""
+    from pphpc_amd import Simulation
+    with Simulation(gpu_params(v2s(64)), seed=1, capacity=12000, device=0) as sim:
+        sim.set_profiling(True)
+        sim.init()
+        p = {k: n for k, (n, _) in sim.profile().items() if k.startswith("init") or k == "move0"}
+        assert p == {"init_reset": 2, "init": 1, "init_done": 1, "move0": 1}
