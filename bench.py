@@ -149,8 +149,8 @@ def compulsory_bytes(name, c):
 def counted_traffic(kernel, which):
     """Bytes per dispatch of a kernel from the committed rocprofv3 counter
     runs (profiles/hbm_traffic.json: FETCH_SIZE and WRITE_SIZE, scaled by a
-    1 GiB copy; summaries in profiles/hbm_traffic_v2s12800.md and
-    profiles/counters_v2s12800.md): which = "radix" or "auto" at
+    1 GiB copy; summaries in profiles/tile_step.md, profiles/
+    hbm_traffic_v2s12800.md and profiles/counters_v2s12800.md): which = "radix" or "auto" at
     12800x12800, "v2s1600" at 1600x1600. None when not measured."""
     path = os.path.join(ROOT, "profiles", "hbm_traffic.json")
     try:
@@ -534,7 +534,7 @@ def main():
                                                   args.steps), args.seed)
     if args.workload == "v2s1600":
         roof["traffic"] = counted_traffic(roof["kernel"], "v2s1600")
-        roof["traffic_source"] = ("profiles/counters_v2s12800.md (FETCH_SIZE "
+        roof["traffic_source"] = ("profiles/tile_step.md (FETCH_SIZE "
                                   "+ WRITE_SIZE; at this size mostly "
                                   "Infinity Cache, not HBM)")
     log(f"dominant kernel {roof['kernel']}: {roof['achieved']} GB/s")
@@ -553,8 +553,8 @@ def main():
         roof_big_b = measure_roofline(big, 4 * nb, args.big_roofline_steps,
                                       args.seed)
         roof_big_b["traffic"] = counted_traffic(roof_big_b["kernel"], "auto")
-        roof_big_b["traffic_source"] = "profiles/counters_v2s12800.md"
-        log(f"12800^2 auto (buckets): dominant kernel {roof_big_b['kernel']}: "
+        roof_big_b["traffic_source"] = "profiles/tile_step.md"
+        log(f"12800^2 auto (tiles): kernel {roof_big_b['kernel']}: "
             f"{roof_big_b['achieved']} GB/s, "
             f"{roof_big_b['ms_per_iteration']} ms")
 

@@ -340,8 +340,8 @@ int pp_batch_tiles(const pp_batch_t *b, uint32_t out[6]);
  * depend on it. */
 int pp_batch_set_sort(pp_batch_t *b, uint32_t mode);
 
-/* Radix sort launch shape: keys per thread (8 or 16; tile = 256 x that) and
- * the widest radix digit (8 or 11 bits). Results do not depend on it. */
+/* Radix sort launch shape: 8 or 16 for tiles of 2048 or 4096 keys (of which
+ * each of 512 threads holds 4 or 8), and the widest radix digit (8 or 11 bits). Results do not depend on it. */
 int pp_batch_set_shape(pp_batch_t *b, uint32_t keys_per_thread,
 	uint32_t max_digit_bits);
 

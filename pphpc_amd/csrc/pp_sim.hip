@@ -3312,8 +3312,8 @@ struct PendingEvent {
 	hipEvent_t start, stop;
 };
 
-/* Launch shape of the sort: keys per thread of a sort tile (tile = 256 x
- * kpt positions) and the widest digit (passes = ceil(key bits / max_bits),
+/* Launch shape of the sort: positions of a sort tile in units of 256 (by
+ * groups of 512 threads) and the widest digit (passes = ceil(key bits / max_bits),
  * bits spread evenly over the passes). */
 struct SortShape {
 	int kpt;
@@ -4148,8 +4148,8 @@ static void tile_layout(const pp_batch_t *b, const TileGrid *grid, uint32_t n,
 		width = std::max(width, grid[i].rep->gx);
 		cells += grid[i].rep->C;
 	}
-	/* (by little: a stop costs a few milliseconds at most, as what is enqueued
-	 * of the run returns at once, tiles of fewer rows than need be every
+	/* (by little: a stop costs 2 to 3 us for each iteration queued behind it
+	 * and the change of form, tiles of fewer rows than need be every
 	 * iteration: 30 x 1600 x 1600 from iteration 400 on, 311 us
 	 * with the 4 rows that 1.1 gives, 369 with 3) */
 	for (uint32_t i = 0; i < b->tile_dense; i++) dens *= 1.1;
@@ -4205,10 +4205,14 @@ static void tile_layout(const pp_batch_t *b, const TileGrid *grid, uint32_t n,
 			break;
 	}
 	if (p.d2) {
-		/* 256 threads while their slots hold the agents of all the cells, else
-		 * 512 threads with 32 rows, before tiles of fewer rows: 6000 x 6000,
-		 * 0.31 agents a cell after 500 iterations, 169 -> 134 us, 64 replicas
-		 * of up to 3200 x 3200 880 -> 615 us */
+		/* 256 threads while their slots hold the agents of all the cells
+		 * (16 rows; 32 rows in 512 threads move fewer neighbours' agents but
+		 * wait for each other longer: 12800 x 12800, 0.26 agents a cell, 560 us
+		 * against 587, 4001 x 2999 48.4 and 48.8, with 0.16 a cell 43.6 and
+		 * 44.4, 6000 x 6000, 0.18 a cell, 122 and 127), else 512 threads with
+		 * 32 rows, before tiles of fewer rows: 6000 x 6000, 0.31 agents a cell
+		 * after 500 iterations, 169 -> 134 us, 64 replicas of up to 3200 x 3200
+		 * 880 -> 615 us (512 threads with 16 rows: 12800 x 12800 848) */
 		limits(0);
 		if (rows_max(bx) * bx < tile_shapes[0].cells) limits(1);
 	} else if (c == shapes) {

@@ -23,7 +23,7 @@
  * more than its four neighbours' border cells.
  *
  * What bounds it: on small grids the chain of one group's phases (two round
- * trips to memory, seven barriers, and fetching some 20 KB of instructions
+ * trips to memory, eight barriers, and fetching some 20 KB of instructions
  * that each wave runs through about once); on large ones the vector units.
  * Per iteration, against the three staged kernels: 100 x 100 24.5 -> 6.8 us,
  * 400 x 400 27.5 -> 9.5, 1600 x 1600 41 -> 17.2, 12800 x 12800 768 -> 540;
@@ -31,7 +31,9 @@
  *
  * A tile that outgrows its LDS or border lists sets Ctl::stop; the tick
  * after it is then not run (every group of a later launch returns), and the
- * host goes on with smaller tiles or the staged step.
+ * host goes on with smaller tiles or the staged step. Where the agents of all
+ * replicas are more than the capacity, the batch fails with that tick, no tick
+ * runs after it, and the records that it started from stay.
  *
  * Included by pp_sim.hip, inside its namespace.
  */

@@ -127,6 +127,7 @@ def test_states_of_a_failed_batch(tile, pieces, monkeypatch):
             for rid, d, (states, _) in zip(ids, (GROWS, STAYS), ref):
                 assert_state_equal(b.state(rid), _left(d, states, FAILS),
                                    f"replica {rid}")
+            assert b.add(gpu_params(STAYS), 3, 300) is None
             b.set_sort(0)
 
 
