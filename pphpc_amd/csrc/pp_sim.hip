@@ -961,6 +961,30 @@ __global__ __launch_bounds__(WG) void k_publish(const Ctl *ctl, RepCtl *rctl,
 			reinterpret_cast<const uint32_t *>(rc)[i];
 }
 
+/* Copies from pinned host memory, a few in one launch. Asynchronous copies by
+ * the runtime on a handle's stream made later allocations and new streams slow:
+ * of simulations made, initialised and destroyed in turn, 400 x 400, making one
+ * took 0.2 to 1 ms, 1000 x 1000 up to 2.5; with this kernel 0.13 and 0.17. The
+ * runtime's synchronous copies take 7 us each, of which an initialisation has
+ * six (100 x 100: 122 us with those and a launch for each kind, 74 with
+ * asynchronous ones, 52 now). */
+static_assert(sizeof(Rep) % 4 == 0 && sizeof(Admit) % 4 == 0, "copied as words");
+constexpr uint32_t UPLOADS = 8;
+struct Upload {
+	uint32_t *dst;
+	uint32_t at, words;
+};
+struct Uploads {
+	Upload u[UPLOADS];
+	uint32_t n;
+};
+
+__global__ __launch_bounds__(WG) void k_upload(Uploads U, const uint32_t *stage) {
+	for (uint32_t k = 0; k < U.n; k++)
+		for (uint32_t i = blockIdx.x * WG + threadIdx.x; i < U.u[k].words; i += gridDim.x * WG)
+			U.u[k].dst[i] = stage[U.u[k].at + i];
+}
+
 /* Before k_move_soa: no pairs (positions of replicas that have ended stay
  * so), no survivors counted, and the partial sums at zero. */
 __global__ __launch_bounds__(WG) void k_pairs_clear(uint32_t *keys, Ctl *ctl,
@@ -3548,9 +3572,11 @@ struct pp_batch {
 	Admit *admit_dev = nullptr;
 	uint32_t next_pos = 0;        /* batch position after their agents */
 	int table_dirty = 0;          /* the device's replica table is not current */
-	/* host copies of the replica table, which asynchronous copies read */
-	std::vector<uint32_t> h_cbs, h_order, h_bbase, h_crep, h_brep;
-	uint32_t h_counts[2] = {0, 0};
+	/* pinned memory that the copies to the device read (upload), after
+	 * stats_host in its allocation; used since the stream was last idle */
+	uint32_t *stage = nullptr;
+	uint32_t stage_words = 0, stage_used = 0;
+	Uploads uploads{};            /* copies not sent yet */
 	uint64_t table_version = 0;   /* replica table uploads */
 	uint32_t table_nrep = 0;      /* replicas in the table */
 	std::vector<uint32_t> table_slots;
@@ -3977,17 +4003,43 @@ static void launch_tiles_out(pp_batch_t *b) {
 		b->P, b->table_nrep, (GT *)b->grass_at, b->cell, b->energy, b->type);
 }
 
+/* Launches the copies that upload has listed. */
+static int send_uploads(pp_batch_t *b) {
+	if (!b->uploads.n) return PP_SUCCESS;
+	k_upload<<<16, WG, 0, b->stream>>>(b->uploads, b->stage);
+	b->uploads.n = 0;
+	HIP_OK(hipGetLastError());
+	return PP_SUCCESS;
+}
+
+/* Words of the host for the device, in stream order once sent: by a kernel,
+ * from pinned memory (k_upload). What does not fit there is copied at once,
+ * behind what the stream holds. */
+static int upload(pp_batch_t *b, void *dst, const void *src, size_t bytes) {
+	const size_t words = bytes / 4;
+	if (!words) return PP_SUCCESS;
+	if (b->stage_used + words > b->stage_words) {
+		PP_TRY(send_uploads(b));
+		HIP_OK(hipStreamSynchronize(b->stream));
+		HIP_OK(hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice));
+		return PP_SUCCESS;
+	}
+	if (b->uploads.n == UPLOADS) PP_TRY(send_uploads(b));
+	memcpy(b->stage + b->stage_used, src, bytes);
+	b->uploads.u[b->uploads.n++] = Upload{(uint32_t *)dst, b->stage_used, (uint32_t)words};
+	b->stage_used += (uint32_t)words;
+	return PP_SUCCESS;
+}
+
 /* SoA state (in cell order) -> tiles. */
 static int tiles_in(pp_batch_t *b) {
 	const bool d2 = b->plan.d2;
 	const TilePlan &p = b->plan;
 	if (b->table_nrep > 1) {
-		HIP_OK(hipMemcpyAsync(p.trep, p.h_trep.data(), p.h_trep.size() * sizeof(TileRep),
-			hipMemcpyHostToDevice, b->stream));
-		HIP_OK(hipMemcpyAsync(p.tk, p.h_tk.data(), p.h_tk.size() * 4,
-			hipMemcpyHostToDevice, b->stream));
-		HIP_OK(hipMemcpyAsync(p.bk, p.h_bk.data(), p.h_bk.size() * 4,
-			hipMemcpyHostToDevice, b->stream));
+		PP_TRY(upload(b, p.trep, p.h_trep.data(), p.h_trep.size() * sizeof(TileRep)));
+		PP_TRY(upload(b, p.tk, p.h_tk.data(), p.h_tk.size() * 4));
+		PP_TRY(upload(b, p.bk, p.h_bk.data(), p.h_bk.size() * 4));
+		PP_TRY(send_uploads(b));
 	}
 	if (b->grass_bytes == 1) d2 ? launch_tiles_in<uint8_t, true>(b) : launch_tiles_in<uint8_t, false>(b);
 	else if (b->grass_bytes == 2) d2 ? launch_tiles_in<uint16_t, true>(b) : launch_tiles_in<uint16_t, false>(b);
@@ -4402,6 +4454,7 @@ static int read_ctl(pp_batch_t *b) {
 		b->stats_rows, b->ctl_host, b->rctl_host, b->stats_host);
 	HIP_OK(hipGetLastError());
 	HIP_OK(hipStreamSynchronize(b->stream));
+	b->stage_used = 0;
 	b->ctl_fresh = 1;
 	return prof_collect(b);
 }
@@ -4410,49 +4463,41 @@ static int read_ctl(pp_batch_t *b) {
  * stream must be idle. */
 static int upload_table(pp_batch_t *b) {
 	PP_TRY(to_soa(b));
-	/* (the copies below read vectors that the last upload may still use) */
 	HIP_OK(hipStreamSynchronize(b->stream));
+	b->stage_used = 0;
 	b->table_dirty = 0;
 	std::vector<std::pair<uint32_t, uint32_t>> t;
 	for (uint32_t s = 0; s < b->max_rep; s++)
 		if (b->slot_rid[s] >= 0) t.push_back({b->rep_host[s].cb, s});
 	std::sort(t.begin(), t.end());
-	std::vector<uint32_t> &cbs = b->h_cbs, &order = b->h_order;
-	cbs.resize(t.size());
-	order.resize(t.size());
+	std::vector<uint32_t> cbs(t.size()), order(t.size());
 	for (size_t i = 0; i < t.size(); i++) {
 		cbs[i] = t[i].first;
 		order[i] = t[i].second;
 	}
-	auto up = [&](void *dst, const void *src, size_t bytes) {
-		return bytes ? hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, b->stream)
-			: hipSuccess;
-	};
 	if (!t.empty()) {
 		const auto mm = std::minmax_element(order.begin(), order.end());
 		const uint32_t s0 = *mm.first, s1 = *mm.second + 1;
-		HIP_OK(up(b->rep_dev + s0, &b->rep_host[s0], (s1 - s0) * sizeof(Rep)));
-		HIP_OK(up(b->cbs_dev, cbs.data(), t.size() * 4));
-		HIP_OK(up(b->order_dev, order.data(), t.size() * 4));
+		PP_TRY(upload(b, b->rep_dev + s0, &b->rep_host[s0], (s1 - s0) * sizeof(Rep)));
+		PP_TRY(upload(b, b->cbs_dev, cbs.data(), t.size() * 4));
+		PP_TRY(upload(b, b->order_dev, order.data(), t.size() * 4));
 	}
 	const uint32_t nrep = (uint32_t)t.size();
 	/* the cell-chunk table of rep_index, for a table of several */
 	if (nrep > 1) {
-		std::vector<uint32_t> &crep = b->h_crep;
-		crep.resize((size_t)(b->P.C >> CREP_SHIFT) + 1);
+		std::vector<uint32_t> crep((size_t)(b->P.C >> CREP_SHIFT) + 1);
 		uint32_t k = 0;
 		for (size_t i = 0; i < crep.size(); i++) {
 			const uint64_t c0 = (uint64_t)i << CREP_SHIFT;
 			while (k + 1 < nrep && cbs[k + 1] <= c0) k++;
 			crep[i] = k;
 		}
-		HIP_OK(up(b->crep_dev, crep.data(), crep.size() * 4));
+		PP_TRY(upload(b, b->crep_dev, crep.data(), crep.size() * 4));
 	}
 	/* bucket layout: rows of blocks of 2^bshift cells, replicas in table
 	 * order */
 	const uint32_t shift = b->sort_mode >= 8 ? b->sort_mode : 11u;
-	std::vector<uint32_t> &bbase = b->h_bbase;
-	bbase.resize(nrep + 1);
+	std::vector<uint32_t> bbase(nrep + 1);
 	uint64_t nbk = 0;
 	for (uint32_t i = 0; i < nrep; i++) {
 		bbase[i] = (uint32_t)std::min<uint64_t>(nbk, 0xFFFFFFFFull);
@@ -4461,7 +4506,7 @@ static int upload_table(pp_batch_t *b) {
 		nbk += (uint64_t)((rp.gy + h - 1) / h) * row_blocks(rp.gx, shift);
 	}
 	bbase[nrep] = (uint32_t)std::min<uint64_t>(nbk, 0xFFFFFFFFull);
-	HIP_OK(up(b->bbase_dev, bbase.data(), (nrep + 1) * 4));
+	PP_TRY(upload(b, b->bbase_dev, bbase.data(), (nrep + 1) * 4));
 	/* Row buckets when chosen, or automatically: always for one replica,
 	 * for several while the buckets are few or dense enough that their
 	 * per-bucket latency stays below the radix sort's passes. The density
@@ -4478,11 +4523,10 @@ static int upload_table(pp_batch_t *b) {
 	while (top + 1 < (uint32_t)CNT_LEVELS && (nbk >> (6 * (top + 1))) > 0) top++;
 	/* the replica of each bucket, for the bucket sort of several */
 	if (on && nrep > 1) {
-		std::vector<uint32_t> &brep = b->h_brep;
-		brep.resize(nbk);
+		std::vector<uint32_t> brep(nbk);
 		for (uint32_t i = 0; i < nrep; i++)
 			std::fill(brep.begin() + bbase[i], brep.begin() + bbase[i + 1], i);
-		HIP_OK(up(b->brep_dev, brep.data(), nbk * 4));
+		PP_TRY(upload(b, b->brep_dev, brep.data(), nbk * 4));
 	}
 	const uint32_t one = nrep == 1 ? order[0] : 0u;
 	const uint32_t solo = nrep == 1 ? 1u : 0u;
@@ -4519,9 +4563,9 @@ static int upload_table(pp_batch_t *b) {
 	}
 	const uint32_t nb32 = on ? (uint32_t)nbk : 0u;
 	static_assert(offsetof(Ctl, nbuckets) == offsetof(Ctl, nrep) + 4, "copied as one");
-	b->h_counts[0] = nrep;
-	b->h_counts[1] = nb32;
-	HIP_OK(up(&b->ctl->nrep, b->h_counts, 8));
+	const uint32_t counts[2] = {nrep, nb32};
+	PP_TRY(upload(b, &b->ctl->nrep, counts, 8));
+	PP_TRY(send_uploads(b));
 	b->ctl_host->nrep = nrep;
 	b->ctl_host->nbuckets = nb32;
 	b->need_radix = 1;
@@ -4585,10 +4629,9 @@ static int flush_admitted(pp_batch_t *b) {
 		ga = std::max(ga, init_groups(b->rep_host[a.slot].n0, INIT_AGENTS));
 	}
 	const uint32_t n = (uint32_t)b->admitted.size();
-	HIP_OK(hipMemcpyAsync(b->admit_dev, b->admitted.data(), n * sizeof(Admit),
-		hipMemcpyHostToDevice, b->stream));
+	PP_TRY(upload(b, b->admit_dev, b->admitted.data(), n * sizeof(Admit)));
+	PP_TRY(send_uploads(b));
 	PP_TRY(enqueue_init(b, n, b->next_pos, gc, ga));
-	HIP_OK(hipStreamSynchronize(b->stream));   /* (the list has been read) */
 	for (auto &kv : b->reps) kv.second.pending = 0;
 	b->admitted.clear();
 	b->ctl_fresh = 0;
@@ -4876,8 +4919,14 @@ static int batch_alloc(pp_batch_t *b) {
 	HIP_OK(hipMemset(b->ncnt, 0, nbw * 4));
 	HIP_OK(hipMemset(b->P.part, 0, PART_SLOTS * PART_STRIDE * 8));
 	const size_t srows = (size_t)b->max_rep * b->stats_rows;
-	HIP_OK(hipHostMalloc(&b->stats_host, srows * sizeof(pp_stats64_t),
+	/* the tables of as many replicas, and, of several, 64 KB for those that
+	 * grow with their grids */
+	const size_t words = std::min<size_t>(1u << 18, (b->max_rep == 1 ? 256 : 16384) +
+		b->max_rep * ((sizeof(Rep) + sizeof(TileRep) + sizeof(Admit)) / 4 + 4));
+	HIP_OK(hipHostMalloc(&b->stats_host, srows * sizeof(pp_stats64_t) + words * 4,
 		hipHostMallocDefault));
+	b->stage = (uint32_t *)(b->stats_host + srows);
+	b->stage_words = (uint32_t)words;
 	HIP_OK(hipHostMalloc(&b->ctl_host, sizeof(Ctl), hipHostMallocDefault));
 	HIP_OK(hipHostMalloc(&b->rctl_host, (size_t)b->max_rep * sizeof(RepCtl),
 		hipHostMallocDefault));

@@ -70,3 +70,24 @@ def test_the_profile_names_what_is_launched():
         sim.init()
         p = {k: n for k, (n, _) in sim.profile().items() if k.startswith("init") or k == "move0"}
         assert p == {"init_reset": 2, "init": 1, "init_done": 1, "move0": 1}
+
+
+def test_tables_larger_than_the_pinned_memory(monkeypatch):
+    """24,000 tiles of one row: their table is copied in one piece, not from
+    the handle's pinned memory; the next admission's tables are."""
+    from oracle.pp_oracle import simulate
+    from pphpc_amd import Batch
+    monkeypatch.setenv("PPHPC_TILE", "0,0,1")
+    print("[case] large tables", flush=True)
+    ds = [(v2s(gx=4, gy=8000, iters=40), 1), (v1(gx=5, gy=16000, iters=60), 2),
+          (v2s(gx=9, gy=70, iters=15), 3)]
+    room = [2 * d["grid_xy"] for d, _ in ds]
+    # (the tiles' tables lie in those of the cells' buckets)
+    with Batch(sum(room), 1 << 23, 3, 15, device=0) as b:
+        ids = [b.add(gpu_params(d), s, r) for (d, s), r in zip(ds[:2], room)]
+        b.run(20)
+        assert b.tiles()["tiles"] == 24000 and b.tiles()["in_use"] == 1
+        ids.append(b.add(gpu_params(ds[2][0]), ds[2][1], room[2]))
+        b.run(60)
+        for rid, (d, s), r in zip(ids, ds, room):
+            assert np.array_equal(b.rows_array(rid), simulate(d, seed=s, capacity=r)), s
