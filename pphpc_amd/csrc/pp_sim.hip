@@ -961,9 +961,10 @@ __global__ __launch_bounds__(WG) void k_publish(const Ctl *ctl, RepCtl *rctl,
 			reinterpret_cast<const uint32_t *>(rc)[i];
 }
 
-/* Copies from pinned host memory, a few in one launch. Asynchronous copies by
- * the runtime on a handle's stream made later allocations and new streams slow:
- * of simulations made, initialised and destroyed in turn, 400 x 400, making one
+/* Copies from pinned host memory, a few in one launch. With asynchronous copies
+ * by the runtime on the handle's stream in its place, from pageable or pinned
+ * memory, allocations and new streams were often slow afterwards: of
+ * simulations made, initialised and destroyed in turn, 400 x 400, making one
  * took 0.2 to 1 ms, 1000 x 1000 up to 2.5; with this kernel 0.13 and 0.17. The
  * runtime's synchronous copies take 7 us each, of which an initialisation has
  * six (100 x 100: 122 us with those and a launch for each kind, 74 with
