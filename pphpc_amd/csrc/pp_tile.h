@@ -177,14 +177,15 @@ __device__ void tile_finish(const TileStat *units, uint32_t nunits, uint32_t k,
 #pragma unroll
 	for (int i = 0; i < 8; i++) a[i] = __shfl(sum, i);
 	if (lane != 0) return;
-	const unsigned long long out64 = a[0] + a[1];
-	if (nrep == 1) total = out64;
-	const bool beyond = total > P.cap;
-	/* (the tick counts on when every replica is done) */
-	if (k == 0 && !failed && !beyond && (int32_t)(t + 1 - ctl->tick) > 0)
+	/* (the tick counts on when every replica is done; one replica's total:
+	 * below) */
+	if (k == 0 && !failed && total <= P.cap && (int32_t)(t + 1 - ctl->tick) > 0)
 		ctl->tick = t + 1;
 	if (!due) return;
-	if (beyond) {
+	const unsigned long long out64 = a[0] + a[1];
+	if (nrep == 1) total = out64;
+	if (total > P.cap) {
+		if (k == 0) ctl->tick = t;
 		set_error(ctl, PP_OUT_OF_RESOURCES, t, -1);
 		return;
 	}
