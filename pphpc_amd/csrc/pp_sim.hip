@@ -4463,10 +4463,11 @@ static int read_ctl(pp_batch_t *b) {
 /* Replica table: the slots in use sorted by first cell, and its length. The
  * stream must be idle. */
 static int upload_table(pp_batch_t *b) {
+	b->table_dirty = 1;  /* until it is whole */
 	PP_TRY(to_soa(b));
 	HIP_OK(hipStreamSynchronize(b->stream));
 	b->stage_used = 0;
-	b->table_dirty = 0;
+	b->uploads.n = 0;    /* (of an upload that an exception ended) */
 	std::vector<std::pair<uint32_t, uint32_t>> t;
 	for (uint32_t s = 0; s < b->max_rep; s++)
 		if (b->slot_rid[s] >= 0) t.push_back({b->rep_host[s].cb, s});
@@ -4576,6 +4577,7 @@ static int upload_table(pp_batch_t *b) {
 	b->tile_dense = 0;
 	b->piece = UINT32_MAX;
 	table_plan(b);
+	b->table_dirty = 0;
 	return PP_SUCCESS;
 }
 
